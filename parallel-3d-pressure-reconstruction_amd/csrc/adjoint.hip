@@ -496,10 +496,14 @@ hipError_t launch_adj_fixed(int nS, const double* t, DevScalars* sc, long long* 
 template <int kBits>
 __global__ void __launch_bounds__(1024)
 k_adj_seg_u(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __restrict__ segs,
-            GridDesc g, TileGrid tg, const double* __restrict__ u, double* __restrict__ useg) {
+            GridDesc g, TileGrid tg, const double* __restrict__ u, double* __restrict__ useg,
+            int parts) {
   constexpr int kTile = 1 << kBits, kTileMask = kTile - 1, kVox = kTile * kTile * kTile;
   __shared__ double U[kVox];
-  const int tile = (int)xcd_block();
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tp.tile;
+  const unsigned long long b = tile_ptr1[tile], e = tile_ptr1[tile + 1];
+  if (b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
@@ -508,8 +512,8 @@ k_adj_seg_u(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __re
     U[lds_slot<kBits>(l)] = (i < g.X && j < g.Y && k < g.Z) ? u[i + j * sy + k * sz] : 0.0;
   }
   __syncthreads();
-  const unsigned long long b = tile_ptr1[tile], e = tile_ptr1[tile + 1];
-  for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
+  for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
     const SegRec sr = segs[jj];
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
     const unsigned int n = (sr.info >> kSegLvBits) & 63u;
@@ -553,11 +557,15 @@ template <int kBits>
 __global__ void __launch_bounds__(1024)
 k_adj_tile_scatter(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
                    GridDesc g, TileGrid tg, WalkParams wp, const double* __restrict__ u,
-                   const double* __restrict__ tafter, double* __restrict__ dg) {
+                   const double* __restrict__ tafter, double* __restrict__ dg, int parts) {
   constexpr int kTile = 1 << kBits, kTileMask = kTile - 1, kVox = kTile * kTile * kTile;
   __shared__ double U[kVox];
   __shared__ double A[3][kVox];
-  const int tile = (int)xcd_block();
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tp.tile;
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
+  // (parts > 1: dg is cleared before the launch)
+  if (parts > 1 && b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
@@ -569,8 +577,8 @@ k_adj_tile_scatter(const unsigned long long* __restrict__ tile_ptr, const SegRec
     A[0][sl] = A[1][sl] = A[2][sl] = 0.0;
   }
   __syncthreads();
-  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
-  for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
+  for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
     const SegRec sr = segs[jj];
     const int lv0 = (int)(sr.info & ((1u << kSegLvBits) - 1u));
     const unsigned int n = (sr.info >> kSegLvBits) & 63u;
@@ -630,9 +638,15 @@ k_adj_tile_scatter(const unsigned long long* __restrict__ tile_ptr, const SegRec
     if (i >= g.X || j >= g.Y || k >= g.Z) continue;
     const int64_t v = i + j * sy + k * sz;
     const int sl = lds_slot<kBits>(l);
-    dg[v] = A[0][sl];
-    dg[V + v] = A[1][sl];
-    dg[2 * V + v] = A[2][sl];
+    if (parts == 1) {
+      dg[v] = A[0][sl];
+      dg[V + v] = A[1][sl];
+      dg[2 * V + v] = A[2][sl];
+    } else {
+      unsafeAtomicAdd(&dg[v], A[0][sl]);
+      unsafeAtomicAdd(&dg[V + v], A[1][sl]);
+      unsafeAtomicAdd(&dg[2 * V + v], A[2][sl]);
+    }
   }
 }
 
@@ -649,21 +663,26 @@ hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile
                        rays, nrays, g, nseg, val_off, useg, tvol);
     return hipGetLastError();
   }
+  const int parts = tile_parts(ntiles, false);
   if (what == 0) {
     if (tg.bits == 3)
-      hipLaunchKernelGGL(k_adj_seg_u<3>, dim3(ntiles), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
-                         tg, u, useg);
+      hipLaunchKernelGGL(k_adj_seg_u<3>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
+                         tg, u, useg, parts);
     else
-      hipLaunchKernelGGL(k_adj_seg_u<4>, dim3(ntiles), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
-                         tg, u, useg);
+      hipLaunchKernelGGL(k_adj_seg_u<4>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
+                         tg, u, useg, parts);
     return hipGetLastError();
   }
+  if (parts > 1) {
+    const hipError_t e = launch_fill_f64(dg, 3 * (int64_t)g.X * g.Y * g.Z, 0.0, st);
+    if (e != hipSuccess) return e;
+  }
   if (tg.bits == 3)
-    hipLaunchKernelGGL(k_adj_tile_scatter<3>, dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g,
-                       tg, wp, u, useg, dg);
+    hipLaunchKernelGGL(k_adj_tile_scatter<3>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr, segs, g,
+                       tg, wp, u, useg, dg, parts);
   else
-    hipLaunchKernelGGL(k_adj_tile_scatter<4>, dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g,
-                       tg, wp, u, useg, dg);
+    hipLaunchKernelGGL(k_adj_tile_scatter<4>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr, segs, g,
+                       tg, wp, u, useg, dg, parts);
   return hipGetLastError();
 }
 

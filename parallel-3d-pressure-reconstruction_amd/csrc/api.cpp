@@ -1392,26 +1392,26 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
     }
   } else {
     // entry counts per tile, their offsets, then the entries
-    const int nt = pl.ntiles;
+    const int nt = pl.ntiles, parts = tile_entries_parts(m, nt), np = nt * parts;
     DevBuf tcnt;
-    OMNI_TRY_HIP(ctx, tcnt.alloc(sizeof(unsigned int) * ((size_t)nt + 1)));
-    OMNI_TRY_HIP(ctx, ctx->am_tbase.alloc(sizeof(unsigned long long) * ((size_t)nt + 1)));
+    OMNI_TRY_HIP(ctx, tcnt.alloc(sizeof(unsigned int) * ((size_t)np + 1)));
+    OMNI_TRY_HIP(ctx, ctx->am_tbase.alloc(sizeof(unsigned long long) * ((size_t)np + 1)));
     OMNI_TRY_HIP(ctx, launch_tile_entries(false, m, nt, pl.tile_ptr.as<unsigned long long>(),
                                           pl.segs.as<SegRec>(), pl.g, pl.tg, wp, aux,
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
                                           ctx->mk_wn.as<double>(), ctx->am_run.as<uint32_t>(),
                                           sid, tfirst, tcnt.as<unsigned int>(), nullptr, nullptr,
                                           nullptr, nullptr, st));
-    OMNI_TRY_HIP(ctx, stmp.alloc(scan_u32_tmp_bytes(nt)));
-    OMNI_TRY_HIP(ctx, launch_scan_u32(tcnt.as<unsigned int>(), nt,
+    OMNI_TRY_HIP(ctx, stmp.alloc(scan_u32_tmp_bytes(np)));
+    OMNI_TRY_HIP(ctx, launch_scan_u32(tcnt.as<unsigned int>(), np,
                                       ctx->am_tbase.as<unsigned long long>(), 0, stmp.as<void>(),
                                       stmp.size(), st));
-    std::vector<unsigned long long> hbase((size_t)nt + 1);
+    std::vector<unsigned long long> hbase((size_t)np + 1);
     OMNI_TRY_HIP(ctx, hipMemcpyAsync(hbase.data(), ctx->am_tbase.as<void>(),
-                                     sizeof(unsigned long long) * ((size_t)nt + 1),
+                                     sizeof(unsigned long long) * ((size_t)np + 1),
                                      hipMemcpyDeviceToHost, st));
     OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
-    nnz = hbase[nt];
+    nnz = hbase[np];
     if (nnz == 0) {
       *fallback = true;
       return OMNI3D_OK;
@@ -1433,8 +1433,9 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
         2048ull, std::min<unsigned long long>(65536ull, nnz / 4096ull));
     std::vector<MaskChunk> chunks;
     for (int t = 0; t < nt; t++)
-      for (unsigned long long b = hbase[t]; b < hbase[t + 1]; b += csz)
-        chunks.push_back(MaskChunk{b, std::min(hbase[t + 1], b + csz), t, 0});
+      for (unsigned long long b = hbase[(size_t)t * parts], e = hbase[(size_t)(t + 1) * parts];
+           b < e; b += csz)
+        chunks.push_back(MaskChunk{b, std::min(e, b + csz), t, 0});
     nchunks = (int)chunks.size();
     OMNI_TRY_HIP(ctx, ctx->am_chunks.alloc(sizeof(MaskChunk) * chunks.size()));
     OMNI_TRY_HIP(ctx, hipMemcpy(ctx->am_chunks.as<void>(), chunks.data(),

@@ -201,13 +201,16 @@ __global__ void __launch_bounds__(1024)
 k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
             GridDesc g, TileGrid tg, WalkParams wp,
             const typename Vec4<T>::type* __restrict__ field, const double* __restrict__ aux,
-            RuleSegs rs) {
+            RuleSegs rs, int parts) {
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kVox = kTile * kTile * kTile;
   constexpr bool kAux = kMethod != kMaskPlain;
   __shared__ double s_aux[kAux ? kVox : 1];
-  const int tile = (int)xcd_block();
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tp.tile;
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
+  if (b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
@@ -227,8 +230,8 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
     if constexpr (kAux) return s_aux[lds_slot<kBits>(l)];
     else return 0.0;
   };
-  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
-  for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
+  for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
     const SegRec sr = segs[jj];
     const int lv0 = (int)(sr.info & ((1u << kSegLvBits) - 1u));
     const unsigned int n = (sr.info >> kSegLvBits) & 63u;
@@ -459,7 +462,7 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
               const DevScalars* __restrict__ sc, long long* __restrict__ sumfx,
               double* __restrict__ sumd, double* __restrict__ segS,
               unsigned int* __restrict__ wcnt, double* __restrict__ wsum,
-              uint8_t* __restrict__ src) {
+              uint8_t* __restrict__ src, int parts) {
   using V4 = typename Vec4<T>::type;
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
@@ -469,7 +472,11 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
   __shared__ MaskLds<T, kMethod, kVox> L;
   if (sc->converged) return;
   const double* __restrict__ p = ((k - 1) & 1) ? p1 : p0;
-  const int tile = (int)xcd_block();
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tp.tile;
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
+  // (parts > 1: the outputs are cleared before the launch)
+  if (parts > 1 && b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
@@ -519,8 +526,8 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
       atomicAdd(&L.acc[sl], curl_value(c, curl, cnt));
     }
   };
-  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
-  for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
+  for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
     const SegRec sr = segs[jj];
     const uint32_t f = F[sr.g];
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
@@ -603,13 +610,21 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
     if (i >= g.X || j >= g.Y || kk >= g.Z) continue;
     const int64_t gv = i + j * sy + kk * sz;
     const int sl = lds_slot<kBits>(l);
+    const auto x = L.acc[sl];
     if constexpr (kSetup) {
-      if constexpr (kMethod == kMaskUnit) wcnt[gv] = (unsigned int)L.acc[sl];
-      else if constexpr (kCurlW<kMethod>) wsum[gv] = L.acc[sl];
+      if constexpr (kMethod == kMaskUnit) {
+        if (parts == 1) wcnt[gv] = (unsigned int)x;
+        else if (x) atomicAdd(&wcnt[gv], (unsigned int)x);
+      } else if constexpr (kCurlW<kMethod>) {
+        if (parts == 1) wsum[gv] = x;
+        else if (x != 0.0) unsafeAtomicAdd(&wsum[gv], x);
+      }
     } else if constexpr (!kCurlW<kMethod>) {
-      sumfx[gv] = L.acc[sl];
+      if (parts == 1) sumfx[gv] = x;
+      else if (x) fx_add(&sumfx[gv], x);
     } else {
-      sumd[gv] = L.acc[sl];
+      if (parts == 1) sumd[gv] = x;
+      else if (x != 0.0) unsafeAtomicAdd(&sumd[gv], x);
     }
   }
 }
@@ -626,10 +641,23 @@ hipError_t launch_tile_pass_masked(int method, int ntiles, const unsigned long l
   using V4 = typename Vec4<T>::type;
   const V4* f = static_cast<const V4*>(field);
   constexpr int kThreads = 1024;
+  const bool curl = method == kMaskSelect || method == kMaskWeighted;
+  const int parts = tile_parts(ntiles, curl);
+  if (parts > 1) {
+    const int64_t V = (int64_t)g.X * g.Y * g.Z;
+    hipError_t e = hipSuccess;
+    if (kSetup) {
+      if (curl) e = launch_fill_u32(wsum, 2 * V, 0u, st);
+      else if (method == kMaskUnit) e = launch_fill_u32(wcnt, V, 0u, st);
+    } else {
+      e = launch_fill_u32(curl ? static_cast<void*>(sumd) : sumfx, 2 * V, 0u, st);
+    }
+    if (e != hipSuccess) return e;
+  }
 #define OMNI_TM(M, B)                                                                           \
-  hipLaunchKernelGGL((k_tile_masked<T, M, B, kThreads, kSetup>), dim3(ntiles), dim3(kThreads), 0, \
-                     st, tile_ptr, segs, g, tg, wp, f, aux, F, wc, wn, cval, p0, p1, k, sc, sumfx, \
-                     sumd, segS, wcnt, wsum, src)
+  hipLaunchKernelGGL((k_tile_masked<T, M, B, kThreads, kSetup>), dim3(ntiles * parts),            \
+                     dim3(kThreads), 0, st, tile_ptr, segs, g, tg, wp, f, aux, F, wc, wn, cval, p0, \
+                     p1, k, sc, sumfx, sumd, segS, wcnt, wsum, src, parts)
   if (tg.bits == 3) {
     switch (method) {
       case kMaskPlain: OMNI_TM(kMaskPlain, 3); break;
@@ -673,9 +701,10 @@ hipError_t launch_rule_replay(int method, int64_t nrays, const unsigned int* nse
   rs.f = reinterpret_cast<uint32_t*>(base);
   rs.r = rs.f + planes * nv;
   rs.nval = nv;
+  const int parts = tile_parts(ntiles, curl);
 #define OMNI_RT(M, B)                                                                         \
-  hipLaunchKernelGGL((k_rule_tile<T, M, B>), dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g, \
-                     tg, wp, f, aux, rs)
+  hipLaunchKernelGGL((k_rule_tile<T, M, B>), dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr,  \
+                     segs, g, tg, wp, f, aux, rs, parts)
 #define OMNI_RT_M(B)                                  \
   switch (method) {                                   \
     case kMaskPlain: OMNI_RT(kMaskPlain, B); break;   \
@@ -969,11 +998,12 @@ k_tile_rows(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
 
 // The rows in tile layout (curl weights, and unit weights past the merged-
 // word format): the entries whose row is a voxel of tile t sit in
-// [tbase[t], tbase[t + 1]) in the order the tile pass emits them (source id,
-// the row's index among the tile's rows, weight), so the pass writes them
-// coalesced (a wavefront takes consecutive slots from one LDS counter) and
-// the iteration streams a tile's entries with neighbouring rays' sources side
-// by side.  kFill == false stores each tile's entry count into tcnt.
+// [tbase[t * parts], tbase[(t + 1) * parts]), each of the tile's `parts`
+// workgroups' in the order it emits them (source id, the row's index among
+// the tile's rows, weight), so the pass writes them coalesced (a wavefront
+// takes consecutive slots from one LDS counter) and the iteration streams a
+// tile's entries with neighbouring rays' sources side by side.  kFill == false
+// stores each workgroup's entry count into tcnt[t * parts + part].
 template <int kMethod, int kBits, bool kFill>
 __global__ void __launch_bounds__(1024)
 k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
@@ -983,14 +1013,15 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
                const int* __restrict__ sid, const int* __restrict__ tfirst,
                unsigned int* __restrict__ tcnt, const unsigned long long* __restrict__ tbase,
                unsigned int* __restrict__ esrc, unsigned short* __restrict__ erow,
-               double* __restrict__ ew) {
+               double* __restrict__ ew, int parts) {
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kVox = kTile * kTile * kTile;
   __shared__ double s_aux[kVox];
   __shared__ int s_sid[kVox];
   __shared__ unsigned int s_total;
-  const int tile = (int)xcd_block();
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tp.tile;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
@@ -1005,14 +1036,15 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
   }
   __syncthreads();
   const int first = kFill ? tfirst[tile] : 0;
-  const unsigned long long base = kFill ? tbase[tile] : 0ull;
+  const unsigned long long base = kFill ? tbase[tile * parts + (int)tp.part] : 0ull;
   const int lane = threadIdx.x & 63;
   auto gvox = [&](int l) -> int64_t {
     return (int64_t)(ox + (l & kTileMask)) + (int64_t)(oy + ((l >> kBits) & kTileMask)) * sy +
            (int64_t)(oz + (l >> (2 * kBits))) * sz;
   };
   const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
-  for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
+  for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
     const SegRec sr = segs[jj];
     const uint32_t f = F[sr.g];
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
@@ -1085,7 +1117,7 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
   }
   if constexpr (!kFill) {
     __syncthreads();
-    if (threadIdx.x == 0) tcnt[tile] = s_total;
+    if (threadIdx.x == 0) tcnt[tile * parts + (int)tp.part] = s_total;
   }
 }
 
@@ -1471,6 +1503,10 @@ hipError_t launch_widen_keys(int64_t n, const unsigned int* esrc, unsigned long 
   return hipGetLastError();
 }
 
+int tile_entries_parts(int method, int ntiles) {
+  return tile_parts(ntiles, method == kMaskSelect || method == kMaskWeighted);
+}
+
 hipError_t launch_tile_entries(bool fill, int method, int ntiles,
                                const unsigned long long* tile_ptr, const SegRec* segs, GridDesc g,
                                TileGrid tg, const WalkParams& wp, const double* aux,
@@ -1479,9 +1515,11 @@ hipError_t launch_tile_entries(bool fill, int method, int ntiles,
                                unsigned int* tcnt, const unsigned long long* tbase,
                                unsigned int* esrc, unsigned short* erow, double* ew,
                                hipStream_t st) {
+  const int parts = tile_entries_parts(method, ntiles);
 #define OMNI_TE(M, B, FL)                                                                       \
-  hipLaunchKernelGGL((k_tile_entries<M, B, FL>), dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, \
-                     g, tg, wp, aux, F, wc, wn, runsrc, sid, tfirst, tcnt, tbase, esrc, erow, ew)
+  hipLaunchKernelGGL((k_tile_entries<M, B, FL>), dim3(ntiles * parts), dim3(1024), 0, st,         \
+                     tile_ptr, segs, g, tg, wp, aux, F, wc, wn, runsrc, sid, tfirst, tcnt, tbase,  \
+                     esrc, erow, ew, parts)
 #define OMNI_TE_B(M, FL)                  \
   do {                                    \
     if (tg.bits == 3) OMNI_TE(M, 3, FL);  \

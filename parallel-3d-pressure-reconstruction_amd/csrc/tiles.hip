@@ -16,6 +16,8 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "launch.hpp"
 #include "tiles.hpp"
@@ -178,7 +180,7 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
             const unsigned int* __restrict__ vcnt,
             const double* __restrict__ pbuf0, const double* __restrict__ pbuf1,
             const DevScalars* __restrict__ sc, T* __restrict__ segval,
-            long long* __restrict__ out) {
+            long long* __restrict__ out, int parts) {
   using V4 = typename Vec4<T>::type;
   constexpr int kTileBits = kBits;
   constexpr int kTile = 1 << kBits;
@@ -190,8 +192,15 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
   constexpr int kPlane = kHalo ? kHaloVox : kTileVox;
   __shared__ TileLds<T, kTileVox, kHaloVox, kMode> L;
   // contiguous tile ranges per XCD: neighbouring tiles share an L2
-  const int tb = (int)xcd_block();
-  const int tile = tile_list ? tile_list[tb] : tb;
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tile_list ? tile_list[tp.tile] : tp.tile;
+  // kSourceSums walks the compact list of the tile's segments that reach a
+  // source voxel and kLocalSum the tile's segments in value-slot order (one
+  // range per tile: coalesced slot stores); kFull the length groups
+  constexpr int kStride = kMode == kFull ? kLenBuckets : 1;
+  const unsigned long long b = tile_ptr[tile * kStride], e = tile_ptr[(tile + 1) * kStride];
+  // (parts > 1: the output is cleared before the launch)
+  if (parts > 1 && b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kTileBits, oy = ty << kTileBits, oz = tz << kTileBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
@@ -228,18 +237,13 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
   __syncthreads();
   const double scale = sc->scale;
   const double* __restrict__ ps = ((sc->kstar - 1) & 1) ? pbuf1 : pbuf0;
-  // kSourceSums walks the compact list of the tile's segments that reach a
-  // source voxel and kLocalSum the tile's segments in value-slot order (one
-  // range per tile: coalesced slot stores); kFull the length groups
-  constexpr int kStride = kMode == kFull ? kLenBuckets : 1;
-  const unsigned long long b = tile_ptr[tile * kStride], e = tile_ptr[(tile + 1) * kStride];
   // software pipeline over a thread's segments: the record two segments
   // ahead and the values the next segment starts from (its carry, entry
   // term and source pressure) are in flight while this segment is walked
   struct Pre {
     double pin = 0.0, cv = 0.0;
   };
-  const unsigned int bd = blockDim.x;
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
   auto fetch = [&](const SegRec& r, unsigned long long jj) {
     Pre q;
     const bool fs = (r.info >> 21) & 1u;
@@ -250,7 +254,7 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
     (void)jj;
     return q;
   };
-  unsigned long long j = b + threadIdx.x;
+  unsigned long long j = part_begin(b, tp);
   SegRec r1, r2;
   Pre p1;
   if (j < e) r1 = segs[j];
@@ -373,12 +377,20 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
     const int64_t v = i + j * sy + k * sz;
     const int sl = lds_slot<kBits>(l);
     // (every visit of v is walked by this tile: cnt[v] biased adds)
-    if constexpr (kMode == kFull)
-      out[v] = (long long)((unsigned long long)L.acc[sl] -
-                           (unsigned long long)vcnt[v] * 0x4338000000000000ull);
+    // several parts: their biased sums add up in memory (modulo 2^64, in any
+    // order), the first one takes the bias of all of the voxel's visits off
+    if constexpr (kMode == kFull) {
+      unsigned long long x = (unsigned long long)L.acc[sl];
+      if (tp.part == 0) x -= (unsigned long long)vcnt[v] * 0x4338000000000000ull;
+      if (parts == 1) out[v] = (long long)x;
+      else if (x) atomicAdd(reinterpret_cast<unsigned long long*>(&out[v]), x);
+    }
     if constexpr (kMode == kSourceSums) {
       const int s = L.sidl[sl];
-      if (s >= 0) out[s] = L.acc[sl];
+      if (s >= 0) {
+        if (parts == 1) out[s] = L.acc[sl];
+        else fx_add(&out[s], L.acc[sl]);
+      }
     }
   }
 }
@@ -764,6 +776,21 @@ k_scan_final(const unsigned int* __restrict__ cnt, int64_t n, int words,
 // ---------------------------------------------------------------------------
 // Launchers.
 
+// One workgroup per tile leaves CUs idle on small grids (32^3: 8 tiles;
+// 100 x 47 x 38: 63) and gives others an uneven last round, while every
+// further workgroup of a tile stages the tile once more and adds its sums in
+// memory.  Measured on whole calls (parts 1 / 2 / 4 / 8 / 16, ms): plain and
+// unit weights 100 x 47 x 38 (63 tiles) 1.44 / 1.13 / 0.97 / 0.99 / 1.01,
+// 160 x 128 x 96 (480) 4.84 / 4.84 / 4.94 / 4.98 / 5.19, 256^3 (4096) 15.1 /
+// 15.2 / 15.6 / 16.1 / 16.9; curl weights, whose steps cost more, 100 x 47 x
+// 38 16.2 / 9.1 / 5.4 / 5.5 / 5.4, 112 x 96 x 80 (210) 13.8 / 13.3 / 13.3 /
+// 12.5 / 12.4, 128^3 (512) 14.1 / 13.7 / 13.5 / 13.5 / 13.7.  So about 384
+// workgroups in all, 1536 with curl weights, and at most 16 per tile.
+int tile_parts(int ntiles, bool curl_weights) {
+  const int units = curl_weights ? 1536 : 384;
+  return std::max(1, std::min(16, (units + ntiles - 1) / std::max(ntiles, 1)));
+}
+
 hipError_t launch_tile_count(const RayRec* rays, int64_t nrays, const DirConst* dirs, GridDesc g,
                              TileGrid tg, unsigned int* nseg, unsigned int* tile_cnt,
                              const SrcRows& rows, hipStream_t st) {
@@ -859,9 +886,11 @@ static void tile_pass_threads(int threads, int ntiles, const int* tile_list,
                               const unsigned int* vcnt, const double* p0,
                               const double* p1, const DevScalars* sc, T* segval,
                               long long* out, hipStream_t st) {
+  const int parts = tile_parts(ntiles, false);
 #define OMNI_TILE(NT)                                                                        \
-  hipLaunchKernelGGL((k_tile_pass<T, kMode, kBits, NT>), dim3(ntiles), dim3(NT), 0, st,       \
-                     tile_list, tile_ptr, segs, g, tg, wp, f, sid, vcnt, p0, p1, sc, segval, out)
+  hipLaunchKernelGGL((k_tile_pass<T, kMode, kBits, NT>), dim3(ntiles * parts), dim3(NT), 0, st, \
+                     tile_list, tile_ptr, segs, g, tg, wp, f, sid, vcnt, p0, p1, sc, segval,    \
+                     out, parts)
   if (threads <= 256) OMNI_TILE(256);
   else if (threads <= 512) OMNI_TILE(512);
   else OMNI_TILE(1024);
@@ -899,9 +928,14 @@ hipError_t launch_tile_pass(int mode, int threads, int ntiles, const int* tile_l
   else if (mode == kSourceSums)
     tile_pass_bits<T, kSourceSums>(threads, ntiles, tile_list, tile_ptr, segs, g, tg, wp, f, sid,
                                    vcnt, p0, p1, sc, segval, out, st);
-  else
+  else {
+    if (tile_parts(ntiles, false) > 1) {
+      const hipError_t e = launch_fill_u32(out, 2 * (int64_t)g.X * g.Y * g.Z, 0u, st);
+      if (e != hipSuccess) return e;
+    }
     tile_pass_bits<T, kFull>(threads, ntiles, tile_list, tile_ptr, segs, g, tg, wp, f, sid,
                              vcnt, p0, p1, sc, segval, out, st);
+  }
   return hipGetLastError();
 }
 

@@ -31,6 +31,26 @@ __device__ __forceinline__ int tile_of(int i, int j, int k, const TileGrid& tg) 
   return (i >> b) + (j >> b) * tg.ntx + (k >> b) * tg.ntx * tg.nty;
 }
 
+// Workgroups per tile of a tile pass: the tile's segments dealt in blocks to
+// `parts` workgroups, each of which stages the tile for itself and adds its
+// sums to the tile's voxels in memory (one workgroup stores them).  See
+// tile_parts for when.
+struct TilePart {
+  int tile;           // position in the launch's tile list
+  unsigned int part;  // 0 .. parts - 1
+};
+__device__ __forceinline__ TilePart tile_part(unsigned int block, int parts) {
+  TilePart q;
+  q.tile = (int)(block / (unsigned int)parts);
+  q.part = block - (unsigned int)q.tile * (unsigned int)parts;
+  return q;
+}
+// first segment of this thread, and the stride of its segments
+__device__ __forceinline__ unsigned long long part_begin(unsigned long long b, TilePart q) {
+  return b + (unsigned long long)q.part * blockDim.x + threadIdx.x;
+}
+int tile_parts(int ntiles, bool curl_weights);
+
 // LDS slot of in-tile voxel l = x + (y << b) + (z << 2b): x is XORed with
 // bits of y and z, so that voxels one step apart along y or z -- the
 // positions of neighbouring parallel rays at the same step -- fall in
@@ -247,6 +267,9 @@ struct MaskChunk {
   unsigned long long begin, end;  // entries [begin, end) of one tile
   int tile, pad;
 };
+// (tcnt and tbase: one count / offset per workgroup, tile_entries_parts of
+// them per tile, and the total)
+int tile_entries_parts(int method, int ntiles);
 hipError_t launch_tile_entries(bool fill, int method, int ntiles,
                                const unsigned long long* tile_ptr, const SegRec* segs, GridDesc g,
                                TileGrid tg, const WalkParams& wp, const double* aux,
