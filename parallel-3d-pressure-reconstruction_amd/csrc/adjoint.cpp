@@ -32,65 +32,6 @@ int io_dtype(const omni3d_ctx* ctx) {
   return ctx->prm.precision == OMNI3D_FP64 ? OMNI3D_F64 : OMNI3D_F32;
 }
 
-// Merged words of sorted CSR rows in the forward iteration's layout (groups
-// of 8 chunks, 4 from 2^21 sources on, sized to about equal entries and as
-// many as fill the CUs evenly) when they fit it -- sources below 2^22, rows
-// shorter than 4096 entries (int64 row sums); *dense tells whether they
-// were built, *gchunks / *ngroups / grow the groups.
-int build_row_words(omni3d_ctx* ctx, int nS, unsigned long long n, const DevBuf& tptr,
-                    const DevBuf& key, DevBuf* tdent, DevBuf* twptr, DevBuf* grow,
-                    int* gchunks, int* ngroups, bool* dense) {
-  hipStream_t st = ctx->stream;
-  *dense = false;
-  std::vector<unsigned long long> hp((size_t)nS + 1);
-  OMNI_TRY_HIP(ctx, hipMemcpyAsync(hp.data(), tptr.as<void>(),
-                                   sizeof(unsigned long long) * (nS + 1), hipMemcpyDeviceToHost,
-                                   st));
-  OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
-  unsigned long long mx = 0;
-  for (int r = 0; r < nS; r++) mx = std::max(mx, hp[r + 1] - hp[r]);
-  if (!(nS < (1 << 22) && mx < 4096 && n > 0 && n < (1ull << 31))) return OMNI3D_OK;
-  const int grp = nS < (1 << 21) ? 8 : 4;
-  int dev = 0, ncu = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  std::vector<int> hgrow, hrg((size_t)nS);
-  balance_groups(hp, 64 * grp, std::max(ncu, 1), &hgrow, &hrg);
-  const int ng = (int)hgrow.size() - 1;
-  DevBuf rgroup;
-  OMNI_TRY_HIP(ctx, grow->alloc(sizeof(int) * hgrow.size()));
-  OMNI_TRY_HIP(ctx, rgroup.alloc(sizeof(int) * (size_t)nS));
-  OMNI_TRY_HIP(ctx, hipMemcpy(grow->as<void>(), hgrow.data(), sizeof(int) * hgrow.size(),
-                              hipMemcpyHostToDevice));
-  OMNI_TRY_HIP(ctx, hipMemcpy(rgroup.as<void>(), hrg.data(), sizeof(int) * (size_t)nS,
-                              hipMemcpyHostToDevice));
-  DevBuf ka, kb, tmp, flag, excl;
-  OMNI_TRY_HIP(ctx, ka.alloc(sizeof(unsigned long long) * n));
-  OMNI_TRY_HIP(ctx, kb.alloc(sizeof(unsigned long long) * n));
-  OMNI_TRY_HIP(ctx, tmp.alloc(dense_tmp_bytes((int64_t)n)));
-  OMNI_TRY_HIP(ctx, tdent->alloc(sizeof(unsigned int) * (n + 8)));
-  OMNI_TRY_HIP(ctx, launch_fill_u32(tdent->as<void>(), (int64_t)n + 8, 0u, st));
-  OMNI_TRY_HIP(ctx, build_dense_entries(nS, (int64_t)n, grp, tptr.as<unsigned long long>(),
-                                        key.as<unsigned long long>(), ka.as<unsigned long long>(),
-                                        kb.as<unsigned long long>(), tmp.as<void>(), tmp.size(),
-                                        tdent->as<unsigned int>(), st, rgroup.as<int>(),
-                                        grow->as<int>(), ng));
-  OMNI_TRY_HIP(ctx, flag.alloc(sizeof(unsigned int) * n));
-  OMNI_TRY_HIP(ctx, excl.alloc(sizeof(unsigned int) * n));
-  OMNI_TRY_HIP(ctx, twptr->alloc(sizeof(unsigned int) * (ng + 1)));
-  unsigned int nw = 0;
-  OMNI_TRY_HIP(ctx, merge_dense_entries(nS, (int64_t)n, grp, tptr.as<unsigned long long>(),
-                                        kb.as<unsigned long long>(), flag.as<unsigned int>(),
-                                        excl.as<unsigned int>(), tmp.as<void>(), tmp.size(),
-                                        tdent->as<unsigned int>(), twptr->as<unsigned int>(), &nw,
-                                        st, grow->as<int>(), ng));
-  OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
-  *gchunks = grp;
-  *ngroups = ng;
-  *dense = true;
-  return OMNI3D_OK;
-}
-
 // Transposed source rows of the plain method, kept with the plan: row s'
 // lists the source voxels that rays entering at s' visit after their entry
 // (the entries of the forward source rows, regrouped by their source).
@@ -123,11 +64,10 @@ int build_transposed_rows(omni3d_ctx* ctx) {
   OMNI_TRY_HIP(ctx, launch_sort_rows(nS, pl.tptr.as<unsigned long long>(),
                                      key.as<unsigned long long>(), st));
   {
-    bool dense = false;
-    const int rc = build_row_words(ctx, nS, n, pl.tptr, key, &pl.tdent, &pl.twptr, &pl.tgrow,
-                                   &pl.tgroup, &pl.tngroups, &dense);
+    const int rc = build_words(ctx, nS, 0, cu_count(), pl.tptr.as<unsigned long long>(),
+                               key.as<unsigned long long>(), pl.diag.as<unsigned int>(),
+                               pl.cnt.as<unsigned int>(), pl.slist.as<int>(), &pl.twords);
     if (rc) return rc;
-    pl.tdense = dense;
   }
   OMNI_TRY_HIP(ctx, pl.tent.alloc(sizeof(unsigned int) * (n + 1)));
   OMNI_TRY_HIP(ctx, launch_adj_narrow(key.as<unsigned long long>(), (int64_t)n,
@@ -166,7 +106,7 @@ int build_mask_rows(omni3d_ctx* ctx, const double* mask, MaskRows* mr) {
   if (nsrc >= (1ull << 31)) return fail(ctx, OMNI3D_ERR_ARG, "too many run starts");
   const int nS = (int)nsrc;
   mr->nS = nS;
-  mr->tdense = false;
+  mr->twords.valid = false;
   if (nS == 0) return OMNI3D_OK;
   OMNI_TRY_HIP(ctx, mr->sid.alloc(sizeof(int) * V));
   OMNI_TRY_HIP(ctx, mr->slist.alloc(sizeof(int) * nS));
@@ -194,11 +134,10 @@ int build_mask_rows(omni3d_ctx* ctx, const double* mask, MaskRows* mr) {
   OMNI_TRY_HIP(ctx, launch_sort_rows(nS, mr->tptr.as<unsigned long long>(),
                                      key.as<unsigned long long>(), st));
   {
-    bool dense = false;
-    const int rc = build_row_words(ctx, nS, n, mr->tptr, key, &mr->tdent, &mr->twptr, &mr->tgrow,
-                                   &mr->tgroup, &mr->tngroups, &dense);
+    const int rc = build_words(ctx, nS, 0, cu_count(), mr->tptr.as<unsigned long long>(),
+                               key.as<unsigned long long>(), nullptr, mr->cnt.as<unsigned int>(),
+                               mr->slist.as<int>(), &mr->twords);
     if (rc) return rc;
-    mr->tdense = dense;
   }
   OMNI_TRY_HIP(ctx, mr->tent.alloc(sizeof(unsigned int) * (n + 1)));
   OMNI_TRY_HIP(ctx, launch_adj_narrow(key.as<unsigned long long>(), (int64_t)n,
@@ -378,12 +317,11 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
       }
     }
     if (P.max_iterations > 1 && nS > 0) {
-      OMNI_TRY_HIP(ctx, ctx->adj_s.alloc(sizeof(double) * 7 * (size_t)nS));
+      OMNI_TRY_HIP(ctx, ctx->adj_s.alloc(sizeof(double) * 6 * (size_t)nS));
       double* ts = ctx->adj_s.as<double>();
       double* h[2] = {ts + nS, ts + 2 * (size_t)nS};
       double* w[2] = {ts + 3 * (size_t)nS, ts + 4 * (size_t)nS};
       double* cs = ts + 5 * (size_t)nS;
-      double* w3 = ts + 6 * (size_t)nS;
       OMNI_TRY_HIP(ctx, launch_adj_scale(V, y, cnt, u, st));
       OMNI_TRY_HIP(ctx, launch_fill_f64(t, V, 0.0, st));
       OMNI_TRY_HIP(ctx, gather(u, t));
@@ -391,36 +329,30 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
       const int M = P.max_iterations - 2;
       // the transposed rows as merged words: the plain method's (with the
       // plan) or the plain-mask rule's (with the mask)
-      const bool tdense = mask_rule ? mr.tdense : pl.tdense;
-      const int tgroup = mask_rule ? mr.tgroup : pl.tgroup;
-      const int tngroups = mask_rule ? mr.tngroups : pl.tngroups;
-      const DevBuf& twptr = mask_rule ? mr.twptr : pl.twptr;
-      const DevBuf& tdent = mask_rule ? mr.tdent : pl.tdent;
-      const DevBuf& tgrow = mask_rule ? mr.tgrow : pl.tgrow;
-      if (tdense && M > 0) {
-        // w <- (t + diag w + sum w) / C is the forward iteration's form: the
-        // grouped kernel on the transposed merged words (exact fixed-point
-        // row sums), t as its source term, w over three buffers (a source
-        // with C = 0 keeps w = 0, as in the one-wavefront-per-row steps)
-        const unsigned int gg = grouped_grid_n(tngroups);
+      const WordPlan& twords = mask_rule ? mr.twords : pl.twords;
+      if (twords.valid && M > 0) {
+        // w <- (t + diag w + sum w) / C is the forward iteration's form: its
+        // kernel on the transposed merged words (exact fixed-point row sums),
+        // t as its source term (a source with C = 0 keeps w = 0, as in the
+        // one-wavefront-per-row steps)
         OMNI_TRY_HIP(ctx, ctx->adj_sc.alloc(sizeof(DevScalars)));
-        OMNI_TRY_HIP(ctx, ctx->adj_part.alloc(sizeof(double) * 4 * (size_t)gg));
         OMNI_TRY_HIP(ctx, ctx->adj_bs.alloc(sizeof(long long) * (size_t)nS));
         DevScalars* asc = ctx->adj_sc.as<DevScalars>();
         OMNI_TRY_HIP(ctx, launch_fill_u32(asc, sizeof(DevScalars) / 4, 0u, st));
         OMNI_TRY_HIP(ctx, launch_absmax<double>(ts, nS, &asc->pmax_bits, st));
         OMNI_TRY_HIP(ctx, launch_adj_fixed(nS, ts, asc, ctx->adj_bs.as<long long>(), st));
         OMNI_TRY_HIP(ctx, launch_absmax<double>(w[0], nS, &asc->itmax_bits[0], st));
-        double* pb3[3] = {w[0], w[1], w3};
-        for (int k = 1; k <= M; k++)
-          OMNI_TRY_HIP(ctx, launch_iterate_dense(tgroup, 0, k, nS, nullptr,
-                                                 twptr.as<unsigned int>(),
-                                                 tdent.as<unsigned int>(), diagp, slist, cnt,
-                                                 ctx->adj_bs.as<long long>(), nullptr, 0,
-                                                 pb3[(k - 1) % 3], pb3[k % 3], asc,
-                                                 ctx->adj_part.as<double>(), M, 0.0, st, nullptr,
-                                                 nullptr, nullptr, tgrow.as<int>(), tngroups));
-        OMNI_TRY_HIP(ctx, launch_adj_src_out(nS, slist, pb3[M % 3], cs, z, st));
+        OMNI_TRY_HIP(ctx, ctx->word_part.alloc(word_part_bytes(twords.G)));
+        WordIter it;
+        it.m = twords.mat();
+        it.slist = slist;
+        it.bs = ctx->adj_bs.as<long long>();
+        it.pb[0] = w[0];
+        it.pb[1] = w[1];
+        it.sc = asc;
+        it.part = ctx->word_part.as<double>();
+        for (int k = 1; k <= M; k++) OMNI_TRY_HIP(ctx, launch_iterate_words(k, it, 0.0, st));
+        OMNI_TRY_HIP(ctx, launch_adj_src_out(nS, slist, w[M & 1], cs, z, st));
       } else {
         int cur = 0;
         for (int m = 2; m < P.max_iterations; m++) {

@@ -356,6 +356,88 @@ int build_tiles(omni3d_ctx* ctx, const GridDesc& g, int64_t nrays, SrcRowBuild* 
   return OMNI3D_OK;
 }
 
+bool increments(const omni3d_params& P) {
+  return P.precision == OMNI3D_FP32_KAHAN && !std::getenv("OMNI3D_NO_INCREMENTS");
+}
+
+int cu_count() {
+  int dev = 0, n = 256;
+  if (hipGetDevice(&dev) == hipSuccess)
+    (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+  return std::max(n, 1);
+}
+
+int build_words(omni3d_ctx* ctx, int nS, int chunks, int fill, const unsigned long long* rowptr,
+                const unsigned long long* key, const unsigned int* diag, const unsigned int* cnt,
+                const int* slist, WordPlan* out) {
+  hipStream_t st = ctx->stream;
+  out->valid = false;
+  if (nS < 1 || nS >= word_max_sources(4)) return OMNI3D_OK;
+  // where 4 wavefronts per group reach every CU, 8 only cost their launch: 32^3
+  // 5.3 us an iteration with 4, 5.6 with 8; 160x128x96 (past the line) 13.5 each
+  if (chunks == 0) chunks = nS <= word_rows(4) * fill ? 4 : 8;
+  if (nS >= word_max_sources(8)) chunks = 4;
+  std::vector<unsigned long long> hrp((size_t)nS + 1);
+  OMNI_TRY_HIP(ctx, hipMemcpyAsync(hrp.data(), rowptr, sizeof(unsigned long long) * hrp.size(),
+                                   hipMemcpyDeviceToHost, st));
+  OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
+  const unsigned long long n = hrp[nS];
+  unsigned long long longest = 0;
+  for (int r = 0; r < nS; r++) longest = std::max(longest, hrp[r + 1] - hrp[r]);
+  if (longest >= 4096 || n == 0 || n >= (1ull << 31)) return OMNI3D_OK;
+  std::vector<int> hgrow, hrg((size_t)nS);
+  balance_groups(hrp, word_rows(chunks), std::max(fill, 1), &hgrow, &hrg);
+  const int ng = (int)hgrow.size() - 1;
+  DevBuf rgroup, ka, kb, tmp, flag, excl, first, nblk, btmp;
+  OMNI_TRY_HIP(ctx, out->grow.alloc(sizeof(int) * hgrow.size()));
+  OMNI_TRY_HIP(ctx, rgroup.alloc(sizeof(int) * (size_t)nS));
+  OMNI_TRY_HIP(ctx, hipMemcpyAsync(out->grow.as<void>(), hgrow.data(), sizeof(int) * hgrow.size(),
+                                   hipMemcpyHostToDevice, st));
+  OMNI_TRY_HIP(ctx, hipMemcpyAsync(rgroup.as<void>(), hrg.data(), sizeof(int) * (size_t)nS,
+                                   hipMemcpyHostToDevice, st));
+  OMNI_TRY_HIP(ctx, ka.alloc(sizeof(unsigned long long) * n));
+  OMNI_TRY_HIP(ctx, kb.alloc(sizeof(unsigned long long) * n));
+  OMNI_TRY_HIP(ctx, tmp.alloc(dense_tmp_bytes((int64_t)n)));
+  OMNI_TRY_HIP(ctx, sort_entry_keys(nS, (int64_t)n, 32 - word_row_shift(chunks), rowptr, key,
+                                    rgroup.as<int>(), out->grow.as<int>(), ng,
+                                    ka.as<unsigned long long>(), kb.as<unsigned long long>(),
+                                    tmp.as<void>(), tmp.size(), st));
+  OMNI_TRY_HIP(ctx, flag.alloc(sizeof(unsigned int) * n));
+  OMNI_TRY_HIP(ctx, excl.alloc(sizeof(unsigned int) * n));
+  OMNI_TRY_HIP(ctx, launch_word_flags((int64_t)n, kb.as<unsigned long long>(),
+                                      flag.as<unsigned int>(), st));
+  unsigned int nw = 0, nb = 0;
+  OMNI_TRY_HIP(ctx, exclusive_sums((int64_t)n, flag.as<unsigned int>(), excl.as<unsigned int>(),
+                                   tmp.as<void>(), tmp.size(), &nw, st));
+  OMNI_TRY_HIP(ctx, first.alloc(sizeof(unsigned int) * ng));
+  OMNI_TRY_HIP(ctx, nblk.alloc(sizeof(unsigned int) * ((size_t)ng + 1)));
+  OMNI_TRY_HIP(ctx, btmp.alloc(dense_tmp_bytes((int64_t)ng + 1)));
+  OMNI_TRY_HIP(ctx, out->bptr.alloc(sizeof(unsigned int) * ((size_t)ng + 1)));
+  OMNI_TRY_HIP(ctx, launch_word_blocks(ng, out->grow.as<int>(), rowptr, (int64_t)n,
+                                       excl.as<unsigned int>(), nw, first.as<unsigned int>(),
+                                       nblk.as<unsigned int>(), st));
+  OMNI_TRY_HIP(ctx, exclusive_sums((int64_t)ng + 1, nblk.as<unsigned int>(),
+                                   out->bptr.as<unsigned int>(), btmp.as<void>(), btmp.size(), &nb,
+                                   st));
+  OMNI_TRY_HIP(ctx, out->words.alloc(sizeof(unsigned int) * kWordBlock * ((size_t)nb + 1)));
+  OMNI_TRY_HIP(ctx, launch_word_write((int64_t)n, chunks, kb.as<unsigned long long>(),
+                                      flag.as<unsigned int>(), excl.as<unsigned int>(),
+                                      first.as<unsigned int>(), out->bptr.as<unsigned int>(), nb,
+                                      out->words.as<unsigned int>(), st));
+  OMNI_TRY_HIP(ctx, out->dc.alloc(sizeof(uint4) * (size_t)nS));
+  OMNI_TRY_HIP(ctx, launch_word_rowdata(nS, rowptr, diag, cnt, slist, out->dc.as<uint4>(), st));
+  OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
+  out->nS = nS;
+  out->G = ng;
+  out->chunks = chunks;
+  out->nwords = (int64_t)nb * kWordBlock;
+  out->valid = true;
+  if (std::getenv("OMNI3D_VERBOSE"))
+    std::fprintf(stderr, "omni3d words: %d rows, %llu entries in %u words, %u blocks, %d groups of %d chunks\n",
+                 nS, n, nw, nb, ng, chunks);
+  return OMNI3D_OK;
+}
+
 // Builds the geometry plan: ray list, visit counts, source voxels and the CSR
 // of visits that land on source voxels.
 int build_plan(omni3d_ctx* ctx) {
@@ -487,29 +569,40 @@ int build_plan(omni3d_ctx* ctx) {
   OMNI_TRY_HIP(ctx, hipMemcpyAsync(mxh, mx.as<unsigned int>(), 8, hipMemcpyDeviceToHost, st));
   OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
   // CSR of visits landing on source voxels (counted and filled by the
-  // tile walks): each row's keys sorted
+  // tile walks)
   const unsigned long long nnz = rows.nnz;
   DevBuf& key = rows.key;
-  OMNI_TRY_HIP(ctx, launch_sort_rows(nS, pl.rowptr.as<unsigned long long>(),
-                                     key.as<unsigned long long>(), st));
-  // the dense layout (default iteration) unless sizes exceed its word format:
-  // 24-bit source ids, rows shorter than 4096 entries (int64 row sums of
-  // terms below 2^51); otherwise (e.g. thousands of directions) the masked
-  // sliced-ELL layout
   const char* iter_env = std::getenv("OMNI3D_ITER");
-  // groups of 8 (4) chunks use merged words with 21-bit (22-bit) sources
-  int grp = ctx->dense_group;
-  if (grp == 8 && nS >= (1 << 21)) grp = 4;
-  if (grp == 4 && nS >= (1 << 22)) grp = 1;
+  pl.dense = pl.words.valid = pl.staged = false;
+  pl.ncell = pl.nwords = 0;
 #ifdef OMNI3D_LAYOUT_STUDY
   const bool want_slots = iter_env && (std::strcmp(iter_env, "slots") == 0 ||
                                        std::strcmp(iter_env, "staged") == 0);
 #else
   const bool want_slots = iter_env && std::strcmp(iter_env, "slots") == 0;
 #endif
-  const bool use_dense = !want_slots && nS < (1 << (32 - dense_row_bits(grp))) &&
-                         mxh[0] < 4096u && nnz > 0 && nnz < (1ull << 31);
-  pl.ncell = 0;
+  // merged words (the default iteration) unless sizes exceed their format;
+  // as many groups as fill the CUs evenly, so that the launch does not wait
+  // on the largest uniform group (256^3: 768 groups 34.3 us, 1024 37 us; the
+  // least, one per CU, at small sizes: 512 cost 160x128x96 15.4 us for 13.5);
+  // a batch's snapshots share a launch and its CUs
+  if (!want_slots && ctx->dense_group != 1 && mxh[0] < 4096u) {
+    const int rc = build_words(ctx, nS, ctx->dense_group, std::max(1, cu_count() / ctx->cu_share),
+                               pl.rowptr.as<unsigned long long>(), key.as<unsigned long long>(),
+                               pl.diag.as<unsigned int>(), pl.cnt.as<unsigned int>(),
+                               pl.slist.as<int>(), &pl.words);
+    if (rc) return rc;
+    pl.nwords = pl.words.nwords;
+  }
+  if (!pl.words.valid) {
+  // each row's keys sorted
+  OMNI_TRY_HIP(ctx, launch_sort_rows(nS, pl.rowptr.as<unsigned long long>(),
+                                     key.as<unsigned long long>(), st));
+  // dense words unless sizes exceed their format: 24-bit source ids, rows
+  // shorter than 4096 entries (int64 row sums of terms below 2^51); otherwise
+  // (e.g. thousands of directions) the masked sliced-ELL layout
+  const bool use_dense = !want_slots && nS < (1 << (32 - kDenseRowBits)) && mxh[0] < 4096u &&
+                         nnz > 0 && nnz < (1ull << 31);
   if (!use_dense) {
     // masked sliced-ELL copy of the sorted rows for the iteration
     if (D > 4096) return fail(ctx, OMNI3D_ERR_ARG, "at most 4096 directions");
@@ -540,7 +633,6 @@ int build_plan(omni3d_ctx* ctx) {
     pl.ncell = (int64_t)nm;
   }
   {
-    pl.dense = false;
     if (use_dense) {
       DevBuf ka, kb, tmp;
       OMNI_TRY_HIP(ctx, ka.alloc(sizeof(unsigned long long) * nnz));
@@ -549,80 +641,24 @@ int build_plan(omni3d_ctx* ctx) {
       // slack after the words: the iteration stages them with 16-byte loads
       OMNI_TRY_HIP(ctx, pl.dent.alloc(sizeof(unsigned int) * (nnz + 8)));
       OMNI_TRY_HIP(ctx, hipMemsetAsync(pl.dent.as<void>(), 0, sizeof(unsigned int) * (nnz + 8), st));
-      // groups of at most 64 * grp consecutive rows holding about equal entries:
-      // one workgroup per group, as many groups as fill the CUs evenly, so
-      // the launch does not wait on the largest uniform group
-      DevBuf rgroup;
-      if (grp > 1) {
-        std::vector<unsigned long long> hrp((size_t)nS + 1);
-        OMNI_TRY_HIP(ctx, hipMemcpy(hrp.data(), pl.rowptr.as<void>(),
-                                    sizeof(unsigned long long) * ((size_t)nS + 1),
-                                    hipMemcpyDeviceToHost));
-        int dev = 0, ncu = 256;
-        if (hipGetDevice(&dev) == hipSuccess)
-          (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        ncu = ctx->groups_fill_cus ? std::max(ncu, 1) : 1;
-        std::vector<int> hgrow, hrg((size_t)nS);
-        balance_groups(hrp, 64 * grp, ncu, &hgrow, &hrg);
-        pl.dense_ngroups = (int)hgrow.size() - 1;
-        OMNI_TRY_HIP(ctx, pl.dense_grow.alloc(sizeof(int) * hgrow.size()));
-        OMNI_TRY_HIP(ctx, rgroup.alloc(sizeof(int) * (size_t)std::max(nS, 1)));
-        OMNI_TRY_HIP(ctx, hipMemcpy(pl.dense_grow.as<void>(), hgrow.data(),
-                                    sizeof(int) * hgrow.size(), hipMemcpyHostToDevice));
-        OMNI_TRY_HIP(ctx, hipMemcpy(rgroup.as<void>(), hrg.data(), sizeof(int) * (size_t)nS,
-                                    hipMemcpyHostToDevice));
-      }
-      OMNI_TRY_HIP(ctx, build_dense_entries(nS, (int64_t)nnz, grp, pl.rowptr.as<unsigned long long>(),
-                                            key.as<unsigned long long>(),
-                                            ka.as<unsigned long long>(), kb.as<unsigned long long>(),
-                                            tmp.as<void>(), tmp.size(), pl.dent.as<unsigned int>(),
-                                            st, grp > 1 ? rgroup.as<int>() : nullptr,
-                                            grp > 1 ? pl.dense_grow.as<int>() : nullptr,
-                                            pl.dense_ngroups));
+      OMNI_TRY_HIP(ctx, sort_entry_keys(nS, (int64_t)nnz, kDenseRowBits,
+                                        pl.rowptr.as<unsigned long long>(),
+                                        key.as<unsigned long long>(), nullptr, nullptr, 0,
+                                        ka.as<unsigned long long>(), kb.as<unsigned long long>(),
+                                        tmp.as<void>(), tmp.size(), st));
+      OMNI_TRY_HIP(ctx, launch_dense_words((int64_t)nnz, kb.as<unsigned long long>(),
+                                           pl.dent.as<unsigned int>(), st));
       pl.nwords = (int64_t)nnz;
-      if (grp > 1) {
-        DevBuf flag, excl;
-        OMNI_TRY_HIP(ctx, flag.alloc(sizeof(unsigned int) * nnz));
-        OMNI_TRY_HIP(ctx, excl.alloc(sizeof(unsigned int) * nnz));
-        const int ng = pl.dense_ngroups;
-        OMNI_TRY_HIP(ctx, pl.dense_wptr.alloc(sizeof(unsigned int) * (ng + 1)));
-        unsigned int nw = 0;
-        OMNI_TRY_HIP(ctx, merge_dense_entries(nS, (int64_t)nnz, grp,
-                                              pl.rowptr.as<unsigned long long>(),
-                                              kb.as<unsigned long long>(), flag.as<unsigned int>(),
-                                              excl.as<unsigned int>(), tmp.as<void>(), tmp.size(),
-                                              pl.dent.as<unsigned int>(),
-                                              pl.dense_wptr.as<unsigned int>(), &nw, st,
-                                              pl.dense_grow.as<int>(), ng));
-        pl.nwords = nw;
-      }
       OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
       pl.dense = true;
-      pl.dense_group = grp;
-      if (std::getenv("OMNI3D_VERBOSE")) {
-        std::fprintf(stderr, "omni3d plan: %lld entries in %lld dense words (groups of %d chunks)\n",
-                     (long long)nnz, (long long)pl.nwords, grp);
-        if (grp > 1) {
-          const int ng = pl.dense_ngroups;
-          std::vector<unsigned int> wp(ng + 1);
-          if (hipMemcpy(wp.data(), pl.dense_wptr.as<void>(), sizeof(unsigned int) * (ng + 1),
-                        hipMemcpyDeviceToHost) == hipSuccess) {
-            std::vector<unsigned int> n(ng);
-            for (int i = 0; i < ng; i++) n[i] = wp[i + 1] - wp[i];
-            std::sort(n.begin(), n.end());
-            std::fprintf(stderr, "omni3d plan: words per group min %u median %u p90 %u max %u\n",
-                         n[0], n[ng / 2], n[(ng * 9) / 10], n[ng - 1]);
-          }
-        }
-      }
     }
-    pl.staged = false;
 #ifdef OMNI3D_LAYOUT_STUDY
     if (iter_env && std::strcmp(iter_env, "staged") == 0) {
       const int rc = build_staged(ctx, nS, D, (int64_t)nnz);
       if (rc) return rc;
     }
 #endif
+  }
   }
   OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
   pl.X = X;
@@ -812,35 +848,37 @@ int run_affine(omni3d_ctx* ctx, int seed) {
   OMNI_TRY_HIP(ctx, ctx->partials.alloc(
                         sizeof(double) * 2 *
                         std::max(iterate_grid(pl.nS),
-                                 std::max(study_grid(pl.nS),
-                                          std::max(dense_grid(pl.nS),
-                                                   2 * grouped_grid_n(pl.dense_ngroups))))));
+                                 std::max(study_grid(pl.nS), dense_grid(pl.nS)))));
   if (phase != 2) {
     OMNI_TRY_HIP(ctx, launch_gather_sources(pl.slist.as<int>(), pl.nS, pinit, ctx->ps0.as<double>(), st));
     // max |p_S| of the starting values: the fixed-point scale of iteration 1
     OMNI_TRY_HIP(ctx, launch_absmax<double>(ctx->ps0.as<double>(), pl.nS, &sc->itmax_bits[0], st));
   }
   double* pbuf[2] = {ctx->ps0.as<double>(), ctx->ps1.as<double>()};
-  // the grouped dense iteration runs one launch ahead of its stop rule, so
-  // p_S rotates over three buffers and p_S^{k*-1} is copied out after the loop
-  const bool rot3 = pl.dense && pl.dense_group > 1 && !pl.staged && P.max_iterations > 0;
-  double* pb3[3] = {pbuf[0], pbuf[1], nullptr};
-  if (rot3) {
-    OMNI_TRY_HIP(ctx, ctx->ps2.alloc(sizeof(double) * ns16));
-    OMNI_TRY_HIP(ctx, ctx->psel.alloc(sizeof(double) * ns16));
-    pb3[2] = ctx->ps2.as<double>();
-  }
-  // FP32 ray sums: the grouped dense iteration runs in increment form
-  const bool inc = std::is_same<T, float>::value && pl.dense && pl.dense_group > 1 &&
-                   !std::getenv("OMNI3D_NO_INCREMENTS");
+  const bool merged = pl.words.valid && P.max_iterations > 0;
+  if (merged) OMNI_TRY_HIP(ctx, ctx->word_part.alloc(word_part_bytes(pl.words.G)));
+  // FP32 ray sums: the merged words' iteration runs in increment form
+  const bool inc = merged && increments(P);
   if (inc) {
     OMNI_TRY_HIP(ctx, ctx->srow.alloc(sizeof(double) * ns));
     OMNI_TRY_HIP(ctx, ctx->dinc0.alloc(sizeof(float) * ns16));
     OMNI_TRY_HIP(ctx, ctx->dinc1.alloc(sizeof(float) * ns16));
   }
-  float* dbuf[2] = {ctx->dinc0.as<float>(), ctx->dinc1.as<float>()};
   if (phase == 1) return OMNI3D_OK;
+  WordIter wi;
+  if (merged) {
+    wi = affine_word_iter(ctx);
+    wi.pinit = pinit;
+    wi.seed = seed > 0 ? 1 : 0;
+  }
   auto iterations = [&](hipStream_t s) -> hipError_t {
+    if (merged) {
+      for (int k = 1; k <= P.max_iterations; k++) {
+        const hipError_t e = launch_iterate_words(k, wi, P.tolerance, s);
+        if (e != hipSuccess) return e;
+      }
+      return launch_words_finish(P.max_iterations, wi, P.max_iterations, P.tolerance, s);
+    }
     StagedIter si;
     si.nS = pl.nS;
     si.D = pl.D;
@@ -856,27 +894,12 @@ int run_affine(omni3d_ctx* ctx, int seed) {
     for (int k = 1; k <= P.max_iterations; k++) {
       if (pl.dense && !pl.staged) {
         const hipError_t e = launch_iterate_dense(
-            pl.dense_group, ctx->dense_variant, k, pl.nS, pl.rowptr.as<unsigned long long>(),
-            pl.dense_wptr.as<unsigned int>(), pl.dent.as<unsigned int>(),
-            pl.diag.as<unsigned int>(), pl.slist.as<int>(), pl.cnt.as<unsigned int>(),
-            ctx->bs.as<long long>(), pinit, seed > 0 ? 1 : 0,
-            rot3 ? pb3[(k - 1) % 3] : pbuf[(k - 1) & 1], rot3 ? pb3[k % 3] : pbuf[k & 1], sc,
-            ctx->partials.as<double>(), P.max_iterations, P.tolerance, s,
-            inc ? ctx->srow.as<double>() : nullptr, inc ? dbuf[(k - 1) & 1] : nullptr,
-            inc ? dbuf[k & 1] : nullptr, pl.dense_group > 1 ? pl.dense_grow.as<int>() : nullptr,
-            pl.dense_ngroups);
+            ctx->dense_variant, k, pl.nS, pl.rowptr.as<unsigned long long>(),
+            pl.dent.as<unsigned int>(), pl.diag.as<unsigned int>(), pl.slist.as<int>(),
+            pl.cnt.as<unsigned int>(), ctx->bs.as<long long>(), pinit, seed > 0 ? 1 : 0,
+            pbuf[(k - 1) & 1], pbuf[k & 1], sc, ctx->partials.as<double>(), P.max_iterations,
+            P.tolerance, s);
         if (e != hipSuccess) return e;
-        if (rot3 && k == P.max_iterations) {
-          // the stop rule of the last iteration (each grouped launch runs
-          // the previous one's), then p_S^{k*-1} for pass B
-          const unsigned int gg = grouped_grid_n(pl.dense_ngroups);
-          hipError_t e2 = launch_iter_finish(
-              k, (int)gg, ctx->partials.as<double>() + (size_t)(k & 1) * 2 * gg, sc,
-              P.max_iterations, P.tolerance, s);
-          if (e2 == hipSuccess)
-            e2 = launch_select_ps(pl.nS, pb3[0], pb3[1], pb3[2], sc, ctx->psel.as<double>(), s);
-          if (e2 != hipSuccess) return e2;
-        }
         continue;
       }
 #ifdef OMNI3D_LAYOUT_STUDY
@@ -902,17 +925,8 @@ int run_affine(omni3d_ctx* ctx, int seed) {
     return hipSuccess;
   };
   if (phase == 2) {
-    // the iterations ran elsewhere: the stop rule of the last one, then
-    // p_S^{k*-1} for pass B
-    if (rot3) {
-      const int k = P.max_iterations;
-      const unsigned int gg = grouped_grid_n(pl.dense_ngroups);
-      OMNI_TRY_HIP(ctx, launch_iter_finish(k, (int)gg,
-                                           ctx->partials.as<double>() + (size_t)(k & 1) * 2 * gg,
-                                           sc, P.max_iterations, P.tolerance, st));
-      OMNI_TRY_HIP(ctx, launch_select_ps(pl.nS, pb3[0], pb3[1], pb3[2], sc,
-                                         ctx->psel.as<double>(), st));
-    }
+    // the iterations ran elsewhere: the stop rule of the last one
+    OMNI_TRY_HIP(ctx, launch_words_finish(P.max_iterations, wi, P.max_iterations, P.tolerance, st));
   } else if (ctx->capturing) {
     OMNI_TRY_HIP(ctx, iterations(st));
   } else {
@@ -933,9 +947,9 @@ int run_affine(omni3d_ctx* ctx, int seed) {
         (uint64_t)(uintptr_t)pl.soff.as<void>(), (uint64_t)(uintptr_t)pl.ulines.as<void>(),
         (uint64_t)(uintptr_t)pl.st_cse.as<void>(), (uint64_t)pl.dense,
         (uint64_t)(uintptr_t)pl.dent.as<void>(), (uint64_t)(uintptr_t)pl.rowptr.as<void>(), (uint64_t)ctx->dense_variant,
-        (uint64_t)pl.dense_group, (uint64_t)inc, (uint64_t)(uintptr_t)ctx->srow.as<void>(),
-        (uint64_t)rot3, (uint64_t)(uintptr_t)pb3[2], (uint64_t)(uintptr_t)ctx->psel.as<void>(),
-        (uint64_t)(uintptr_t)dbuf[0], (uint64_t)(uintptr_t)dbuf[1]};
+        (uint64_t)inc, (uint64_t)(uintptr_t)ctx->srow.as<void>(),
+        (uint64_t)(uintptr_t)ctx->dinc0.as<void>(), (uint64_t)(uintptr_t)ctx->dinc1.as<void>(),
+        merged ? pl.epoch : 0, (uint64_t)(uintptr_t)ctx->word_part.as<void>()};
     if (!ctx->it_exec || key != ctx->it_key) {
       drop_iteration_graph(ctx);
       if (!ctx->cap_stream) OMNI_TRY_HIP(ctx, hipStreamCreate(&ctx->cap_stream));
@@ -965,8 +979,8 @@ int run_affine(omni3d_ctx* ctx, int seed) {
                                           pl.tile_ptr.as<unsigned long long>(),
                                           pl.segs.as<SegRec>(), pl.g, pl.tg, wp, field,
                                           pl.sid.as<int>(), pl.cnt.as<unsigned int>(),
-                                          rot3 ? ctx->psel.as<double>() : pbuf[0],
-                                          rot3 ? ctx->psel.as<double>() : pbuf[1], sc,
+                                          pbuf[0],
+                                          pbuf[1], sc,
                                           ctx->segval.as<T>(),
                                           ctx->sum.as<long long>(), st));
   } else {
@@ -974,8 +988,8 @@ int run_affine(omni3d_ctx* ctx, int seed) {
     record_event(ctx, 5);
     OMNI_TRY_HIP(ctx, launch_walk_plain<T>(true, trilinear(P), pl.rays.as<RayRec>(), pl.nrays,
                                            pl.dirs.as<DirConst>(), pl.g, wp, field, pl.sid.as<int>(),
-                                           rot3 ? ctx->psel.as<double>() : pbuf[0],
-                                           rot3 ? ctx->psel.as<double>() : pbuf[1], sc,
+                                           pbuf[0],
+                                           pbuf[1], sc,
                                            ctx->sum.as<long long>(), V, nc, st));
   }
   record_event(ctx, 6);
@@ -1295,12 +1309,10 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                          pl.val_off.as<unsigned long long>(),
                                          ctx->mk_r.as<uint32_t>(), ctx->mk_f.as<uint32_t>(),
                                          ctx->am_run.as<uint32_t>(), st));
-  // unit weights (plain-mask): the rows as the merged-word layout of the
-  // plain method's source iteration (k_iterate_grp: groups of up to 512
-  // rows sized to about equal entries, as many as fill the CUs evenly;
-  // words sorted by source, equal entries merged), built from CSR rows;
-  // otherwise the rows in tile layout (k_mtile_accum / k_mtile_finish)
-  const bool grouped = fixed && nS < (1 << 22);
+  // unit weights (plain-mask): the rows as the merged words of the plain
+  // method's source iteration, built from CSR rows; otherwise the rows in
+  // tile layout (k_mtile_accum / k_mtile_finish)
+  const bool grouped = fixed && nS < word_max_sources(4);
   unsigned long long nnz = 0;
   unsigned int nwords = 0;
   int nchunks = 0;
@@ -1334,55 +1346,19 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                        ctx->mk_f.as<uint32_t>(), ctx->am_run.as<uint32_t>(), sid,
                                        rcnt.as<unsigned int>(), ctx->am_ptr.as<unsigned long long>(),
                                        ctx->am_src.as<unsigned int>(), st));
-    DevBuf keys, ka, kb, tmp, flag, excl;
+    DevBuf keys;
     OMNI_TRY_HIP(ctx, keys.alloc(sizeof(unsigned long long) * nnz));
-    OMNI_TRY_HIP(ctx, ka.alloc(sizeof(unsigned long long) * nnz));
-    OMNI_TRY_HIP(ctx, kb.alloc(sizeof(unsigned long long) * nnz));
-    OMNI_TRY_HIP(ctx, tmp.alloc(dense_tmp_bytes((int64_t)nnz)));
-    OMNI_TRY_HIP(ctx, flag.alloc(sizeof(unsigned int) * nnz));
-    OMNI_TRY_HIP(ctx, excl.alloc(sizeof(unsigned int) * nnz));
-    // slack after the words: the iteration stages them with 16-byte loads
-    OMNI_TRY_HIP(ctx, ctx->am_dent.alloc(sizeof(unsigned int) * (nnz + 8)));
-    OMNI_TRY_HIP(ctx, launch_fill_u32(ctx->am_dent.as<void>(), (int64_t)nnz + 8, 0u, st));
-    // groups of 8 chunks (4 from 2^21 run starts on), balanced as the plain
-    // method's
-    const int grp = nS < (1 << 21) ? 8 : 4;
-    std::vector<unsigned long long> hrp((size_t)nS + 1);
-    OMNI_TRY_HIP(ctx, hipMemcpy(hrp.data(), ctx->am_ptr.as<void>(),
-                                sizeof(unsigned long long) * ((size_t)nS + 1),
-                                hipMemcpyDeviceToHost));
-    int dev = 0, ncu = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-      (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    std::vector<int> hgrow, hrg((size_t)nS);
-    balance_groups(hrp, 64 * grp, std::max(ncu, 1), &hgrow, &hrg);
-    const int ng = (int)hgrow.size() - 1;
-    DevBuf rgroup;
-    OMNI_TRY_HIP(ctx, ctx->am_grow.alloc(sizeof(int) * hgrow.size()));
-    OMNI_TRY_HIP(ctx, rgroup.alloc(sizeof(int) * (size_t)nS));
-    OMNI_TRY_HIP(ctx, hipMemcpy(ctx->am_grow.as<void>(), hgrow.data(), sizeof(int) * hgrow.size(),
-                                hipMemcpyHostToDevice));
-    OMNI_TRY_HIP(ctx, hipMemcpy(rgroup.as<void>(), hrg.data(), sizeof(int) * (size_t)nS,
-                                hipMemcpyHostToDevice));
-    ctx->am_group = grp;
-    ctx->am_ngroups = ng;
-    OMNI_TRY_HIP(ctx, ctx->am_wptr.alloc(sizeof(unsigned int) * ((size_t)ng + 1)));
     OMNI_TRY_HIP(ctx, launch_widen_keys((int64_t)nnz, ctx->am_src.as<unsigned int>(),
                                         keys.as<unsigned long long>(), st));
-    OMNI_TRY_HIP(ctx, build_dense_entries(nS, (int64_t)nnz, grp,
-                                          ctx->am_ptr.as<unsigned long long>(),
-                                          keys.as<unsigned long long>(),
-                                          ka.as<unsigned long long>(), kb.as<unsigned long long>(),
-                                          tmp.as<void>(), tmp.size(),
-                                          ctx->am_dent.as<unsigned int>(), st, rgroup.as<int>(),
-                                          ctx->am_grow.as<int>(), ng));
-    OMNI_TRY_HIP(ctx, merge_dense_entries(nS, (int64_t)nnz, grp,
-                                          ctx->am_ptr.as<unsigned long long>(),
-                                          kb.as<unsigned long long>(), flag.as<unsigned int>(),
-                                          excl.as<unsigned int>(), tmp.as<void>(), tmp.size(),
-                                          ctx->am_dent.as<unsigned int>(),
-                                          ctx->am_wptr.as<unsigned int>(), &nwords, st,
-                                          ctx->am_grow.as<int>(), ng));
+    // (no diagonal: a run start's own visits are entries)
+    const int rc = build_words(ctx, nS, 0, cu_count(), ctx->am_ptr.as<unsigned long long>(),
+                               keys.as<unsigned long long>(), nullptr, wcnt, slist, &ctx->am_rows);
+    if (rc) return rc;
+    if (!ctx->am_rows.valid) {
+      *fallback = true;
+      return OMNI3D_OK;
+    }
+    nwords = (unsigned int)ctx->am_rows.nwords;
     if (m == OMNI3D_METHOD_PLAIN_MASK) {
       cache.mask_epoch = mepoch;
       cache.plan_epoch = pl.epoch;
@@ -1469,50 +1445,39 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
   double* q0 = nullptr;
   double* q1 = nullptr;
   if (grouped) {
-    // the plain method's iteration on these rows: p_new = (bs * inv + M p) / W
-    // (no diagonal: a run start's own visits are entries), p_S over three
-    // buffers (each launch runs the previous iteration's stop rule), the
-    // increment form for FP32 ray sums
+    // the plain method's iteration on these rows, p_new = (bs * inv + M p) / W,
+    // the increment form for FP32 ray sums
     OMNI_TRY_HIP(ctx, ctx->am_bs.alloc(sizeof(long long) * ns));
-    OMNI_TRY_HIP(ctx, ctx->am_diag.alloc(sizeof(unsigned int) * ns));
     OMNI_TRY_HIP(ctx, launch_masked_bs(nS, slist, sumfx, ctx->am_bs.as<long long>(), st));
-    OMNI_TRY_HIP(ctx, launch_fill_u32(ctx->am_diag.as<void>(), (int64_t)ns, 0u, st));
     record_event(ctx, 3);
     OMNI_TRY_HIP(ctx, ctx->ps0.alloc(sizeof(double) * ns16));
     OMNI_TRY_HIP(ctx, ctx->ps1.alloc(sizeof(double) * ns16));
-    OMNI_TRY_HIP(ctx, ctx->ps2.alloc(sizeof(double) * ns16));
-    OMNI_TRY_HIP(ctx, ctx->psel.alloc(sizeof(double) * ns16));
-    double* pb3[3] = {ctx->ps0.as<double>(), ctx->ps1.as<double>(), ctx->ps2.as<double>()};
-    const bool inc = std::is_same<T, float>::value && !std::getenv("OMNI3D_NO_INCREMENTS");
-    if (inc) {
+    q0 = ctx->ps0.as<double>();
+    q1 = ctx->ps1.as<double>();
+    OMNI_TRY_HIP(ctx, launch_gather_sources(slist, nS, pinit, q0, st));
+    OMNI_TRY_HIP(ctx, launch_absmax<double>(q0, nS, &sc->itmax_bits[0], st));
+    OMNI_TRY_HIP(ctx, ctx->word_part.alloc(word_part_bytes(ctx->am_rows.G)));
+    WordIter it;
+    it.m = ctx->am_rows.mat();
+    it.slist = slist;
+    it.bs = ctx->am_bs.as<long long>();
+    it.pinit = pinit;
+    it.seed = seed > 0 ? 1 : 0;
+    it.pb[0] = q0;
+    it.pb[1] = q1;
+    if (increments(P)) {
       OMNI_TRY_HIP(ctx, ctx->srow.alloc(sizeof(double) * ns));
       OMNI_TRY_HIP(ctx, ctx->dinc0.alloc(sizeof(float) * ns16));
       OMNI_TRY_HIP(ctx, ctx->dinc1.alloc(sizeof(float) * ns16));
+      it.srow = ctx->srow.as<double>();
+      it.db[0] = ctx->dinc0.as<float>();
+      it.db[1] = ctx->dinc1.as<float>();
     }
-    float* dbuf[2] = {ctx->dinc0.as<float>(), ctx->dinc1.as<float>()};
-    const unsigned int gg = grouped_grid_n(ctx->am_ngroups);
-    OMNI_TRY_HIP(ctx, ctx->partials.alloc(sizeof(double) * 4 * gg));
-    OMNI_TRY_HIP(ctx, launch_gather_sources(slist, nS, pinit, pb3[0], st));
-    OMNI_TRY_HIP(ctx, launch_absmax<double>(pb3[0], nS, &sc->itmax_bits[0], st));
-    for (int k = 1; k <= P.max_iterations; k++)
-      OMNI_TRY_HIP(ctx, launch_iterate_dense(ctx->am_group, 0, k, nS,
-                                             ctx->am_ptr.as<unsigned long long>(),
-                                             ctx->am_wptr.as<unsigned int>(),
-                                             ctx->am_dent.as<unsigned int>(),
-                                             ctx->am_diag.as<unsigned int>(), slist, wcnt,
-                                             ctx->am_bs.as<long long>(), pinit, seed > 0 ? 1 : 0,
-                                             pb3[(k - 1) % 3], pb3[k % 3], sc,
-                                             ctx->partials.as<double>(), P.max_iterations,
-                                             P.tolerance, st, inc ? ctx->srow.as<double>() : nullptr,
-                                             inc ? dbuf[(k - 1) & 1] : nullptr,
-                                             inc ? dbuf[k & 1] : nullptr,
-                                             ctx->am_grow.as<int>(), ctx->am_ngroups));
+    it.sc = sc;
+    it.part = ctx->word_part.as<double>();
     const int K = P.max_iterations;
-    OMNI_TRY_HIP(ctx, launch_iter_finish(K, (int)gg,
-                                         ctx->partials.as<double>() + (size_t)(K & 1) * 2 * gg, sc,
-                                         K, P.tolerance, st));
-    OMNI_TRY_HIP(ctx, launch_select_ps(nS, pb3[0], pb3[1], pb3[2], sc, ctx->psel.as<double>(), st));
-    q0 = q1 = ctx->psel.as<double>();
+    for (int k = 1; k <= K; k++) OMNI_TRY_HIP(ctx, launch_iterate_words(k, it, P.tolerance, st));
+    if (K > 0) OMNI_TRY_HIP(ctx, launch_words_finish(K, it, K, P.tolerance, st));
   } else {
     OMNI_TRY_HIP(ctx, ctx->am_b.alloc(sizeof(double) * ns));
     OMNI_TRY_HIP(ctx, ctx->am_wv.alloc(sizeof(double) * ns));
@@ -1821,44 +1786,34 @@ int mask_epoch_now(omni3d_ctx* ctx, uint64_t* epoch) {
 }
 
 // Whether a reconstruction's source iteration can run inside a
-// multi-snapshot launch: the plain method on the affine solver with the
-// grouped dense iteration (tile engine, p_S over three buffers).
+// multi-snapshot launch: the plain method on the affine solver with merged
+// words (tile engine).
 bool affine_fusable(const omni3d_ctx* ctx) {
   const omni3d_params& P = ctx->prm;
   const Plan& pl = *ctx->plan;
   return P.solver == OMNI3D_SOLVER_AFFINE && P.method == OMNI3D_METHOD_PLAIN && pl.valid &&
-         pl.dense && pl.dense_group > 1 && !pl.staged && !ray_engine(ctx) &&
+         pl.words.valid && !ray_engine(ctx) &&
          P.max_iterations > 0 && pl.nS > 0;
 }
 
-// The iteration descriptor of a prepared context (buffers sized by an
+// The iteration's arguments of a prepared context (buffers sized by an
 // earlier reconstruction), seedless (zero initial pressure).
-IterDesc affine_iter_desc(omni3d_ctx* ctx, int first) {
+WordIter affine_word_iter(omni3d_ctx* ctx) {
   const Plan& pl = *ctx->plan;
-  const bool inc = ctx->prm.precision == OMNI3D_FP32_KAHAN && !std::getenv("OMNI3D_NO_INCREMENTS");
-  IterDesc d{};
-  d.nS = pl.nS;
-  d.nb = (int)grouped_grid_n(pl.dense_ngroups);
-  d.grow = pl.dense_grow.as<int>();
-  d.ngr = pl.dense_ngroups;
-  d.first = first;
-  d.seed = 0;
-  d.wptr = pl.dense_wptr.as<unsigned int>();
-  d.dent = pl.dent.as<unsigned int>();
-  d.diag = pl.diag.as<unsigned int>();
-  d.slist = pl.slist.as<int>();
-  d.cnt = pl.cnt.as<unsigned int>();
-  d.bs = ctx->bs.as<long long>();
-  d.pinit = nullptr;
-  d.pb[0] = ctx->ps0.as<double>();
-  d.pb[1] = ctx->ps1.as<double>();
-  d.pb[2] = ctx->ps2.as<double>();
-  d.srow = inc ? ctx->srow.as<double>() : nullptr;
-  d.db[0] = inc ? ctx->dinc0.as<float>() : nullptr;
-  d.db[1] = inc ? ctx->dinc1.as<float>() : nullptr;
-  d.sc = ctx->scal.as<DevScalars>();
-  d.partials = ctx->partials.as<double>();
-  return d;
+  WordIter b;
+  b.m = pl.words.mat();
+  b.slist = pl.slist.as<int>();
+  b.bs = ctx->bs.as<long long>();
+  b.pb[0] = ctx->ps0.as<double>();
+  b.pb[1] = ctx->ps1.as<double>();
+  if (increments(ctx->prm)) {
+    b.srow = ctx->srow.as<double>();
+    b.db[0] = ctx->dinc0.as<float>();
+    b.db[1] = ctx->dinc1.as<float>();
+  }
+  b.sc = ctx->scal.as<DevScalars>();
+  b.part = ctx->word_part.as<double>();
+  return b;
 }
 
 // Queues a whole reconstruction of the context's field on its stream (no

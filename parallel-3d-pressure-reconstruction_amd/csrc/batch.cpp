@@ -160,17 +160,18 @@ int fused_descriptors(omni3d_batch* b, bool* fused) {
   if (std::getenv("OMNI3D_BATCH_SEPARATE")) return OMNI3D_OK;
   for (omni3d_ctx* c : b->snap)
     if (!affine_fusable(c) || c->prm.precision != b->snap[0]->prm.precision ||
-        c->plan->dense_group != b->snap[0]->plan->dense_group)
+        c->plan->words.chunks != b->snap[0]->plan->words.chunks)
       return OMNI3D_OK;
-  std::vector<IterDesc> d;
+  std::vector<WordIter> d;
   std::vector<unsigned int> blk;
   for (int i = 0; i < (int)b->snap.size(); i++) {
-    d.push_back(affine_iter_desc(b->snap[i], (int)blk.size()));
-    blk.insert(blk.end(), (size_t)d.back().nb, (unsigned int)i);
+    d.push_back(affine_word_iter(b->snap[i]));
+    d.back().first = (int)blk.size();
+    blk.insert(blk.end(), (size_t)d.back().m.G, (unsigned int)i);
   }
-  BATCH_TRY_HIP(b, b->desc.alloc(sizeof(IterDesc) * d.size()));
+  BATCH_TRY_HIP(b, b->desc.alloc(sizeof(WordIter) * d.size()));
   BATCH_TRY_HIP(b, b->blk.alloc(sizeof(unsigned int) * blk.size()));
-  BATCH_TRY_HIP(b, hipMemcpy(b->desc.as<void>(), d.data(), sizeof(IterDesc) * d.size(),
+  BATCH_TRY_HIP(b, hipMemcpy(b->desc.as<void>(), d.data(), sizeof(WordIter) * d.size(),
                              hipMemcpyHostToDevice));
   BATCH_TRY_HIP(b, hipMemcpy(b->blk.as<void>(), blk.data(), sizeof(unsigned int) * blk.size(),
                              hipMemcpyHostToDevice));
@@ -218,12 +219,11 @@ int capture(omni3d_batch* b) {
   rc = enqueue_branches(b, fused ? 1 : 0, b->fork);
   if (rc == OMNI3D_OK && fused) {
     const omni3d_params& P = b->snap[0]->prm;
-    const int inc = P.precision == OMNI3D_FP32_KAHAN && !std::getenv("OMNI3D_NO_INCREMENTS");
+    const Plan& pl = *b->snap[0]->plan;
     hipError_t e = hipSuccess;
     for (int k = 1; e == hipSuccess && k <= P.max_iterations; k++)
-      e = launch_iterate_multi(b->snap[0]->plan->dense_group, inc, k, b->desc.as<IterDesc>(),
-                               b->blk.as<unsigned int>(), b->nblk,
-                               P.max_iterations, P.tolerance, b->main);
+      e = launch_iterate_words_multi(pl.words.chunks, increments(P), k, b->desc.as<WordIter>(),
+                                     b->blk.as<unsigned int>(), b->nblk, P.tolerance, b->main);
     if (e != hipSuccess) rc = bfail(b, OMNI3D_ERR_HIP, std::string("iterations: ") + hipGetErrorString(e));
     if (rc == OMNI3D_OK) rc = enqueue_branches(b, 2, b->fork2);
   }
@@ -267,9 +267,7 @@ int omni3d_batch_create(const omni3d_params* base, int count, const int* nx, con
     // the host (a synchronisation per field): a captured graph replays the
     // reference schedule instead
     c->affine_masked = false;
-    // the snapshots' iterations share one launch: no group count rounded up
-    // to fill the CUs per snapshot
-    c->groups_fill_cus = false;
+    c->cu_share = count;  // the snapshots' iterations share one launch
     b->snap.push_back(c);
   }
   for (int i = 0; i < count; i++) b->out.emplace_back(new DevBuf());

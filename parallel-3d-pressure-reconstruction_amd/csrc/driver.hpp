@@ -37,6 +37,18 @@ double path_bound(const omni3d_params& P, const Plan& pl);
 // first row of every group (nS last), rgroup[nS] the group of every row.
 void balance_groups(const std::vector<unsigned long long>& rowptr, int maxrows, int ncu,
                     std::vector<int>* grow, std::vector<int>* rgroup);
+// CSR rows (nS + 1 offsets rowptr on the device, the entries' sources in the
+// low halves of key) as merged words in groups of `chunks` (8 or 4; 4 where
+// the sources need it) times 64 rows at most, sized to about equal entries,
+// their number a multiple of `fill`; row r's diagonal diag[r] (0 if null) and
+// visit count cnt[slist[r]].  out->valid is false where the words do not fit
+// (2^22 sources, rows of 4096 entries or more: their int64 sums hold fewer).
+int build_words(omni3d_ctx* ctx, int nS, int chunks, int fill, const unsigned long long* rowptr,
+                const unsigned long long* key, const unsigned int* diag, const unsigned int* cnt,
+                const int* slist, WordPlan* out);
+int cu_count();
+// whether the FP32 mode iterates on increments (not OMNI3D_NO_INCREMENTS)
+bool increments(const omni3d_params& P);
 // Reference-schedule iteration; the result of iteration k* goes to
 // pdst/wdst (device, dtype), seed: -1 no initial pressure, 0 p only,
 // 1 p and the seed term.
@@ -47,7 +59,7 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype);
 int enqueue_solve(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype);
 // multi-snapshot source iteration (snapshot batches)
 bool affine_fusable(const omni3d_ctx* ctx);
-IterDesc affine_iter_desc(omni3d_ctx* ctx, int first);
+WordIter affine_word_iter(omni3d_ctx* ctx);
 // Releases the context's cached graph of the iteration launches.
 void drop_iteration_graph(omni3d_ctx* ctx);
 // Phase timing event i of the context (skipped during graph capture).

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/omni3d.h"
+#include "words.hpp"
 #include "geometry.hpp"
 #include "kernels.hpp"
 #include "tiles.hpp"
@@ -57,6 +58,25 @@ class DevBuf {
   size_t size_ = 0;
 };
 
+// Rows of the source iteration as merged words (words.hpp).
+struct WordPlan {
+  bool valid = false;
+  int nS = 0, G = 0, chunks = 8;
+  int64_t nwords = 0;  // 4-byte words an iteration reads
+  DevBuf grow, bptr, words, dc;
+  WordMat mat() const {
+    WordMat m;
+    m.nS = nS;
+    m.G = G;
+    m.chunks = chunks;
+    m.grow = grow.as<int>();
+    m.bptr = bptr.as<unsigned int>();
+    m.words = words.as<unsigned int>();
+    m.dc = dc.as<uint4>();
+    return m;
+  }
+};
+
 // Geometry plan: everything that depends only on the grid, the direction set
 // and the line spacing (not on the field), reused across snapshots.
 struct Plan {
@@ -93,15 +113,14 @@ struct Plan {
   DevBuf st_cse;       // uint32[ngroups*D*kStageGroup] end slot of each (stage, chunk)
   DevBuf ulines;       // uint32[nlines] source line (16 sources) of each distinct triple
   DevBuf soff;         // uint16[nnz+16] LDS position of each packed entry
-  // dense iteration layout (valid when dense): per chunk, entries sorted by
-  // source, word (row in chunk << 24 | source), in the CSR range of its rows
+  // the layout of the source iteration: merged words; where sources or rows
+  // exceed their format (or by choice) the dense words below, or the slots
+  WordPlan words;
+  // dense words (valid when dense): per chunk, entries sorted by source, word
+  // (row in chunk << 24 | source), in the CSR range of its rows
   bool dense = false;
-  int dense_group = 1; // chunks per group of the words (1, 4 or 8)
-  int64_t nwords = 0;  // dense words (merged equal entries for groups)
+  int64_t nwords = 0;  // 4-byte words an iteration reads
   DevBuf dent;         // uint32[nnz+8]
-  DevBuf dense_wptr;   // uint32[ngroups+1] first word of each group (groups only)
-  DevBuf dense_grow;   // int32[ngroups+1] first row of each group (groups only)
-  int dense_ngroups = 0;
   // tile engine: compiled paths and per-tile segment lists
   TileGrid tg{};
   int ntiles = 0;
@@ -124,14 +143,7 @@ struct Plan {
   bool trows = false;
   DevBuf tptr;  // uint64[nS+1]
   DevBuf tent;  // uint32[nnz+1]
-  // the same rows as merged words in groups of tgroup chunks sized to equal
-  // entries (the layout of the forward iteration), when sizes allow
-  bool tdense = false;
-  int tgroup = 8;     // chunks per group (8, or 4 for 2^21 sources or more)
-  int tngroups = 0;   // groups
-  DevBuf tdent;   // uint32[nnz+8]
-  DevBuf twptr;   // uint32[ngroups+1]
-  DevBuf tgrow;   // int32[ngroups+1] first row of each group
+  WordPlan twords;  // the same rows as merged words (where they fit)
 };
 
 }  // namespace omni3d
@@ -148,11 +160,12 @@ struct omni3d_ctx {
   int tile_threads = 1024;                   // workgroup size of the tile passes
   int iter_waves = 2;                        // wavefronts per 64-row chunk of the iteration
   int dense_variant = 0;                     // dense iteration: wavefronts x round size
-  int dense_group = 8;                       // dense iteration: chunks per row group (1, 4, 8)
-  // the row groups of the grouped iteration are as many as fill the CUs
-  // evenly (a lone reconstruction); a batch, whose snapshots share one
-  // launch per iteration, keeps the uniform count
-  bool groups_fill_cus = true;
+  // chunks of 64 rows per group of the merged words (4 or 8, 0: by the sizes),
+  // 1: dense words
+  int dense_group = 0;
+  // the iteration's row groups are a multiple of the CUs over this (a batch,
+  // whose snapshots share one launch per iteration: their number)
+  int cu_share = 1;
   bool capturing = false;                    // work is being captured into a graph
   int affine_phase = 0;                      // 1: up to the source iteration, 2: after it
   // graph of the source-iteration launches, reused while its arguments stay
@@ -173,7 +186,6 @@ struct omni3d_ctx {
   omni3d::DevBuf pinit;     // double[V]
   omni3d::DevBuf bs;        // int64[nS]
   omni3d::DevBuf ps0, ps1;  // double[nS]
-  omni3d::DevBuf ps2, psel; // third p_S buffer of the grouped iteration, p_S^{k*-1}
   // increment form of the iteration (FP32 ray sums): row sums of p_S and the
   // FP32 increments of two consecutive iterations
   omni3d::DevBuf srow, dinc0, dinc1;
@@ -210,15 +222,11 @@ struct omni3d_ctx {
     uint64_t mask_epoch = 0, plan_epoch = 0;
     int nS = 0;
     omni3d::DevBuf cnt, sid, slist, tptr, tent, diag;
-    // the rows as merged words (the forward iteration's layout), when sizes
-    // allow: chunks per group, groups, words, first word and row per group
-    bool tdense = false;
-    int tgroup = 8, tngroups = 0;
-    omni3d::DevBuf tdent, twptr, tgrow;
+    omni3d::WordPlan twords;  // the rows as merged words (where they fit)
   } adj_mask;
-  // the transposed iteration on merged words: its scalars, partial sums and
-  // fixed-point source term
-  omni3d::DevBuf adj_sc, adj_part, adj_bs;
+  // the transposed iteration on merged words: its scalars and fixed-point
+  // source term
+  omni3d::DevBuf adj_sc, adj_bs;
   // masked methods on the tile engine: per value slot the first-visit record
   // (E, S, R, F, curl weights) of the field and the carries of an iteration
   omni3d::DevBuf mk_e, mk_s, mk_r, mk_f, mk_wc, mk_wn, mk_c;
@@ -228,12 +236,10 @@ struct omni3d_ctx {
   // the rows (pointers, source ids, weights); per row b, W and p_S (two);
   // max weight; the final pass's scalars
   omni3d::DevBuf am_run, am_sid, am_slist, am_ptr, am_src, am_w, am_b, am_wv, am_p0, am_p1;
-  omni3d::DevBuf am_wmax, am_sc, am_dent, am_wptr, am_bs, am_diag;
+  omni3d::DevBuf am_wmax, am_sc, am_bs;
   omni3d::DevBuf am_tfirst, am_tbase, am_erow, am_chunks, am_rowsum;
-  // plain-mask rows as merged words: chunks per group, groups, first row of
-  // each group (int32[ngroups+1])
-  int am_group = 8, am_ngroups = 0;
-  omni3d::DevBuf am_grow;
+  omni3d::WordPlan am_rows;     // plain-mask rows as merged words
+  omni3d::DevBuf word_part;     // the word iteration's partial sums (word_part_bytes)
   bool affine_masked = true;  // off for snapshot batches (their graphs replay the reference schedule)
   // plain-mask on the affine schedule: the mask-only structures (rule
   // records F and R, run-start ids, run sources, the rows as merged words)

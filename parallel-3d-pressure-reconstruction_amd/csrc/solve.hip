@@ -565,261 +565,14 @@ __device__ void finish_iteration(int k, int nparts, const double* __restrict__ p
   }
 }
 
-// The dense iteration over groups of kG chunks: a workgroup of kG
-// wavefronts owns a group (rows [grow[g], grow[g + 1]), at most kG * 64 =
-// 256 or 512, the group's words sorted by source, word (row in group << (32
-// - b)) | (multiplicity - 1) << (30 - b) | source with b = 8 or 9 row bits,
-// the group's words from wptr[g]), its wavefronts take the
-// group's rounds of 512 words in turn and add into the group's LDS row sums;
-// each wavefront then finishes the 64 rows of its chunk.  Sources shared by
-// neighbouring chunks touch the same 128-byte lines in one gather.
-//
-// kInc selects the increment form (FP32 ray-sum precision): a row keeps
-// S = sum of its entries' p_S in FP64 across iterations.  kInc == 1 (the
-// first iteration) gathers p_S, stores S and the FP32 increment dnew = p_new
-// - p_old; kInc == 2 gathers the previous increments din (4 bytes per entry)
-// and adds their sum to S.  The fixed-point scale then follows max |increment|
-// instead of max |p_S|, so the FP32 rounding applies to increments only.
-// The body of one workgroup: block lb of the nb workgroups of this
-// iteration (one snapshot's, in a multi-snapshot launch).
-template <int kG, int kInc>
-__device__ __forceinline__ void iterate_grp_body(
-    const unsigned int lb, const unsigned int nb, int k, int nS,
-    const unsigned int* __restrict__ wptr, const unsigned int* __restrict__ dent,
-    const int* __restrict__ grow, int ngr, const unsigned int* __restrict__ diag, const int* __restrict__ slist,
-    const unsigned int* __restrict__ cnt, const long long* __restrict__ bs,
-    const double* __restrict__ pinit, int seed, const double* __restrict__ pold,
-    double* __restrict__ pnew, double* __restrict__ srow, const float* __restrict__ din,
-    float* __restrict__ dnew, DevScalars* __restrict__ sc, double* __restrict__ partials,
-    int max_iter, double tol) {
-  // the first group's word range and rows ([grow[g], grow[g + 1]), at most
-  // kRows, chosen so that groups hold about equal words) are loaded with the
-  // stop flag: independent loads in flight together
-  unsigned int fw0 = 0, fw1 = 0;
-  int fr0 = 0, fr1 = 0;
-  if ((int)lb < ngr) {
-    fw0 = wptr[lb];
-    fw1 = wptr[lb + 1];
-    fr0 = grow[lb];
-    fr1 = grow[lb + 1];
-  }
-  // the stop rule of iteration k - 1 runs in workgroup 0 of this launch: the
-  // launch computes iteration k before knowing it (the buffers keep p_S of
-  // k - 1), and launch k + 1 returns at once if k - 1 stopped
-  if (sc->converged) return;
-  constexpr int kU = 8;
-  constexpr int kRows = 64 * kG;
-  static_assert(kRows == 256 || kRows == 512, "merged words hold 8- or 9-bit rows");
-  constexpr int kRowShift = kRows == 256 ? 24 : 23;
-  constexpr int kMulShift = kRowShift - 2;
-  constexpr unsigned int kSrcMask = (1u << kMulShift) - 1u;
-  __shared__ unsigned long long s_acc[kRows];
-  __shared__ __attribute__((aligned(16))) unsigned int s_ent[kG][kU * 64];
-  __shared__ double s_red[2][kG];
-  __shared__ unsigned long long s_max[kG];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  unsigned int* __restrict__ se = s_ent[wave];
-  const int4* __restrict__ d4 = reinterpret_cast<const int4*>(dent);
-  // the first group's first words, issued before the loads of the scale
-  // (and before workgroup 0's stop rule) so that their latencies overlap
-  int4 pre[kU / 4];
-  {
-    const unsigned long long q1 = ((unsigned long long)fw1 + 3) >> 2;
-    const unsigned long long base = (fw0 & ~3ull) + (unsigned long long)wave * (kU * 64);
-#pragma unroll
-    for (int j = 0; j < kU / 4; j++) {
-      const unsigned long long q = (base >> 2) + (unsigned long long)(j * 64 + lane);
-      pre[j] = q < q1 ? d4[q] : int4{0, 0, 0, 0};
-    }
-  }
-  const double* __restrict__ prev_part = partials + (size_t)((k - 1) & 1) * 2 * nb;
-  partials += (size_t)(k & 1) * 2 * nb;
-  if (lb == 0) {
-    if (k > 1) finish_iteration<64 * kG>(k - 1, nb, prev_part, sc, max_iter, tol);
-    // the max slot launch k + 1 fills (launch k - 1 read it)
-    if (threadIdx.x == 0) sc->itmax_bits[(k + 1) % 3] = 0ull;
-  }
-  const double inv = sc->inv_scale;
-  const double B = __longlong_as_double((long long)sc->itmax_bits[(k - 1) % 3]);
-  const bool finite = B <= DBL_MAX;
-  int ex = 0;
-  (void)frexp(finite ? B : 1.0, &ex);
-  ex = ex < -960 ? -960 : ex;  // (a tiny bound: keep the scale finite)
-  const double scale = ldexp(1.0, 51 - ex), iscale = ldexp(1.0, ex - 51);
-  double d2 = 0.0, n2 = 0.0;
-  unsigned long long pm = 0ull;
-  for (int g = (int)lb; g < ngr; g += (int)nb) {
-    const bool first = g == (int)lb;
-    const int rbeg = first ? fr0 : grow[g];
-    const int nrows = (first ? fr1 : grow[g + 1]) - rbeg;
-    const unsigned long long e0 = first ? fw0 : wptr[g], e1 = first ? fw1 : wptr[g + 1];
-    const unsigned long long q1 = (e1 + 3) >> 2;
-    unsigned long long base = (e0 & ~3ull) + (unsigned long long)wave * (kU * 64);
-    if (!first) {
-#pragma unroll
-      for (int j = 0; j < kU / 4; j++) {
-        const unsigned long long q = (base >> 2) + (unsigned long long)(j * 64 + lane);
-        pre[j] = q < q1 ? d4[q] : int4{0, 0, 0, 0};
-      }
-    }
-    // the row sums are cleared while the first words are in flight (the
-    // previous group's rows were read before the barrier that ended it)
-    s_acc[threadIdx.x] = 0ull;
-    __syncthreads();
-    for (; base < e1; base += (unsigned long long)kG * (kU * 64)) {
-#pragma unroll
-      for (int j = 0; j < kU / 4; j++) reinterpret_cast<int4*>(se)[j * 64 + lane] = pre[j];
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const unsigned long long nb = base + (unsigned long long)kG * (kU * 64);
-      if (nb < e1) {
-#pragma unroll
-        for (int j = 0; j < kU / 4; j++) {
-          const unsigned long long q = (nb >> 2) + (unsigned long long)(j * 64 + lane);
-          if (q < q1) pre[j] = d4[q];
-        }
-      }
-      // this round's words i with lo <= i < hi belong to the group (lo <= 3:
-      // the group's first round may start up to 3 words early; both bounds
-      // fit 32 bits)
-      const unsigned int lo = (unsigned int)(e0 > base ? e0 - base : 0ull);
-      const unsigned long long hl = e1 - base;
-      const unsigned int hi = hl < (unsigned long long)(kU * 64) ? (unsigned int)hl : kU * 64;
-      unsigned int w[kU];
-      double x[kU];
-      bool ok[kU];
-#pragma unroll
-      for (int u = 0; u < kU; u++) {
-        const unsigned int i = u * 64 + lane;
-        ok[u] = i >= lo && i < hi;
-        w[u] = ok[u] ? se[i] : se[lo];
-      }
-#pragma unroll
-      for (int u = 0; u < kU; u++) {
-        if constexpr (kInc == 2) x[u] = (double)din[w[u] & kSrcMask];
-        else x[u] = pold[w[u] & kSrcMask];
-      }
-#pragma unroll
-      for (int u = 0; u < kU; u++) {
-        // a word stands for 1..4 equal entries (the same source in one row):
-        // the fixed-point value times its multiplicity (an integer product,
-        // exact; scaling x first would leave the bias rounding's 2^51 range);
-        // lanes outside the group's words add 0 (no branch around the add)
-        const unsigned int m = ok[u] ? ((w[u] >> kMulShift) & 3u) + 1u : 0u;
-        atomicAdd(&s_acc[w[u] >> kRowShift], (unsigned long long)to_fixed(x[u], scale) * m);
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-    // the row's own values do not depend on the row sums: loaded before the
-    // barrier, they arrive while the group's last wavefronts finish
-    const int row = rbeg + wave * 64 + lane;
-    const bool own = wave * 64 + lane < nrows;
-    int v = 0;
-    unsigned int c = 0, dg = 0;
-    double po = 0.0, sr = 0.0;
-    long long bv = 0;
-    if (own) {
-      v = slist[row];
-      c = cnt[v];
-      po = pold[row];
-      bv = bs[row];
-      dg = diag[row];
-      if constexpr (kInc == 2) sr = srow[row];
-    }
-    __syncthreads();
-    if (own) {
-      double acc = (double)(long long)s_acc[wave * 64 + lane] * iscale;
-      if (!finite) acc = B - B;
-      if constexpr (kInc == 2) acc += sr;
-      if constexpr (kInc != 0) srow[row] = acc;
-      double tot = (double)bv * inv + (double)dg * po + acc;
-      if (k == 1 && seed && pinit) tot += pinit[v];
-      const double pn = c > 0 ? tot / (double)c : po;
-      pnew[row] = pn;
-      const double df = pn - po;
-      d2 += df * df;
-      n2 += pn * pn;
-      double mv = pn;
-      if constexpr (kInc != 0) {
-        const float dq = (float)df;
-        dnew[row] = dq;
-        mv = (double)dq;
-      }
-      const unsigned long long b = (unsigned long long)__double_as_longlong(fabs(mv));
-      pm = b > pm ? b : pm;
-    }
-    __syncthreads();
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    d2 += __shfl_xor(d2, off);
-    n2 += __shfl_xor(n2, off);
-    const unsigned long long o = __shfl_xor(pm, off);
-    pm = o > pm ? o : pm;
-  }
-  if (lane == 0) {
-    s_red[0][wave] = d2;
-    s_red[1][wave] = n2;
-    s_max[wave] = pm;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double a = 0.0, c = 0.0;
-    unsigned long long m = 0ull;
-    for (int q = 0; q < kG; q++) {
-      a += s_red[0][q];
-      c += s_red[1][q];
-      m = s_max[q] > m ? s_max[q] : m;
-    }
-    partials[2 * lb] = a;
-    partials[2 * lb + 1] = c;
-    atomicMax(&sc->itmax_bits[k % 3], m);
-  }
-}
-
-template <int kG, int kInc>
-__global__ void __launch_bounds__(64 * kG)
-k_iterate_grp(int k, int nS, const unsigned int* __restrict__ wptr,
-              const unsigned int* __restrict__ dent, const int* __restrict__ grow, int ngr,
-              const unsigned int* __restrict__ diag,
-              const int* __restrict__ slist, const unsigned int* __restrict__ cnt,
-              const long long* __restrict__ bs, const double* __restrict__ pinit, int seed,
-              const double* __restrict__ pold, double* __restrict__ pnew,
-              double* __restrict__ srow, const float* __restrict__ din, float* __restrict__ dnew,
-              DevScalars* __restrict__ sc, double* __restrict__ partials, int max_iter,
-              double tol) {
-  iterate_grp_body<kG, kInc>(blockIdx.x, gridDim.x, k, nS, wptr, dent, grow, ngr, diag, slist,
-                             cnt, bs, pinit, seed, pold, pnew, srow, din, dnew, sc, partials,
-                             max_iter, tol);
-}
-
-// Iteration k of many snapshots in one launch (a snapshot batch): workgroup
-// b works for snapshot blk_snap[b] as its block b - first of nb, on that
-// snapshot's buffers (p_S rotating over three, increments over two, as in
-// the one-snapshot launches), so every snapshot's result is the one its own
-// launches give; a snapshot that stopped returns at once.
-template <int kG, int kInc>
-__global__ void __launch_bounds__(64 * kG)
-k_iterate_multi(int k, const IterDesc* __restrict__ desc, const unsigned int* __restrict__ blk_snap,
-                int max_iter, double tol) {
-  const IterDesc& q = desc[blk_snap[blockIdx.x]];
-  const unsigned int lb = blockIdx.x - (unsigned int)q.first;
-  iterate_grp_body<kG, kInc>(lb, (unsigned int)q.nb, k, q.nS, q.wptr, q.dent, q.grow, q.ngr,
-                             q.diag, q.slist,
-                             q.cnt, q.bs, q.pinit, q.seed, q.pb[(k - 1) % 3], q.pb[k % 3],
-                             q.srow, kInc == 2 ? q.db[(k - 1) & 1] : nullptr,
-                             kInc != 0 ? q.db[k & 1] : nullptr, q.sc, q.partials, max_iter, tol);
-}
-
 // Relative change of iteration k from the workgroups' partial sums (fixed
 // order: a strided share per thread, then a tree), and the stop rule.
 __global__ void __launch_bounds__(kFinishBlock)
 k_iter_finish(int k, int nparts, const double* __restrict__ partials, DevScalars* __restrict__ sc,
-              int max_iter, double tol, int slots) {
+              int max_iter, double tol) {
   if (sc->converged) return;
   // the max |p_S| slot iteration k + 1 fills (iteration k read it)
-  if (threadIdx.x == 0 && slots == 2) sc->itmax_bits[(k + 1) & 1] = 0ull;
+  if (threadIdx.x == 0) sc->itmax_bits[(k + 1) & 1] = 0ull;
   finish_iteration<kFinishBlock>(k, nparts, partials, sc, max_iter, tol);
 }
 
@@ -1060,38 +813,14 @@ hipError_t launch_iterate(int waves, int k, int nS, const unsigned long long* mo
 #endif
 #undef OMNI_ITER
   hipLaunchKernelGGL(k_iter_finish, dim3(1), dim3(kFinishBlock), 0, st, k, (int)grid, partials, sc,
-                     max_iter, tol, 2);
-  return hipGetLastError();
-}
-
-// p_S of iteration k* - 1 out of the three rotating buffers of the grouped
-// iteration (iteration k writes buffer k % 3).
-__global__ void k_select_ps(int nS, const double* __restrict__ b0, const double* __restrict__ b1,
-                            const double* __restrict__ b2, const DevScalars* __restrict__ sc,
-                            double* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nS) return;
-  const int q = (sc->kstar - 1) % 3;
-  out[i] = q == 0 ? b0[i] : (q == 1 ? b1[i] : b2[i]);
-}
-
-hipError_t launch_select_ps(int nS, const double* b0, const double* b1, const double* b2,
-                            const DevScalars* sc, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_select_ps, dim3(grid_for(nS)), dim3(256), 0, st, nS, b0, b1, b2, sc, out);
+                     max_iter, tol);
   return hipGetLastError();
 }
 
 hipError_t launch_iter_finish2(int k, int nparts, const double* partials, DevScalars* sc,
                                int max_iter, double tol, hipStream_t st) {
   hipLaunchKernelGGL(k_iter_finish, dim3(1), dim3(kFinishBlock), 0, st, k, nparts, partials, sc,
-                     max_iter, tol, 2);
-  return hipGetLastError();
-}
-
-hipError_t launch_iter_finish(int k, int nparts, const double* partials, DevScalars* sc,
-                              int max_iter, double tol, hipStream_t st) {
-  hipLaunchKernelGGL(k_iter_finish, dim3(1), dim3(kFinishBlock), 0, st, k, nparts, partials, sc,
-                     max_iter, tol, 3);
+                     max_iter, tol);
   return hipGetLastError();
 }
 
@@ -1101,37 +830,13 @@ unsigned int dense_grid(int nS) {
   return (unsigned int)std::max(1, std::min(nch, 65536));
 }
 
-hipError_t launch_iterate_dense(int gchunks, int variant, int k, int nS,
-                                const unsigned long long* rowptr, const unsigned int* wptr,
+hipError_t launch_iterate_dense(int variant, int k, int nS, const unsigned long long* rowptr,
                                 const unsigned int* dent, const unsigned int* diag,
                                 const int* slist, const unsigned int* cnt, const long long* bs,
                                 const double* pinit, int seed, const double* pold, double* pnew,
                                 DevScalars* sc, double* partials, int max_iter, double tol,
-                                hipStream_t st, double* srow, const float* din, float* dnew,
-                                const int* grow, int ngroups) {
-  unsigned int grid = dense_grid(nS);
-  if (gchunks > 1) {
-    // groups carry their first rows (grow[ngroups + 1])
-    if (!grow || ngroups < 1) return hipErrorInvalidValue;
-    const int ngr = ngroups;
-    grid = grouped_grid_n(ngr);
-    const int inc = srow ? (k == 1 ? 1 : 2) : 0;
-#define OMNI_GRP(G, I)                                                                         \
-  hipLaunchKernelGGL((k_iterate_grp<G, I>), dim3(grid), dim3(64 * G), 0, st, k, nS, wptr, dent,  \
-                     grow, ngr, diag, slist, cnt, bs, pinit, seed, pold, pnew, srow, din, dnew,   \
-                     sc, partials, max_iter, tol)
-    if (gchunks == 8) {
-      if (inc == 1) OMNI_GRP(8, 1);
-      else if (inc == 2) OMNI_GRP(8, 2);
-      else OMNI_GRP(8, 0);
-    } else {
-      if (inc == 1) OMNI_GRP(4, 1);
-      else if (inc == 2) OMNI_GRP(4, 2);
-      else OMNI_GRP(4, 0);
-    }
-#undef OMNI_GRP
-    return hipGetLastError();
-  }
+                                hipStream_t st) {
+  unsigned int grid = 0;
 #define OMNI_DENSE(W, U)                                                                       \
   hipLaunchKernelGGL((k_iterate_dense<W, U>), dim3(grid), dim3(64 * W), 0, st, k, nS, rowptr,    \
                      dent, diag, slist, cnt, bs, pinit, seed, pold, pnew, sc, partials)
@@ -1153,27 +858,7 @@ hipError_t launch_iterate_dense(int gchunks, int variant, int k, int nS,
 #endif
 #undef OMNI_DENSE
   hipLaunchKernelGGL(k_iter_finish, dim3(1), dim3(kFinishBlock), 0, st, k, (int)grid, partials, sc,
-                     max_iter, tol, 2);
-  return hipGetLastError();
-}
-
-hipError_t launch_iterate_multi(int gchunks, int inc, int k, const IterDesc* desc,
-                                const unsigned int* blk_snap, unsigned int nblocks, int max_iter,
-                                double tol, hipStream_t st) {
-  const int v = inc ? (k == 1 ? 1 : 2) : 0;
-#define OMNI_MULTI(G, I)                                                                      \
-  hipLaunchKernelGGL((k_iterate_multi<G, I>), dim3(nblocks), dim3(64 * G), 0, st, k, desc,       \
-                     blk_snap, max_iter, tol)
-  if (gchunks == 8) {
-    if (v == 1) OMNI_MULTI(8, 1);
-    else if (v == 2) OMNI_MULTI(8, 2);
-    else OMNI_MULTI(8, 0);
-  } else {
-    if (v == 1) OMNI_MULTI(4, 1);
-    else if (v == 2) OMNI_MULTI(4, 2);
-    else OMNI_MULTI(4, 0);
-  }
-#undef OMNI_MULTI
+                     max_iter, tol);
   return hipGetLastError();
 }
 
@@ -1193,7 +878,7 @@ hipError_t launch_iterate_staged(const StagedIter& si, int k, const unsigned int
   hipLaunchKernelGGL((k_iterate_staged<kStageGroup, kStageCap>), dim3(grid), dim3(64 * kStageGroup),
                      0, st, si, k, diag, slist, cnt, bs, pinit, seed, pold, pnew, sc, partials);
   hipLaunchKernelGGL(k_iter_finish, dim3(1), dim3(kFinishBlock), 0, st, k, (int)grid, partials, sc,
-                     max_iter, tol, 2);
+                     max_iter, tol);
   return hipGetLastError();
 }
 #endif  // OMNI3D_LAYOUT_STUDY

@@ -145,16 +145,15 @@ __global__ void k_stage_offsets(int64_t n, int lb, int db, int D,
 
 unsigned int grid1(int64_t n) { return (unsigned int)((n + 255) / 256); }
 
-// One lane per row: key (group, source, row in group) of each CSR entry
-// (CSR keys are (direction << 32) | source); a group is 2^gshift rows.
-__global__ void k_dense_keys(int nS, int gshift, int rb, const unsigned long long* __restrict__ rowptr,
+// One lane per row: key (group, source, row in group) of each CSR entry.
+__global__ void k_dense_keys(int nS, int rb, const unsigned long long* __restrict__ rowptr,
                              const unsigned long long* __restrict__ ckey,
                              const int* __restrict__ rgroup, const int* __restrict__ grow,
                              unsigned long long* __restrict__ keys) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= nS) return;
-  const int g = rgroup ? rgroup[r] : r >> gshift;
-  const int rin = rgroup ? r - grow[g] : r & ((1 << gshift) - 1);
+  const int g = rgroup ? rgroup[r] : r >> 6;
+  const int rin = rgroup ? r - grow[g] : r & 63;
   const unsigned long long hi = ((unsigned long long)g << 32) | (unsigned long long)rin;
   const unsigned long long smask = (1ull << (32 - rb)) - 1ull;
   for (unsigned long long j = rowptr[r]; j < rowptr[r + 1]; j++)
@@ -171,44 +170,6 @@ __global__ void k_dense_words(int64_t n, int rb, const unsigned long long* __res
   dent[i] = (row << (32 - rb)) | src;
 }
 
-// Merge of equal (group, source, row) keys into one word with a
-// multiplicity of 1..4: flag the first key of every run of up to 4.
-__global__ void k_merge_flags(int64_t n, const unsigned long long* __restrict__ k,
-                              unsigned int* __restrict__ flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int64_t c = 0;
-  while (i - c - 1 >= 0 && k[i - c - 1] == k[i]) c++;
-  flag[i] = (c & 3) == 0 ? 1u : 0u;
-}
-
-// word (row << (32 - rb)) | (multiplicity - 1) << (30 - rb) | source at the
-// run's slot
-__global__ void k_merge_write(int64_t n, int rb, const unsigned long long* __restrict__ k,
-                              const unsigned int* __restrict__ flag,
-                              const unsigned int* __restrict__ excl, unsigned int* __restrict__ dent) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || !flag[i]) return;
-  unsigned int m = 1;
-  while (m < 4 && i + m < n && k[i + m] == k[i]) m++;
-  const unsigned long long key = k[i];
-  const unsigned int row = (unsigned int)(key & ((1ull << rb) - 1ull));
-  const unsigned int src = (unsigned int)((key >> rb) & ((1ull << (30 - rb)) - 1ull));
-  dent[excl[i]] = (row << (32 - rb)) | ((m - 1u) << (30 - rb)) | src;
-}
-
-// first word of every group: the merged index of the group's first entry
-__global__ void k_merge_gptr(int ng, int rows, int nS, int64_t n,
-                             const unsigned long long* __restrict__ rowptr,
-                             const unsigned int* __restrict__ excl, unsigned int nwords,
-                             const int* __restrict__ grow, unsigned int* __restrict__ wptr) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g > ng) return;
-  const long long r = grow ? (long long)grow[g] : (long long)g * rows;
-  const unsigned long long pos = rowptr[r < nS ? r : nS];
-  wptr[g] = pos < (unsigned long long)n ? excl[pos] : nwords;
-}
-
 }  // namespace
 
 size_t dense_tmp_bytes(int64_t nnz) {
@@ -220,56 +181,41 @@ size_t dense_tmp_bytes(int64_t nnz) {
   return std::max(a, b) + 256;
 }
 
-hipError_t merge_dense_entries(int nS, int64_t nnz, int gchunks, const unsigned long long* rowptr,
-                               const unsigned long long* keys, unsigned int* flag,
-                               unsigned int* excl, void* tmp, size_t tmp_bytes, unsigned int* dent,
-                               unsigned int* wptr, unsigned int* nwords, hipStream_t st,
-                               const int* grow, int ngroups) {
-  const int rb = dense_row_bits(gchunks);
-  hipLaunchKernelGGL(k_merge_flags, dim3(grid1(nnz)), dim3(256), 0, st, nnz, keys, flag);
-  hipError_t e = hipGetLastError();
+hipError_t sort_entry_keys(int nS, int64_t nnz, int rb, const unsigned long long* rowptr,
+                           const unsigned long long* csr_key, const int* rgroup, const int* grow,
+                           int ngroups, unsigned long long* keys_a, unsigned long long* keys_b,
+                           void* tmp, size_t tmp_bytes, hipStream_t st) {
+  hipLaunchKernelGGL(k_dense_keys, dim3(grid1(nS)), dim3(256), 0, st, nS, rb, rowptr, csr_key,
+                     rgroup, grow, keys_a);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  const int ng = rgroup ? ngroups : (nS + 63) >> 6;
   size_t bytes = tmp_bytes;
-  e = hipcub::DeviceScan::ExclusiveSum(tmp, bytes, flag, excl, (int)nnz, st);
-  if (e != hipSuccess) return e;
-  unsigned int last[2] = {0, 0};
-  e = hipMemcpyAsync(&last[0], excl + (nnz - 1), 4, hipMemcpyDeviceToHost, st);
-  if (e != hipSuccess) return e;
-  e = hipMemcpyAsync(&last[1], flag + (nnz - 1), 4, hipMemcpyDeviceToHost, st);
-  if (e != hipSuccess) return e;
-  e = hipStreamSynchronize(st);
-  if (e != hipSuccess) return e;
-  *nwords = last[0] + last[1];
-  hipLaunchKernelGGL(k_merge_write, dim3(grid1(nnz)), dim3(256), 0, st, nnz, rb, keys, flag, excl,
+  return hipcub::DeviceRadixSort::SortKeys(tmp, bytes, keys_a, keys_b, (int)nnz, 0,
+                                           32 + bits_for((unsigned long long)ng), st);
+}
+
+hipError_t launch_dense_words(int64_t nnz, const unsigned long long* keys, unsigned int* dent,
+                              hipStream_t st) {
+  hipLaunchKernelGGL(k_dense_words, dim3(grid1(nnz)), dim3(256), 0, st, nnz, kDenseRowBits, keys,
                      dent);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int rows = 64 * gchunks;
-  const int ng = grow ? ngroups : (nS + rows - 1) / rows;
-  hipLaunchKernelGGL(k_merge_gptr, dim3(grid1(ng + 1)), dim3(256), 0, st, ng, rows, nS, nnz, rowptr,
-                     excl, *nwords, grow, wptr);
   return hipGetLastError();
 }
 
-hipError_t build_dense_entries(int nS, int64_t nnz, int gchunks, const unsigned long long* rowptr,
-                               const unsigned long long* csr_key, unsigned long long* keys_a,
-                               unsigned long long* keys_b, void* tmp, size_t tmp_bytes,
-                               unsigned int* dent, hipStream_t st, const int* rgroup,
-                               const int* grow, int ngroups) {
-  const int gshift = 6 + bits_for((unsigned long long)gchunks);
-  const int rb = dense_row_bits(gchunks);
-  hipLaunchKernelGGL(k_dense_keys, dim3(grid1(nS)), dim3(256), 0, st, nS, gshift, rb, rowptr,
-                     csr_key, rgroup, grow, keys_a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int ng = rgroup ? ngroups : (nS + (1 << gshift) - 1) >> gshift;
-  const int end_bit = 32 + bits_for((unsigned long long)ng);
+hipError_t exclusive_sums(int64_t n, const unsigned int* flag, unsigned int* excl, void* tmp,
+                          size_t tmp_bytes, unsigned int* total, hipStream_t st) {
   size_t bytes = tmp_bytes;
-  e = hipcub::DeviceRadixSort::SortKeys(tmp, bytes, keys_a, keys_b, (int)nnz, 0, end_bit, st);
+  hipError_t e = hipcub::DeviceScan::ExclusiveSum(tmp, bytes, flag, excl, (int)n, st);
   if (e != hipSuccess) return e;
-  if (gchunks > 1) return hipSuccess;  // merged words: merge_dense_entries
-  hipLaunchKernelGGL(k_dense_words, dim3(grid1(nnz)), dim3(256), 0, st, nnz, rb, keys_b, dent);
-  return hipGetLastError();
+  unsigned int last[2] = {0, 0};
+  e = hipMemcpyAsync(&last[0], excl + (n - 1), 4, hipMemcpyDeviceToHost, st);
+  if (e != hipSuccess) return e;
+  e = hipMemcpyAsync(&last[1], flag + (n - 1), 4, hipMemcpyDeviceToHost, st);
+  if (e != hipSuccess) return e;
+  e = hipStreamSynchronize(st);
+  if (e != hipSuccess) return e;
+  *total = last[0] + last[1];
+  return hipSuccess;
 }
 
 #ifdef OMNI3D_LAYOUT_STUDY

@@ -67,84 +67,29 @@ unsigned int staged_grid(int nS);
 // (row in chunk << 24 | source) each; the chunk's words occupy the CSR range
 // of its rows.
 unsigned int dense_grid(int nS);
-// Stop rule of iteration k alone (after the last grouped dense launch, whose
-// own stop rule the next launch would have run); partials of iteration k.
-hipError_t launch_iter_finish(int k, int nparts, const double* partials, DevScalars* sc,
-                              int max_iter, double tol, hipStream_t st);
-// The grouped iteration rotates p_S over three buffers (its launches run
-// one iteration ahead of the stop rule): out = p_S of iteration k* - 1.
-hipError_t launch_select_ps(int nS, const double* b0, const double* b1, const double* b2,
-                            const DevScalars* sc, double* out, hipStream_t st);
-// grid of the grouped dense iteration (one group per workgroup)
-inline unsigned int grouped_grid_n(int ngroups) {
-  return (unsigned int)(ngroups < 1 ? 1 : (ngroups > 65536 ? 65536 : ngroups));
-}
-// Row bits of a dense word for groups of gchunks chunks: (row << (32 - bits)) | source.
-constexpr int dense_row_bits(int gchunks) { return gchunks <= 4 ? 8 : (gchunks <= 8 ? 9 : 10); }
-// gchunks: chunks per group sharing the LDS row sums (1, 4, 8 or 16); the
-// group's words are sorted by source.  For gchunks > 1 this leaves the sorted
-// keys in keys_b for merge_dense_entries.
-// With rgroup / grow (groups > 1 only): row r belongs to group rgroup[r],
-// whose rows are [grow[g], grow[g + 1]) (at most 64 * gchunks), ngroups in
-// all; without them, groups of 64 * gchunks consecutive rows.
-hipError_t build_dense_entries(int nS, int64_t nnz, int gchunks, const unsigned long long* rowptr,
-                               const unsigned long long* csr_key, unsigned long long* keys_a,
-                               unsigned long long* keys_b, void* tmp, size_t tmp_bytes,
-                               unsigned int* dent, hipStream_t st, const int* rgroup = nullptr,
-                               const int* grow = nullptr, int ngroups = 0);
+// Keys (group << 32 | source << rb | row in group) of the CSR entries (source
+// in the low half of csr_key), sorted into keys_b: row r in group rgroup[r]
+// from row grow[group] on, ngroups in all; without rgroup, groups of 64 rows.
+hipError_t sort_entry_keys(int nS, int64_t nnz, int rb, const unsigned long long* rowptr,
+                           const unsigned long long* csr_key, const int* rgroup, const int* grow,
+                           int ngroups, unsigned long long* keys_a, unsigned long long* keys_b,
+                           void* tmp, size_t tmp_bytes, hipStream_t st);
+// The dense words of keys sorted in groups of 64 rows.
+constexpr int kDenseRowBits = 8;
+hipError_t launch_dense_words(int64_t nnz, const unsigned long long* keys, unsigned int* dent,
+                              hipStream_t st);
+// excl = exclusive sums of flag, *total their sum (synchronises the stream)
+hipError_t exclusive_sums(int64_t n, const unsigned int* flag, unsigned int* excl, void* tmp,
+                          size_t tmp_bytes, unsigned int* total, hipStream_t st);
 size_t dense_tmp_bytes(int64_t nnz);
-// Groups (gchunks > 1): equal (group, source, row) keys of the sorted keys
-// merged into words (row << (32 - b)) | (multiplicity - 1) << (30 - b) |
-// source, b = dense_row_bits(gchunks) (sources below 2^(30 - b)),
-// wptr[ngroups+1] the first word of every group.
-hipError_t merge_dense_entries(int nS, int64_t nnz, int gchunks, const unsigned long long* rowptr,
-                               const unsigned long long* keys, unsigned int* flag,
-                               unsigned int* excl, void* tmp, size_t tmp_bytes, unsigned int* dent,
-                               unsigned int* wptr, unsigned int* nwords, hipStream_t st,
-                               const int* grow = nullptr, int ngroups = 0);
-// gchunks 1: one chunk per wavefront, variant = chunks per workgroup x
-// entries per round (0: 4 x 512, 1: 8 x 512, 2: 8 x 256, 3: 4 x 256,
-// 4: 4 x 1024); gchunks 4 or 8: one group per workgroup of 4 or 8
-// wavefronts sharing the group's LDS row sums, merged words from wptr; partials then hold two
-// halves (iterations alternate) and each launch runs the stop rule of the
-// previous iteration, max |.| slots k % 3 -- launch_iter_finish ends the loop.  With srow (groups only) the
-// increment form: srow[nS] FP64 row sums of p_S kept across iterations,
-// din / dnew the FP32 increments of the previous / this iteration.
-hipError_t launch_iterate_dense(int gchunks, int variant, int k, int nS,
-                                const unsigned long long* rowptr, const unsigned int* wptr,
+// one chunk per wavefront, variant = chunks per workgroup x entries per round
+// (0: 4 x 512, 1: 8 x 512, 2: 8 x 256, 3: 4 x 256, 4: 4 x 1024)
+hipError_t launch_iterate_dense(int variant, int k, int nS, const unsigned long long* rowptr,
                                 const unsigned int* dent, const unsigned int* diag,
                                 const int* slist, const unsigned int* cnt, const long long* bs,
                                 const double* pinit, int seed, const double* pold, double* pnew,
                                 DevScalars* sc, double* partials, int max_iter, double tol,
-                                hipStream_t st, double* srow = nullptr,
-                                const float* din = nullptr, float* dnew = nullptr,
-                                const int* grow = nullptr, int ngroups = 0);
-// One snapshot's share of a multi-snapshot launch of the grouped iteration:
-// its nb = grouped_grid_n(ngr) workgroups start at block `first`; p_S rotates
-// over pb[0..2] and the increments over db[0..1] as in its own launches.
-struct IterDesc {
-  int nS, nb, first, seed;
-  const unsigned int* wptr;
-  const unsigned int* dent;
-  const int* grow;  // first row of each group (ngr + 1 entries)
-  int ngr;          // groups
-  const unsigned int* diag;
-  const int* slist;
-  const unsigned int* cnt;
-  const long long* bs;
-  const double* pinit;
-  double* pb[3];
-  double* srow;
-  float* db[2];
-  DevScalars* sc;
-  double* partials;
-};
-// iteration k of every snapshot described (gchunks: chunks per group, 4 or 8,
-// the same for all; inc: increment form, FP32 ray sums); blk_snap[b] = the
-// snapshot of workgroup b
-hipError_t launch_iterate_multi(int gchunks, int inc, int k, const IterDesc* desc,
-                                const unsigned int* blk_snap, unsigned int nblocks, int max_iter,
-                                double tol, hipStream_t st);
+                                hipStream_t st);
 #ifdef OMNI3D_LAYOUT_STUDY
 hipError_t launch_iterate_staged(const StagedIter& si, int k, const unsigned int* diag,
                                  const int* slist, const unsigned int* cnt, const long long* bs,
