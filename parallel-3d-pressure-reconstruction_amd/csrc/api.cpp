@@ -1082,6 +1082,7 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype) {
       m == OMNI3D_METHOD_PLAIN ? pl.cnt.as<unsigned int>() : ctx->wcnt.as<unsigned int>();
   record_event(ctx, 2);
   void* rule = nullptr;
+  if (tiled) OMNI_TRY_HIP(ctx, ctx->mk_bits.alloc(step_bits_bytes(m, pl.nsegs)));
   if (tiled && !mask_walk_lane()) {
     OMNI_TRY_HIP(ctx, ctx->mk_rule.alloc(mask_rule_bytes(m, pl.nval)));
     rule = ctx->mk_rule.as<void>();
@@ -1098,7 +1099,7 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype) {
                                           m == OMNI3D_METHOD_PLAIN_MASK
                                               ? ctx->wcnt.as<unsigned int>() : nullptr,
                                           fixed ? nullptr : ctx->wsum.as<double>(),
-                                          ctx->srcf.as<uint8_t>(), rule, st));
+                                          ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(), st));
   record_event(ctx, 8);
   record_event(ctx, 3);
   for (int k = 1; k <= P.max_iterations; k++) {
@@ -1114,7 +1115,7 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype) {
                                               ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), pa,
                                               pb, k, sc,
                                               fixed ? ctx->sum.as<long long>() : nullptr,
-                                              fixed ? nullptr : ctx->sumd.as<double>(), st));
+                                              fixed ? nullptr : ctx->sumd.as<double>(), ctx->mk_bits.as<void>(), st));
       OMNI_TRY_HIP(ctx, launch_naive_update(k, V, fixed ? 1 : 0,
                                             fixed ? ctx->sum.as<long long>() : nullptr, cntw,
                                             fixed ? nullptr : ctx->sumd.as<double>(),
@@ -1214,6 +1215,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
   OMNI_TRY_HIP(ctx, ctx->mk_f.alloc(sizeof(uint32_t) * nv));
   OMNI_TRY_HIP(ctx, ctx->mk_wc.alloc(sizeof(double) * (fixed ? 1 : nv)));
   OMNI_TRY_HIP(ctx, ctx->mk_wn.alloc(sizeof(double) * (fixed ? 1 : nv)));
+  OMNI_TRY_HIP(ctx, ctx->mk_bits.alloc(step_bits_bytes(m, pl.nsegs)));
   OMNI_TRY_HIP(ctx, ctx->am_run.alloc(sizeof(uint32_t) * nv));
   OMNI_TRY_HIP(ctx, ctx->pa.alloc(sizeof(double) * V));
   OMNI_TRY_HIP(ctx, ctx->pb.alloc(sizeof(double) * V));
@@ -1259,7 +1261,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                            pl.segs.as<SegRec>(), pl.g, pl.tg, wp, field, aux, sc,
                                            ctx->mk_e.as<double>(), ctx->mk_s.as<double>(),
                                            ctx->mk_f.as<uint32_t>(), wcnt,
-                                           ctx->srcf.as<uint8_t>(), st));
+                                           ctx->srcf.as<uint8_t>(), ctx->mk_bits.as<void>(), st));
   } else {
     // the rule replay: first-visit records, weights, run starts
     void* rule = nullptr;
@@ -1276,7 +1278,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                           ctx->mk_s.as<double>(), ctx->mk_r.as<uint32_t>(),
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
                                           ctx->mk_wn.as<double>(), wcnt, wsum,
-                                          ctx->srcf.as<uint8_t>(), rule, st));
+                                          ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(), st));
   }
   record_event(ctx, 8);
   // S: compact ids of the run starts (the voxels a pass reads p at), in tile
@@ -1328,7 +1330,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
     OMNI_TRY_HIP(ctx, launch_tile_rows(false, m, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                                        pl.segs.as<SegRec>(), pl.g, pl.tg, wp, aux,
                                        ctx->mk_f.as<uint32_t>(), ctx->am_run.as<uint32_t>(), sid,
-                                       rcnt.as<unsigned int>(), nullptr, nullptr, st));
+                                       rcnt.as<unsigned int>(), nullptr, nullptr, ctx->mk_bits.as<void>(), st));
     OMNI_TRY_HIP(ctx, stmp.alloc(scan_u32_tmp_bytes(nS)));
     OMNI_TRY_HIP(ctx, launch_scan_u32(rcnt.as<unsigned int>(), nS,
                                       ctx->am_ptr.as<unsigned long long>(), 0, stmp.as<void>(),
@@ -1345,7 +1347,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                        pl.segs.as<SegRec>(), pl.g, pl.tg, wp, aux,
                                        ctx->mk_f.as<uint32_t>(), ctx->am_run.as<uint32_t>(), sid,
                                        rcnt.as<unsigned int>(), ctx->am_ptr.as<unsigned long long>(),
-                                       ctx->am_src.as<unsigned int>(), st));
+                                       ctx->am_src.as<unsigned int>(), ctx->mk_bits.as<void>(), st));
     DevBuf keys;
     OMNI_TRY_HIP(ctx, keys.alloc(sizeof(unsigned long long) * nnz));
     OMNI_TRY_HIP(ctx, launch_widen_keys((int64_t)nnz, ctx->am_src.as<unsigned int>(),
@@ -1377,7 +1379,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
                                           ctx->mk_wn.as<double>(), ctx->am_run.as<uint32_t>(),
                                           sid, tfirst, tcnt.as<unsigned int>(), nullptr, nullptr,
-                                          nullptr, nullptr, st));
+                                          nullptr, nullptr, ctx->mk_bits.as<void>(), st));
     OMNI_TRY_HIP(ctx, stmp.alloc(scan_u32_tmp_bytes(np)));
     OMNI_TRY_HIP(ctx, launch_scan_u32(tcnt.as<unsigned int>(), np,
                                       ctx->am_tbase.as<unsigned long long>(), 0, stmp.as<void>(),
@@ -1403,7 +1405,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                           ctx->am_tbase.as<unsigned long long>(),
                                           ctx->am_src.as<unsigned int>(),
                                           ctx->am_erow.as<unsigned short>(),
-                                          fixed ? nullptr : ctx->am_w.as<double>(), st));
+                                          fixed ? nullptr : ctx->am_w.as<double>(), ctx->mk_bits.as<void>(), st));
     // chunks of at most csz entries of one tile, a workgroup each
     const unsigned long long csz = std::max<unsigned long long>(
         2048ull, std::min<unsigned long long>(65536ull, nnz / 4096ull));
@@ -1438,8 +1440,8 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
   OMNI_TRY_HIP(ctx, launch_tile_masked<T>(m, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                                           pl.segs.as<SegRec>(), pl.g, pl.tg, wp, field, aux,
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
-                                          ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), pz, pz,
-                                          1, sc, sumfx, sumd, st));
+                                          ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), nullptr, nullptr,
+                                          1, sc, sumfx, sumd, ctx->mk_bits.as<void>(), st));
   const size_t ns = (size_t)nS;
   const size_t ns16 = (ns + 15) & ~(size_t)15;
   double* q0 = nullptr;
@@ -1526,7 +1528,7 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                           pl.segs.as<SegRec>(), pl.g, pl.tg, wp, field, aux,
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
                                           ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), pa, pa,
-                                          1, scf, sumfx, sumd, st));
+                                          1, scf, sumfx, sumd, ctx->mk_bits.as<void>(), st));
   record_event(ctx, 6);
   const bool f64 = dtype == OMNI3D_F64;
   OMNI_TRY_HIP(ctx, launch_masked_final(V, fixed ? 1 : 0, sumfx, wcnt, sumd, wsum, pinit,

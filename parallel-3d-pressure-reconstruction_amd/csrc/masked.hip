@@ -182,6 +182,15 @@ __device__ __forceinline__ uint32_t rule_state(bool p0set, bool outthr) {
 
 // Select and plain-mask enter a segment in one of three states; the plain
 // and Weighted walks are always in a run after the entry voxel.
+// Where the rule is one (plain-mask, Select): per segment, in the tiles' order
+// of the segments, what its steps do -- 16 steps a word, the visits that add
+// in the low half, those that restart the run in the high half.
+template <int kMethod>
+constexpr bool kRuled = kMethod == kMaskUnit || kMethod == kMaskSelect;
+struct StepBits {
+  uint32_t w[3];
+};
+
 template <int kMethod>
 constexpr int kRulePlanes = (kMethod == kMaskUnit || kMethod == kMaskSelect) ? kRuleStates : 1;
 
@@ -205,8 +214,9 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kVox = kTile * kTile * kTile;
-  constexpr bool kAux = kMethod != kMaskPlain;
-  __shared__ double s_aux[kAux ? kVox : 1];
+  constexpr bool kRule = kRuled<kMethod>, kCurl = kCurlW<kMethod>;
+  __shared__ uint8_t s_cls[kRule ? kVox : 1];
+  __shared__ double s_cw[kCurl ? kVox : 1];  // curl / 10000
   const TilePart tp = tile_part(xcd_block(), parts);
   const int tile = tp.tile;
   const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
@@ -214,11 +224,13 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
-  if constexpr (kAux) {
+  if constexpr (kRule || kCurl) {
     for (int l = threadIdx.x; l < kVox; l += blockDim.x) {
       const int i = ox + (l & kTileMask), j = oy + ((l >> kBits) & kTileMask), kk = oz + (l >> (2 * kBits));
       const bool in = i < g.X && j < g.Y && kk < g.Z;
-      s_aux[lds_slot<kBits>(l)] = in ? aux[i + j * sy + kk * sz] : 0.0;
+      const double cv = in ? aux[i + j * sy + kk * sz] : 0.0;
+      if constexpr (kRule) s_cls[lds_slot<kBits>(l)] = (uint8_t)rule_class(wp, cv);
+      if constexpr (kCurl) s_cw[lds_slot<kBits>(l)] = cv / 10000;
     }
     __syncthreads();
   }
@@ -226,9 +238,9 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
     return (int64_t)(ox + (l & kTileMask)) + (int64_t)(oy + ((l >> kBits) & kTileMask)) * sy +
            (int64_t)(oz + (l >> (2 * kBits))) * sz;
   };
-  auto cval = [&](int l) -> double {
-    if constexpr (kAux) return s_aux[lds_slot<kBits>(l)];
-    else return 0.0;
+  auto cls = [&](int l) -> unsigned int {
+    if constexpr (kRule) return s_cls[lds_slot<kBits>(l)];
+    else return 0u;
   };
   const unsigned int bd = blockDim.x * (unsigned int)parts;
   for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
@@ -241,7 +253,7 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
     const int d0 = (sg & 1u) ? 1 : -1;
     const int d1 = (sg & 2u) ? kTile : -kTile;
     const int d2 = (sg & 4u) ? kTile * kTile : -kTile * kTile;
-    const double c_first = cval(lv0);
+    const unsigned int c_first = cls(lv0);
     // the step into the tile: its term (whether it joins the run depends on
     // the entry state; the scan decides)
     double E = 0.0;
@@ -252,7 +264,7 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
       E = (double)trapezoid<T>(wp, ae, se, component(field[vf], ae), component(field[vp], ae));
     }
     rs.E[sr.g] = E;
-    if constexpr (kCurlW<kMethod>) rs.x[sr.g] = c_first / 10000;
+    if constexpr (kCurl) rs.x[sr.g] = s_cw[lds_slot<kBits>(lv0)];
     const int nplanes = first_seg ? 1 : kRulePlanes<kMethod>;
     for (int st = 0; st < nplanes; st++) {
       // entry state: N, L, H; the single state of the plain / Weighted walks is L
@@ -265,7 +277,7 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
         // the ray's entry voxel (kernel.cu:2302 Select; every entry for the
         // plain and Weighted walks)
         p0set = outthr = false;
-        if (rule_entry<kMethod>(wp, c_first)) {
+        if (rule_entry<kMethod>(wp, kRule ? aux[gvox(lv0)] : 0.0)) {
           p0set = true;
           hasR = true;
           R = (uint32_t)gvox(lv0);
@@ -274,7 +286,7 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
           F = kModeNone;
         }
       } else {
-        const StepRule d = rule_step<kMethod>(wp, ae, c_first, p0set, outthr);
+        const StepRule d = rule_step_class<kMethod>(wp, ae, c_first, p0set, outthr);
         if (d.restart) {
           hasR = true;
           R = (uint32_t)gvox(lv0);
@@ -297,12 +309,12 @@ k_rule_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
           const int a = (int)(cw & 3u);
           cw >>= 2;
           const int ln = lv + (a == 0 ? d0 : (a == 1 ? d1 : d2));
-          const double cn = cval(ln);
-          const StepRule d = rule_step<kMethod>(wp, a, cn, p0set, outthr);
-          if (d.add && kCurlW<kMethod>) {
-            csum += cn / 10000;
-            ccnt += 1u;
-          }
+          const StepRule d = rule_step_class<kMethod>(wp, a, cls(ln), p0set, outthr);
+          if constexpr (kCurl)
+            if (d.add) {
+              csum += s_cw[lds_slot<kBits>(ln)];
+              ccnt += 1u;
+            }
           if (d.restart) {
             hasR = true;
             R = (uint32_t)gvox(ln);
@@ -437,21 +449,20 @@ k_mask_carry(int64_t nrays, const unsigned int* __restrict__ nseg,
   }
 }
 
-template <typename T, int kMethod, int kVox>
-struct MaskLds {
-  using Acc = typename std::conditional<kCurlW<kMethod>, double, long long>::type;
-  T g[3][kVox];
-  Acc acc[kVox];
-  // curl / mask values and the previous iteration's p (read where a run
-  // restarts) in LDS where they fit (FP32 gradient)
-  double aux[sizeof(T) == 4 && kMethod != kMaskPlain ? kVox : 1];
-  double pl[sizeof(T) == 4 ? kVox : 1];
-};
-
-// kSetup (once per field): instead of the visits' values, the visits'
-// weights (visit counts or curl weights, into wcnt / wsum) and each
-// segment's sum of added terms after its last restart (into segS).
-template <typename T, int kMethod, int kBits, int kThreads, bool kSetup>
+// kSetup (once per field): the rule replayed on the voxels' classes -- the
+// visits' weights (visit counts or curl weights, into wcnt / wsum), the run
+// starts, each segment's step bits and its sum of added terms after its last
+// restart (into segS).  Otherwise the visits' values, from the step bits.
+// kP: runs start from p (p0 / p1 by the iteration's parity), else from 0.
+//
+// What bounds it: per visit two LDS reads of the gradient, one LDS atomic and
+// the term's arithmetic; around it the loads a segment starts with, which
+// depend on one another (record, then flags and carry), so the next segment's
+// are in flight while one is walked, as in k_tile_pass.  The rule itself
+// (compares of FP64 curl values, a dozen state operations per step) runs once
+// per field; curl / 10000, the division every curl weight needs, once per
+// voxel.
+template <typename T, int kMethod, int kBits, int kThreads, bool kSetup, bool kP>
 __global__ void __launch_bounds__(kThreads)
 k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
               GridDesc g, TileGrid tg, WalkParams wp,
@@ -462,14 +473,27 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
               const DevScalars* __restrict__ sc, long long* __restrict__ sumfx,
               double* __restrict__ sumd, double* __restrict__ segS,
               unsigned int* __restrict__ wcnt, double* __restrict__ wsum,
-              uint8_t* __restrict__ src, int parts) {
+              uint8_t* __restrict__ src, StepBits* __restrict__ bits, int parts) {
   using V4 = typename Vec4<T>::type;
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kVox = kTile * kTile * kTile;
-  constexpr bool kAuxLds = sizeof(T) == 4;
-  constexpr bool kAux = kMethod != kMaskPlain;  // the plain rule reads no curl / mask
-  __shared__ MaskLds<T, kMethod, kVox> L;
+  constexpr bool kCurl = kCurlW<kMethod>;
+  constexpr bool kRule = kRuled<kMethod>;
+  // LDS: the gradient, the sums; the rule's classes (setup), curl / 10000
+  // where it fits (an FP64 setup pass reads the curl from memory), p where
+  // runs restart inside a tile and it fits
+  constexpr bool kCls = kSetup && kRule;
+  constexpr bool kCw = kCurl && !(kSetup && sizeof(T) == 8);
+  constexpr bool kPl = kP && kRule && sizeof(T) == 4;
+  constexpr bool kCount = kSetup && !kCurl;
+  using Acc = typename std::conditional<
+      kCurl, double, typename std::conditional<kCount, unsigned int, long long>::type>::type;
+  __shared__ T s_g[3][kVox];
+  __shared__ Acc s_acc[kVox];
+  __shared__ uint8_t s_cls[kCls ? kVox : 1];
+  __shared__ double s_cw[kCw ? kVox : 1];
+  __shared__ double s_p[kPl ? kVox : 1];
   if (sc->converged) return;
   const double* __restrict__ p = ((k - 1) & 1) ? p1 : p0;
   const TilePart tp = tile_part(xcd_block(), parts);
@@ -488,22 +512,19 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
     if (in) {
       const int64_t gv = i + j * sy + kk * sz;
       v = field[gv];
-      if (kAuxLds) {
-        if (kAux) cv = aux[gv];
-        if (!kSetup) pv = p[gv];
-      }
+      if (kCls || kCw) cv = aux[gv];
+      if (kPl) pv = p[gv];
     } else {
       v.x = v.y = v.z = v.w = 0;
     }
     const int sl = lds_slot<kBits>(l);
-    L.g[0][sl] = v.x;
-    L.g[1][sl] = v.y;
-    L.g[2][sl] = v.z;
-    L.acc[sl] = 0;
-    if (kAuxLds) {
-      if (kAux) L.aux[sl] = cv;
-      L.pl[sl] = pv;
-    }
+    s_g[0][sl] = v.x;
+    s_g[1][sl] = v.y;
+    s_g[2][sl] = v.z;
+    s_acc[sl] = 0;
+    if constexpr (kCls) s_cls[sl] = (uint8_t)rule_class(wp, cv);
+    if constexpr (kCw) s_cw[sl] = cv / 10000;
+    if constexpr (kPl) s_p[sl] = pv;
   }
   __syncthreads();
   const double scale = sc->scale;
@@ -513,23 +534,55 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
            (int64_t)(oz + (l >> (2 * kBits))) * sz;
   };
   auto add = [&](int sl, double c, double curl, double cnt) {
-    if constexpr (kSetup) {
+    if constexpr (kCount) {
       // the plain method's weights are the plan's visit counts
-      if constexpr (kMethod == kMaskUnit)
-        atomicAdd(reinterpret_cast<unsigned long long*>(&L.acc[sl]), 1ull);
-      else if constexpr (kCurlW<kMethod>)
-        atomicAdd(&L.acc[sl], curl_weight(curl, cnt));
-    } else if constexpr (!kCurlW<kMethod>) {
-      atomicAdd(reinterpret_cast<unsigned long long*>(&L.acc[sl]),
+      if constexpr (kMethod == kMaskUnit) atomicAdd(&s_acc[sl], 1u);
+    } else if constexpr (kSetup) {
+      atomicAdd(&s_acc[sl], curl_weight(curl, cnt));
+    } else if constexpr (!kCurl) {
+      atomicAdd(reinterpret_cast<unsigned long long*>(&s_acc[sl]),
                 (unsigned long long)to_fixed(c, scale));
     } else {
-      atomicAdd(&L.acc[sl], curl_value(c, curl, cnt));
+      atomicAdd(&s_acc[sl], curl_value(c, curl, cnt));
     }
   };
+  auto start = [&](int l, int sl) -> double {
+    if constexpr (!kP) return 0.0;
+    else if constexpr (kPl) return s_p[sl];
+    else return p[gvox(l)];
+  };
+  // the record two segments ahead and what the next one starts with are in
+  // flight while this one is walked
+  struct Pre {
+    uint32_t f = 0;
+    double cv = 0.0, curl = 0.0, cnt = 0.0;
+    StepBits sb{{0, 0, 0}};
+  };
+  auto fetch = [&](const SegRec& r, unsigned long long at) {
+    Pre q;
+    q.f = F[r.g];
+    if constexpr (!kSetup) q.cv = cval[r.g];
+    if constexpr (!kSetup && kRule) q.sb = bits[at];
+    if constexpr (kCurl) {
+      q.curl = wc[r.g];
+      q.cnt = wn[r.g];
+    }
+    return q;
+  };
   const unsigned int bd = blockDim.x * (unsigned int)parts;
-  for (unsigned long long jj = part_begin(b, tp); jj < e; jj += bd) {
-    const SegRec sr = segs[jj];
-    const uint32_t f = F[sr.g];
+  unsigned long long jj = part_begin(b, tp);
+  SegRec r1, r2;
+  Pre q1;
+  if (jj < e) r1 = segs[jj];
+  if (jj + bd < e) r2 = segs[jj + bd];
+  if (jj < e) q1 = fetch(r1, jj);
+  for (; jj < e; jj += bd) {
+    const SegRec sr = r1;
+    const Pre pr = q1;
+    r1 = r2;
+    if (jj + 2ull * bd < e) r2 = segs[jj + 2ull * bd];
+    if (jj + bd < e) q1 = fetch(r1, jj + bd);
+    const uint32_t f = pr.f;
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
     const unsigned int n = (sr.info >> kSegLvBits) & 63u;
     const unsigned int sg = (sr.info >> 18) & 7u;
@@ -542,44 +595,52 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
     const T h2 = step_factor<T>(wp, 2, up2);
     bool p0set = (f & kFlagP0) != 0, outthr = (f & kFlagOut) != 0;
     const uint32_t mode = f & 3u;
-    double c = 0.0, S = 0.0;
-    if constexpr (!kSetup) {
-      if (mode == kModeCont) c = cval[sr.g];
-      else if (mode == kModeRestart) c = kAuxLds ? L.pl[lds_slot<kBits>(lv)] : p[gvox(lv)];
-    }
-    // the run starts (source flags): every voxel a run (re)starts at
-    if constexpr (kSetup)
-      if (mode == kModeRestart) src[gvox(lv)] = 1;
-    double curl = 0.0, cnt = 0.0;
-    if (kCurlW<kMethod>) {
-      curl = wc[sr.g];
-      cnt = wn[sr.g];
-    }
     int slv = lds_slot<kBits>(lv);
+    double c = 0.0;  // (setup: the sum since the last restart)
+    if constexpr (!kSetup) {
+      if (mode == kModeCont) c = pr.cv;
+      else if (mode == kModeRestart) c = start(lv, slv);
+    } else {
+      // the run starts (source flags): every voxel a run (re)starts at
+      if (mode == kModeRestart) src[gvox(lv)] = 1;
+    }
+    double curl = pr.curl, cnt = pr.cnt;
     if (f & kFlagAdd) add(slv, c, curl, cnt);
     uint32_t cw = sr.code[0];
     int rem = (int)n - 1;
+    StepBits sb = pr.sb;
 #pragma unroll 1
     for (int wi = 0; wi < 3 && rem > 0; wi++) {
       const int m = rem < 16 ? rem : 16;
+      uint32_t w = sb.w[0];
+      if constexpr (kSetup) w = 0u;
       for (int q = 0; q < m; q++) {
         const int a = (int)(cw & 3u);
         cw >>= 2;
         const int ln = lv + (a == 0 ? d0 : (a == 1 ? d1 : d2));
         const int sln = lds_slot<kBits>(ln);
-        double cn = 0.0;
-        if constexpr (!kAux) cn = 0.0;
-        else if constexpr (kAuxLds) cn = L.aux[sln];
-        else cn = aux[gvox(ln)];
-        const StepRule d = rule_step<kMethod>(wp, a, cn, p0set, outthr);
+        StepRule d{true, false, false};
+        if constexpr (kRule && kSetup) {
+          d = rule_step_class<kMethod>(wp, a, s_cls[sln], p0set, outthr);
+          w |= (d.add ? 1u << q : 0u) | (d.restart ? 0x10000u << q : 0u);
+        } else if constexpr (kRule) {
+          d.add = w & 1u;
+          d.restart = w & 0x10000u;
+          w >>= 1;
+          // (a run's first start never keeps the weights)
+          if constexpr (kCurl) {
+            d.keep_w = p0set && wp.faithful && a == 2;
+            p0set = p0set || d.restart;
+          }
+        }
+        const T h = a == 0 ? h0 : (a == 1 ? h1 : h2);
+        const T t = h * (s_g[a][sln] + s_g[a][slv]);
         if (d.add) {
-          const T h = a == 0 ? h0 : (a == 1 ? h1 : h2);
-          const T t = h * (L.g[a][sln] + L.g[a][slv]);
-          if constexpr (kSetup) S += (double)t;
-          else c += (double)t;
+          c += (double)t;
           bool added = true;
-          if (kCurlW<kMethod>) {
-            curl += cn / 10000;
+          if constexpr (kCurl) {
+            if constexpr (kCw) curl += s_cw[sln];
+            else curl += aux[gvox(ln)] / 10000;
             cnt += 1.0;
             added = kMethod != kMaskWeighted || curl != 0.0;
           }
@@ -587,10 +648,11 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
         }
         if (d.restart) {
           if constexpr (kSetup) {
-            S = 0.0;
+            c = 0.0;
             src[gvox(ln)] = 1;
-          } else if constexpr (kAuxLds) c = L.pl[sln];
-          else c = p[gvox(ln)];
+          } else {
+            c = start(ln, sln);
+          }
           if (!d.keep_w) {
             curl = 0.0;
             cnt = 0.0;
@@ -599,27 +661,35 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
         lv = ln;
         slv = sln;
       }
+      if constexpr (kSetup) {
+        if (wi == 0) sb.w[0] = w;
+        else if (wi == 1) sb.w[1] = w;
+        else sb.w[2] = w;
+      } else {
+        sb.w[0] = sb.w[1];
+        sb.w[1] = sb.w[2];
+      }
       rem -= m;
       cw = wi == 0 ? sr.code[1] : sr.code[2];
     }
-    if constexpr (kSetup) segS[sr.g] = S;
+    if constexpr (kSetup) segS[sr.g] = c;
+    if constexpr (kSetup && kRule) bits[jj] = sb;
   }
   __syncthreads();
   for (int l = threadIdx.x; l < kVox; l += blockDim.x) {
     const int i = ox + (l & kTileMask), j = oy + ((l >> kBits) & kTileMask), kk = oz + (l >> (2 * kBits));
     if (i >= g.X || j >= g.Y || kk >= g.Z) continue;
     const int64_t gv = i + j * sy + kk * sz;
-    const int sl = lds_slot<kBits>(l);
-    const auto x = L.acc[sl];
-    if constexpr (kSetup) {
+    const Acc x = s_acc[lds_slot<kBits>(l)];
+    if constexpr (kCount) {
       if constexpr (kMethod == kMaskUnit) {
-        if (parts == 1) wcnt[gv] = (unsigned int)x;
-        else if (x) atomicAdd(&wcnt[gv], (unsigned int)x);
-      } else if constexpr (kCurlW<kMethod>) {
-        if (parts == 1) wsum[gv] = x;
-        else if (x != 0.0) unsafeAtomicAdd(&wsum[gv], x);
+        if (parts == 1) wcnt[gv] = x;
+        else if (x) atomicAdd(&wcnt[gv], x);
       }
-    } else if constexpr (!kCurlW<kMethod>) {
+    } else if constexpr (kSetup) {
+      if (parts == 1) wsum[gv] = x;
+      else if (x != 0.0) unsafeAtomicAdd(&wsum[gv], x);
+    } else if constexpr (!kCurl) {
       if (parts == 1) sumfx[gv] = x;
       else if (x) fx_add(&sumfx[gv], x);
     } else {
@@ -629,7 +699,12 @@ k_tile_masked(const unsigned long long* __restrict__ tile_ptr, const SegRec* __r
   }
 }
 
-template <typename T, bool kSetup>
+size_t step_bits_bytes(int method, int64_t nsegs) {
+  return method == kMaskUnit || method == kMaskSelect
+             ? sizeof(StepBits) * (size_t)std::max<int64_t>(nsegs, 1) : 0;
+}
+
+template <typename T, bool kSetup, bool kP>
 hipError_t launch_tile_pass_masked(int method, int ntiles, const unsigned long long* tile_ptr,
                                    const SegRec* segs, GridDesc g, TileGrid tg,
                                    const WalkParams& wp, const void* field, const double* aux,
@@ -637,7 +712,7 @@ hipError_t launch_tile_pass_masked(int method, int ntiles, const unsigned long l
                                    const double* cval, const double* p0, const double* p1, int k,
                                    const DevScalars* sc, long long* sumfx, double* sumd,
                                    double* segS, unsigned int* wcnt, double* wsum,
-                                   uint8_t* src, hipStream_t st) {
+                                   uint8_t* src, void* bits, hipStream_t st) {
   using V4 = typename Vec4<T>::type;
   const V4* f = static_cast<const V4*>(field);
   constexpr int kThreads = 1024;
@@ -655,9 +730,9 @@ hipError_t launch_tile_pass_masked(int method, int ntiles, const unsigned long l
     if (e != hipSuccess) return e;
   }
 #define OMNI_TM(M, B)                                                                           \
-  hipLaunchKernelGGL((k_tile_masked<T, M, B, kThreads, kSetup>), dim3(ntiles * parts),            \
+  hipLaunchKernelGGL((k_tile_masked<T, M, B, kThreads, kSetup, kP>), dim3(ntiles * parts),        \
                      dim3(kThreads), 0, st, tile_ptr, segs, g, tg, wp, f, aux, F, wc, wn, cval, p0, \
-                     p1, k, sc, sumfx, sumd, segS, wcnt, wsum, src, parts)
+                     p1, k, sc, sumfx, sumd, segS, wcnt, wsum, src, static_cast<StepBits*>(bits), parts)
   if (tg.bits == 3) {
     switch (method) {
       case kMaskPlain: OMNI_TM(kMaskPlain, 3); break;
@@ -754,7 +829,7 @@ hipError_t launch_mask_walk(int method, const RayRec* rays, int64_t nrays, const
                             const unsigned long long* tile_ptr, const SegRec* segs,
                             const DevScalars* sc, double* E, double* S, uint32_t* R, uint32_t* F,
                             double* wc, double* wn, unsigned int* wcnt, double* wsum,
-                            uint8_t* src, void* rule, hipStream_t st) {
+                            uint8_t* src, void* rule, void* bits, hipStream_t st) {
   using V4 = typename Vec4<T>::type;
   const V4* f = static_cast<const V4*>(field);
   const MaskSegs ms{E, R, F, wc, wn};
@@ -783,16 +858,16 @@ hipError_t launch_mask_walk(int method, const RayRec* rays, int64_t nrays, const
   }
   // setup tile pass: in-tile sums after the last restart, the weights and
   // the run starts
-  return launch_tile_pass_masked<T, true>(method, ntiles, tile_ptr, segs, g, tg, wp, field, aux, F,
-                                          wc, wn, nullptr, nullptr, nullptr, 1, sc, nullptr,
-                                          nullptr, S, wcnt, wsum, src, st);
+  return launch_tile_pass_masked<T, true, false>(method, ntiles, tile_ptr, segs, g, tg, wp, field,
+                                                 aux, F, wc, wn, nullptr, nullptr, nullptr, 1, sc,
+                                                 nullptr, nullptr, S, wcnt, wsum, src, bits, st);
 }
 #define OMNI_MW_INST(T)                                                                        \
   template hipError_t launch_mask_walk<T>(                                                      \
       int, const RayRec*, int64_t, const DirConst*, GridDesc, TileGrid, const WalkParams&,       \
       const void*, const double*, const unsigned int*, const unsigned long long*, int64_t, int,  \
       const unsigned long long*, const SegRec*, const DevScalars*, double*, double*, uint32_t*,  \
-      uint32_t*, double*, double*, unsigned int*, double*, uint8_t*, void*, hipStream_t);
+      uint32_t*, double*, double*, unsigned int*, double*, uint8_t*, void*, void*, hipStream_t);
 OMNI_MW_INST(float)
 OMNI_MW_INST(double)
 #undef OMNI_MW_INST
@@ -802,7 +877,7 @@ hipError_t launch_mask_reuse(int method, int ntiles, const unsigned long long* t
                              const SegRec* segs, GridDesc g, TileGrid tg, const WalkParams& wp,
                              const void* field, const double* aux, const DevScalars* sc,
                              double* E, double* S, const uint32_t* F, unsigned int* wcnt,
-                             uint8_t* src, hipStream_t st) {
+                             uint8_t* src, void* bits, hipStream_t st) {
   if (method != kMaskUnit) return hipErrorInvalidValue;
   using V4 = typename Vec4<T>::type;
   const V4* f = static_cast<const V4*>(field);
@@ -816,19 +891,20 @@ hipError_t launch_mask_reuse(int method, int ntiles, const unsigned long long* t
                        wp, f, F, E);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return launch_tile_pass_masked<T, true>(method, ntiles, tile_ptr, segs, g, tg, wp, field, aux, F,
-                                          nullptr, nullptr, nullptr, nullptr, nullptr, 1, sc,
-                                          nullptr, nullptr, S, wcnt, nullptr, src, st);
+  return launch_tile_pass_masked<T, true, false>(method, ntiles, tile_ptr, segs, g, tg, wp, field,
+                                                 aux, F, nullptr, nullptr, nullptr, nullptr,
+                                                 nullptr, 1, sc, nullptr, nullptr, S, wcnt,
+                                                 nullptr, src, bits, st);
 }
 template hipError_t launch_mask_reuse<float>(int, int, const unsigned long long*, const SegRec*,
                                              GridDesc, TileGrid, const WalkParams&, const void*,
                                              const double*, const DevScalars*, double*, double*,
-                                             const uint32_t*, unsigned int*, uint8_t*,
+                                             const uint32_t*, unsigned int*, uint8_t*, void*,
                                              hipStream_t);
 template hipError_t launch_mask_reuse<double>(int, int, const unsigned long long*, const SegRec*,
                                               GridDesc, TileGrid, const WalkParams&, const void*,
                                               const double*, const DevScalars*, double*, double*,
-                                              const uint32_t*, unsigned int*, uint8_t*,
+                                              const uint32_t*, unsigned int*, uint8_t*, void*,
                                               hipStream_t);
 
 hipError_t launch_mask_carry(int64_t nrays, const unsigned int* nseg,
@@ -847,23 +923,28 @@ hipError_t launch_tile_masked(int method, int ntiles, const unsigned long long* 
                               const void* field, const double* aux, const uint32_t* F,
                               const double* wc, const double* wn, const double* cval,
                               const double* p0, const double* p1, int k, const DevScalars* sc,
-                              long long* sumfx, double* sumd, hipStream_t st) {
-  return launch_tile_pass_masked<T, false>(method, ntiles, tile_ptr, segs, g, tg, wp, field, aux,
-                                           F, wc, wn, cval, p0, p1, k, sc, sumfx, sumd, nullptr,
-                                           nullptr, nullptr, nullptr, st);
+                              long long* sumfx, double* sumd, void* bits, hipStream_t st) {
+  if (!p0)
+    return launch_tile_pass_masked<T, false, false>(method, ntiles, tile_ptr, segs, g, tg, wp,
+                                                    field, aux, F, wc, wn, cval, p0, p1, k, sc,
+                                                    sumfx, sumd, nullptr, nullptr, nullptr,
+                                                    nullptr, bits, st);
+  return launch_tile_pass_masked<T, false, true>(method, ntiles, tile_ptr, segs, g, tg, wp, field,
+                                                 aux, F, wc, wn, cval, p0, p1, k, sc, sumfx, sumd,
+                                                 nullptr, nullptr, nullptr, nullptr, bits, st);
 }
 template hipError_t launch_tile_masked<float>(int, int, const unsigned long long*, const SegRec*,
                                               GridDesc, TileGrid, const WalkParams&, const void*,
                                               const double*, const uint32_t*, const double*,
                                               const double*, const double*, const double*,
                                               const double*, int, const DevScalars*, long long*,
-                                              double*, hipStream_t);
+                                              double*, void*, hipStream_t);
 template hipError_t launch_tile_masked<double>(int, int, const unsigned long long*, const SegRec*,
                                                GridDesc, TileGrid, const WalkParams&, const void*,
                                                const double*, const uint32_t*, const double*,
                                                const double*, const double*, const double*,
                                                const double*, int, const DevScalars*, long long*,
-                                               double*, hipStream_t);
+                                               double*, void*, hipStream_t);
 
 // ---------------------------------------------------------------------------
 // The masked methods' affine schedule.  A run's value at a visit is
@@ -917,11 +998,11 @@ k_tile_rows(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
             GridDesc g, TileGrid tg, WalkParams wp, const double* __restrict__ aux,
             const uint32_t* __restrict__ F, const uint32_t* __restrict__ runsrc,
             const int* __restrict__ sid, unsigned int* __restrict__ cnt,
-            const unsigned long long* __restrict__ rowptr, unsigned int* __restrict__ esrc) {
+            const unsigned long long* __restrict__ rowptr, unsigned int* __restrict__ esrc,
+            const StepBits* __restrict__ bits) {
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kVox = kTile * kTile * kTile;
-  __shared__ double s_aux[kVox];
   __shared__ int s_sid[kVox];
   __shared__ unsigned int s_n[kVox];
   const int tile = (int)xcd_block();
@@ -933,7 +1014,6 @@ k_tile_rows(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
     const bool in = i < g.X && j < g.Y && kk < g.Z;
     const int64_t gv = i + j * sy + kk * sz;
     const int sl = lds_slot<kBits>(l);
-    s_aux[sl] = in ? aux[gv] : 0.0;
     s_sid[sl] = in ? sid[gv] : -1;
     s_n[sl] = 0u;
   }
@@ -952,7 +1032,7 @@ k_tile_rows(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
     const int d0 = (sg & 1u) ? 1 : -1;
     const int d1 = (sg & 2u) ? kTile : -kTile;
     const int d2 = (sg & 4u) ? kTile * kTile : -kTile * kTile;
-    bool p0set = (f & kFlagP0) != 0, outthr = (f & kFlagOut) != 0;
+    const StepBits sb = bits[jj];
     const uint32_t mode = f & 3u;
     uint32_t t = mode == kModeCont ? runsrc[sr.g]
                                    : (mode == kModeRestart ? (uint32_t)gvox(lv) : kNoRun);
@@ -972,14 +1052,14 @@ k_tile_rows(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
 #pragma unroll 1
     for (int wi = 0; wi < 3 && rem > 0; wi++) {
       const int m = rem < 16 ? rem : 16;
+      uint32_t w = wi == 0 ? sb.w[0] : (wi == 1 ? sb.w[1] : sb.w[2]);
       for (int q = 0; q < m; q++) {
         const int a = (int)(cw & 3u);
         cw >>= 2;
         const int ln = lv + (a == 0 ? d0 : (a == 1 ? d1 : d2));
-        const double cn = s_aux[lds_slot<kBits>(ln)];
-        const StepRule d = rule_step<kMethod>(wp, a, cn, p0set, outthr);
-        if (d.add) emit(ln);
-        if (d.restart) src = s_sid[lds_slot<kBits>(ln)];
+        if (w & 1u) emit(ln);
+        if (w & 0x10000u) src = s_sid[lds_slot<kBits>(ln)];
+        w >>= 1;
         lv = ln;
       }
       rem -= m;
@@ -1013,11 +1093,12 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
                const int* __restrict__ sid, const int* __restrict__ tfirst,
                unsigned int* __restrict__ tcnt, const unsigned long long* __restrict__ tbase,
                unsigned int* __restrict__ esrc, unsigned short* __restrict__ erow,
-               double* __restrict__ ew, int parts) {
+               double* __restrict__ ew, const StepBits* __restrict__ bits, int parts) {
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kVox = kTile * kTile * kTile;
-  __shared__ double s_aux[kVox];
+  constexpr bool kRule = kRuled<kMethod>, kCurl = kCurlW<kMethod>;
+  __shared__ double s_cw[kCurl ? kVox : 1];  // curl / 10000
   __shared__ int s_sid[kVox];
   __shared__ unsigned int s_total;
   const TilePart tp = tile_part(xcd_block(), parts);
@@ -1031,7 +1112,7 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
     const bool in = i < g.X && j < g.Y && kk < g.Z;
     const int64_t gv = i + j * sy + kk * sz;
     const int sl = lds_slot<kBits>(l);
-    s_aux[sl] = in ? aux[gv] : 0.0;
+    if constexpr (kCurl) s_cw[sl] = (in ? aux[gv] : 0.0) / 10000;
     s_sid[sl] = in ? sid[gv] : -1;
   }
   __syncthreads();
@@ -1053,7 +1134,9 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
     const int d0 = (sg & 1u) ? 1 : -1;
     const int d1 = (sg & 2u) ? kTile : -kTile;
     const int d2 = (sg & 4u) ? kTile * kTile : -kTile * kTile;
-    bool p0set = (f & kFlagP0) != 0, outthr = (f & kFlagOut) != 0;
+    bool p0set = (f & kFlagP0) != 0;
+    StepBits sb{{0, 0, 0}};
+    if constexpr (kRule) sb = bits[jj];
     const uint32_t mode = f & 3u;
     const uint32_t t = mode == kModeCont ? runsrc[sr.g]
                                          : (mode == kModeRestart ? (uint32_t)gvox(lv) : kNoRun);
@@ -1087,16 +1170,23 @@ k_tile_entries(const unsigned long long* __restrict__ tile_ptr, const SegRec* __
 #pragma unroll 1
     for (int wi = 0; wi < 3 && rem > 0; wi++) {
       const int m = rem < 16 ? rem : 16;
+      uint32_t w = wi == 0 ? sb.w[0] : (wi == 1 ? sb.w[1] : sb.w[2]);
       for (int q = 0; q < m; q++) {
         const int a = (int)(cw & 3u);
         cw >>= 2;
         const int ln = lv + (a == 0 ? d0 : (a == 1 ? d1 : d2));
-        const double cn = s_aux[lds_slot<kBits>(ln)];
-        const StepRule d = rule_step<kMethod>(wp, a, cn, p0set, outthr);
+        StepRule d{true, false, false};
+        if constexpr (kRule) {
+          d.add = w & 1u;
+          d.restart = w & 0x10000u;
+          d.keep_w = p0set && wp.faithful && a == 2;
+          w >>= 1;
+          p0set = p0set || d.restart;
+        }
         if (d.add) {
           bool added = true;
-          if (kCurlW<kMethod>) {
-            curl += cn / 10000;
+          if constexpr (kCurl) {
+            curl += s_cw[lds_slot<kBits>(ln)];
             num += 1.0;
             added = kMethod != kMaskWeighted || curl != 0.0;
           }
@@ -1450,10 +1540,11 @@ hipError_t launch_tile_rows(bool fill, int method, int ntiles, const unsigned lo
                             const SegRec* segs, GridDesc g, TileGrid tg, const WalkParams& wp,
                             const double* aux, const uint32_t* F, const uint32_t* runsrc,
                             const int* sid, unsigned int* cnt, const unsigned long long* rowptr,
-                            unsigned int* esrc, hipStream_t st) {
+                            unsigned int* esrc, const void* bits, hipStream_t st) {
 #define OMNI_TR(M, B, FL)                                                                       \
   hipLaunchKernelGGL((k_tile_rows<M, B, FL>), dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g, \
-                     tg, wp, aux, F, runsrc, sid, cnt, rowptr, esrc)
+                     tg, wp, aux, F, runsrc, sid, cnt, rowptr, esrc,                                  \
+                     static_cast<const StepBits*>(bits))
 #define OMNI_TR_B(M, FL)                  \
   do {                                    \
     if (tg.bits == 3) OMNI_TR(M, 3, FL);  \
@@ -1514,12 +1605,12 @@ hipError_t launch_tile_entries(bool fill, int method, int ntiles,
                                const uint32_t* runsrc, const int* sid, const int* tfirst,
                                unsigned int* tcnt, const unsigned long long* tbase,
                                unsigned int* esrc, unsigned short* erow, double* ew,
-                               hipStream_t st) {
+                               const void* bits, hipStream_t st) {
   const int parts = tile_entries_parts(method, ntiles);
 #define OMNI_TE(M, B, FL)                                                                       \
   hipLaunchKernelGGL((k_tile_entries<M, B, FL>), dim3(ntiles * parts), dim3(1024), 0, st,         \
                      tile_ptr, segs, g, tg, wp, aux, F, wc, wn, runsrc, sid, tfirst, tcnt, tbase,  \
-                     esrc, erow, ew, parts)
+                     esrc, erow, ew, static_cast<const StepBits*>(bits), parts)
 #define OMNI_TE_B(M, FL)                  \
   do {                                    \
     if (tg.bits == 3) OMNI_TE(M, 3, FL);  \

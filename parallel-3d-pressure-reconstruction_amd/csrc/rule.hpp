@@ -29,43 +29,52 @@ constexpr uint32_t kFlagP0 = 8u;       // run started (p0set) after the first vi
 constexpr uint32_t kFlagOut = 16u;     // inside a high / masked stretch (outthr)
 constexpr uint32_t kFlagRestart = 32u; // some visit of the segment restarts the run
 
-// The rule of one step onto a voxel with curl / mask value cn along axis a
-// (naive_select: the reference's asymmetries when faithful).  add: the visit
-// adds p0 + pint (the step's term joins pint first); restart: p0 = p here,
-// pint = 0, and the curl weights restart unless keep_w.
+// What the rule asks of a voxel's curl / mask value (a NaN is nonzero only).
+constexpr unsigned int kClsValid = 1u;    // below the threshold and nonzero
+constexpr unsigned int kClsNonzero = 2u;
+constexpr unsigned int kClsHigh = 4u;     // at the threshold or above
+__device__ __forceinline__ unsigned int rule_class(const WalkParams& wp, double cn) {
+  const double thr = wp.thr;
+  return (cn < thr && cn != 0.0 ? kClsValid : 0u) | (cn != 0.0 ? kClsNonzero : 0u) |
+         (cn >= thr ? kClsHigh : 0u);
+}
+
+// The rule of one step along axis a onto a voxel of class cls (naive_select:
+// the reference's asymmetries when faithful).  add: the visit adds p0 + pint
+// (the step's term joins pint first); restart: p0 = p here, pint = 0, and the
+// curl weights restart unless keep_w.
 struct StepRule {
   bool add, restart, keep_w;
 };
 
 template <int kMethod>
-__device__ __forceinline__ StepRule rule_step(const WalkParams& wp, int a, double cn, bool& p0set,
-                                              bool& outthr) {
+__device__ __forceinline__ StepRule rule_step_class(const WalkParams& wp, int a, unsigned int cls,
+                                                    bool& p0set, bool& outthr) {
   StepRule r{false, false, false};
   if (kMethod == kMaskWeighted || kMethod == kMaskPlain) {
     r.add = true;  // every step adds (Weighted: when the curl sum is nonzero)
     return r;
   }
-  const double thr = wp.thr;
-  const bool faithful = wp.faithful != 0;
-  const bool valid = cn < thr && cn != 0.0;
-  if (!p0set) {
-    const bool ok = (faithful && a != 0) ? (cn != 0.0) : valid;
-    if (ok) {
-      p0set = true;
-      r.restart = true;
-    }
-  } else {
-    r.add = !outthr && valid;
-    const bool enter_high = (faithful && a != 0) ? (!outthr && cn >= thr)
-                                                 : ((!outthr && cn >= thr) || cn == 0.0);
-    if (enter_high) outthr = true;
-    if (outthr && valid) {
-      r.restart = true;
-      outthr = false;
-      r.keep_w = faithful && a == 2;
-    }
-  }
+  const bool faithful = wp.faithful != 0, loose = faithful && a != 0;
+  const bool valid = cls & kClsValid, nonzero = cls & kClsNonzero, high = cls & kClsHigh;
+  // no run yet: it may start here
+  const bool start = !p0set && (loose ? nonzero : valid);
+  // in a run: a valid voxel adds; a high (or zero) one interrupts it until
+  // the next valid one, which restarts it
+  r.add = p0set && !outthr && valid;
+  const bool out = outthr || high || (!loose && !nonzero);
+  const bool again = p0set && out && valid;
+  r.restart = start || again;
+  r.keep_w = again && faithful && a == 2;
+  outthr = p0set ? out && !valid : outthr;
+  p0set = p0set || start;
   return r;
+}
+
+template <int kMethod>
+__device__ __forceinline__ StepRule rule_step(const WalkParams& wp, int a, double cn, bool& p0set,
+                                              bool& outthr) {
+  return rule_step_class<kMethod>(wp, a, rule_class(wp, cn), p0set, outthr);
 }
 
 // The entry voxel of a ray: a run starts there (p0 = p, no add) when valid.

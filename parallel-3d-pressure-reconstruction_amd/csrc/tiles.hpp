@@ -173,7 +173,10 @@ hipError_t launch_mask_walk(int method, const RayRec* rays, int64_t nrays, const
                             const unsigned long long* tile_ptr, const SegRec* segs,
                             const DevScalars* sc, double* E, double* S, uint32_t* R, uint32_t* F,
                             double* wc, double* wn, unsigned int* wcnt, double* wsum,
-                            uint8_t* src, void* rule, hipStream_t st);
+                            uint8_t* src, void* rule, void* bits, hipStream_t st);
+// step bits of the rule (plain-mask, Select; else none): written by the setup
+// pass, read by the tile passes and the rows
+size_t step_bits_bytes(int method, int64_t nsegs);
 size_t mask_rule_bytes(int method, int64_t nval);
 // plain-mask records F kept from an earlier field with the same mask: the new
 // field's entering-step terms E, then the setup pass (segment sums S, the
@@ -183,7 +186,7 @@ hipError_t launch_mask_reuse(int method, int ntiles, const unsigned long long* t
                              const SegRec* segs, GridDesc g, TileGrid tg, const WalkParams& wp,
                              const void* field, const double* aux, const DevScalars* sc,
                              double* E, double* S, const uint32_t* F, unsigned int* wcnt,
-                             uint8_t* src, hipStream_t st);
+                             uint8_t* src, void* bits, hipStream_t st);
 // the tile rule replay alone (no setup pass): E, R, F (wc, wn) per segment
 template <typename T>
 hipError_t launch_rule_replay(int method, int64_t nrays, const unsigned int* nseg,
@@ -211,13 +214,14 @@ hipError_t launch_mask_carry(int64_t nrays, const unsigned int* nseg,
                              const uint32_t* R, const uint32_t* F, const double* p0,
                              const double* p1, int k, const DevScalars* sc, double* cval,
                              hipStream_t st);
+// p0 null: p = 0
 template <typename T>
 hipError_t launch_tile_masked(int method, int ntiles, const unsigned long long* tile_ptr,
                               const SegRec* segs, GridDesc g, TileGrid tg, const WalkParams& wp,
                               const void* field, const double* aux, const uint32_t* F,
                               const double* wc, const double* wn, const double* cval,
                               const double* p0, const double* p1, int k, const DevScalars* sc,
-                              long long* sumfx, double* sumd, hipStream_t st);
+                              long long* sumfx, double* sumd, void* bits, hipStream_t st);
 
 
 // adjoint.hip: the plain method's transposed traversals on the tile engine
@@ -255,7 +259,7 @@ hipError_t launch_tile_rows(bool fill, int method, int ntiles, const unsigned lo
                             const SegRec* segs, GridDesc g, TileGrid tg, const WalkParams& wp,
                             const double* aux, const uint32_t* F, const uint32_t* runsrc,
                             const int* sid, unsigned int* cnt, const unsigned long long* rowptr,
-                            unsigned int* esrc, hipStream_t st);
+                            unsigned int* esrc, const void* bits, hipStream_t st);
 // compact ids of the flagged voxels in tile order, over many workgroups
 // (bcnt: source_ids_tiled_blocks(tg) u32); tile t's rows are
 // [tfirst[t], tfirst[t + 1]) (tfirst: ntiles + 1 ints)
@@ -277,7 +281,7 @@ hipError_t launch_tile_entries(bool fill, int method, int ntiles,
                                const uint32_t* runsrc, const int* sid, const int* tfirst,
                                unsigned int* tcnt, const unsigned long long* tbase,
                                unsigned int* esrc, unsigned short* erow, double* ew,
-                               hipStream_t st);
+                               const void* bits, hipStream_t st);
 hipError_t launch_mtile_accum(int k, int nchunks, const MaskChunk* chunks, const int* tfirst,
                               const unsigned int* esrc, const unsigned short* erow,
                               const double* ew, const double* p0, const double* p1,
