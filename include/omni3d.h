@@ -267,7 +267,9 @@ int omni3d_es_inner_weighted_minicurl(long X, long Y, long Z, int NoAngles, floa
  * p = pn / pcountinner and pn = 0. */
 int omni3d_devide_count_inner(long X, long Y, long Z, float* p, float* pn,
                               const float* pcountinner, void* hip_stream);
-/* Frees the calling thread's hidden drop-in context (plan, staged field). */
+/* Frees the calling thread's hidden drop-in context (plan, staged field), and
+ * returns the device memory that released objects of the library left for the
+ * next ones (2 GiB at most; also returned when the driver has no more). */
 void omni3d_dropin_release(void);
 
 /* The same six under the reference kernels' own names and argument lists

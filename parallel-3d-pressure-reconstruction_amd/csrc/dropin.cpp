@@ -359,7 +359,10 @@ int omni3d_devide_count_inner(long X, long Y, long Z, float* p, float* pn,
   return OMNI3D_OK;
 }
 
-void omni3d_dropin_release(void) { g_kc.release(); }
+void omni3d_dropin_release(void) {
+  g_kc.release();
+  (void)device_release_unused();
+}
 
 // The reference kernels' own names (a call site minus its <<<grid, block>>>).
 void omni3dparallellinesESInner(long Xsize, long Ysize, long Zsize, int NoAngles,

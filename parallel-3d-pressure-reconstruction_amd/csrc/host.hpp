@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/omni3d.h"
+#include "devpool.hpp"
 #include "words.hpp"
 #include "geometry.hpp"
 #include "kernels.hpp"
@@ -33,19 +34,20 @@ class DevBuf {
   hipError_t alloc(size_t bytes) {
     if (bytes <= size_) return hipSuccess;
     release();
-    hipError_t e = hipMalloc(&ptr_, bytes ? bytes : 1);
+    const hipError_t e = device_alloc(&ptr_, bytes, &cap_, &dev_);
     if (e == hipSuccess) size_ = bytes;
-    else ptr_ = nullptr;
     return e;
   }
   void release() {
-    if (ptr_) (void)hipFree(ptr_);
+    device_free(ptr_, cap_, dev_);
     ptr_ = nullptr;
     size_ = 0;
   }
   void swap(DevBuf& o) {
     std::swap(ptr_, o.ptr_);
     std::swap(size_, o.size_);
+    std::swap(cap_, o.cap_);
+    std::swap(dev_, o.dev_);
   }
   template <typename T>
   T* as() const {
@@ -55,7 +57,8 @@ class DevBuf {
 
  private:
   void* ptr_ = nullptr;
-  size_t size_ = 0;
+  size_t size_ = 0, cap_ = 0;  // asked for; the block's
+  int dev_ = 0;
 };
 
 // Rows of the source iteration as merged words (words.hpp).
