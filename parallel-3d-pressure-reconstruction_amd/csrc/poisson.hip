@@ -275,140 +275,190 @@ k_redblack_fused(int X, int Y, int Z, double omega, const double* __restrict__ p
   }
 }
 
-// kK whole red-black iterations in one pass (temporal blocking): the same
-// z-march with 2 kK half sweeps ("stages") in flight.  Stage s (red for even
-// s, black for odd s, iteration s / 2 + 1) takes plane k - s at step k over
-// the column plus a halo of h = 2 kK - 1 - s voxels in x, y and z: each
-// stage reads the previous stage's colour on the planes around it, which
-// that stage finished one step earlier or earlier in this step, so the
-// stages run in order within a step, a barrier apart.  The column's planes
-// load with a halo of 2 kK (a ring of 2 kK + 3 planes; the plane two steps
-// ahead loads into registers during a step); a plane is stored one step
-// after the last stage finished it.  Reads come from p_in and writes go to
-// p_out; every voxel update is the same expression on the same values as in
-// the half-sweep kernels, so kK iterations here equal kK single ones bit for
-// bit.  The halo voxels are updated redundantly by each column that needs
-// them (the price of one read and one write of p per kK iterations).
-template <int kTX, int kTY, int kZ, int kK, int kThreads>
-__global__ void __launch_bounds__(kThreads)
-k_redblack_multi(int X, int Y, int Z, double omega, const double* __restrict__ pin,
+// s / n for n = 1..6 with r = 1 / n rounded: the quotient's estimate and its
+// exact remainder give the rounded quotient (Markstein's correction) in three
+// operations for the division's dozen; zeros, subnormals, infinities and NaN
+// take the division.
+__device__ __forceinline__ double div_small(double s, double n, double r) {
+  const double q = s * r;
+  const double rem = __builtin_fma(-q, n, s);
+  double v = __builtin_fma(rem, r, q);
+  const unsigned int e = ((unsigned int)(__double_as_longlong(s) >> 32)) & 0x7fffffffu;
+  if (e - 0x07000000u >= 0x78f00000u) v = s / n;  // |s| < 2^-911, infinite or NaN
+  return v;
+}
+
+// kK whole red-black iterations in one pass (temporal blocking): a z-march
+// over a column of kTX x kTY voxels with 2 kK half sweeps ("stages") in
+// flight, stage s (red for even s, black for odd s, iteration s / 2 + 1) on
+// plane k - s at step k, over the column plus a halo of h = 2 kK - 1 - s
+// voxels in x, y and z (updated redundantly by each column that needs them:
+// the price of one read and one write of p per kK iterations).
+//
+// A thread keeps two neighbouring voxels of a row, one of each colour, through
+// all planes: their p and right-hand sides of the planes in flight stay in
+// registers, loaded once, so the neighbours in z and one in x are its own.
+// The other x neighbour and the two in y come through LDS: what stage s - 1
+// wrote of a plane is read by stage s a step later, two slots in turn, one
+// barrier a step.  Within a step the stages run in order, since stage s reads
+// the plane above its own as stage s - 1 has just left it.  (With the planes
+// in an LDS ring and four barriers, every stage read its right-hand side from
+// memory again -- 1.2 GB a pass for 0.5 at 256^3 -- and spent most of its
+// instructions on places and bounds: 232 us a pass; a ring with one barrier
+// 200; this 108, of which one read of p and of the right-hand side and one
+// write take 82.)
+//
+// Voxels outside the box are -0.0, which adds to any value without changing
+// it: no branch per neighbour, same sums bit for bit.  Reads come from p_in
+// and writes go to p_out; every voxel update is the same expression on the
+// same values as in the half-sweep kernels.
+template <int kTX, int kTY, int kK>
+constexpr int rb_multi_threads() {
+  return ((kTX / 2 + 2 * kK) * (kTY + 4 * kK) + 63) / 64 * 64;
+}
+
+template <int kTX, int kTY, int kK>
+__global__ void __launch_bounds__((rb_multi_threads<kTX, kTY, kK>()))
+k_redblack_multi(int X, int Y, int Z, int zc, double omega, const double* __restrict__ pin,
                  const double* __restrict__ rhs, double* __restrict__ pout,
                  const SorState* __restrict__ st) {
-  if (st->stop_at) return;
+  using Two = double __attribute__((ext_vector_type(2), aligned(8)));
   constexpr int kStages = 2 * kK;
   constexpr int kHalo = 2 * kK;
-  constexpr int kW = kTX + 2 * kHalo, kH = kTY + 2 * kHalo;
-  constexpr int kRing = 2 * kK + 3;
-  constexpr int kLoads = (kW * kH + kThreads - 1) / kThreads;
-  static_assert(kTX % 2 == 0, "even column width");
-  __shared__ double P[kRing][kH][kW];
+  constexpr int kPairs = kTX / 2 + kHalo, kH = kTY + 2 * kHalo;
+  constexpr int kCells = kPairs * kH;
+  constexpr int kRing = kStages + 4;  // planes k + 3 .. k - kStages
+  static_assert(kTX % 2 == 0 && kRing % 2 == 0, "pairs; the step's parity is the ring's");
+  __shared__ double s_p[2][kStages][kCells];
+  if (st->stop_at) return;
   const int x0 = (int)blockIdx.x * kTX, y0 = (int)blockIdx.y * kTY;
-  const int z0 = (int)blockIdx.z * kZ, z1 = min(Z, z0 + kZ);
-  const int64_t sy = X, sz = (int64_t)X * Y;
+  const int z0 = (int)blockIdx.z * zc, z1 = min(Z, z0 + zc);
+  const int64_t sz = (int64_t)X * Y;
   const int tid = (int)threadIdx.x;
-  auto slot = [](int k) { return (k + 8 * kRing) % kRing; };  // k >= -2 kHalo
-  double pf[kLoads];
-  auto issue = [&](int k) {
-    if (k < 0 || k >= Z) return;
+  const int cell = tid < kCells ? tid : kCells - 1;  // (the last wavefront's spare lanes)
+  const int jl = cell / kPairs, xh = cell % kPairs;
+  const int j = y0 - kHalo + jl, i = x0 - kHalo + 2 * xh;  // the pair's first voxel (i even)
+  const int kb = z0 - (kStages - 1), ke = z1 - 1 + (kStages - 1);
+  // which of the pair is red at step kb (the black one is stage 0's other)
+  const int e0 = (j + kb) & 1;
+  const bool row_in = j >= 0 && j < Y;
+  const bool in0 = row_in && i >= 0 && i < X, in1 = row_in && i + 1 >= 0 && i + 1 < X;
+  // (a pair at the end of an odd row is loaded one voxel earlier, pairs out
+  // of the box from the plane's first voxels: no load under a branch)
+  const bool odd_end = i == X - 1;
+  const int64_t at = in0 ? (i - (odd_end ? 1 : 0)) + (int64_t)j * X : 0;
+  const int64_t put = in0 ? i + (int64_t)j * X : 0;
+  const bool mine = tid < kCells && jl >= kHalo && jl < kHalo + kTY && xh >= kHalo / 2 &&
+                    xh < kHalo / 2 + kTX / 2;
+  const bool put0 = mine && in0, put1 = mine && in1;
+  // per stage and voxel of the pair: whether this column updates it, and how
+  // many neighbours it has in x and y
+  unsigned int act = 0;
 #pragma unroll
-    for (int m = 0; m < kLoads; m++) {
-      const int l = tid + m * kThreads;
-      const int i = x0 - kHalo + l % kW, j = y0 - kHalo + l / kW;
-      if (l < kW * kH && i >= 0 && i < X && j >= 0 && j < Y) pf[m] = pin[i + j * sy + k * sz];
-    }
-  };
-  auto commit = [&](int k) {
-    if (k < 0 || k >= Z) return;
-#pragma unroll
-    for (int m = 0; m < kLoads; m++) {
-      const int l = tid + m * kThreads;
-      const int i = x0 - kHalo + l % kW, j = y0 - kHalo + l / kW;
-      if (l < kW * kH && i >= 0 && i < X && j >= 0 && j < Y) P[slot(k)][l / kW][l % kW] = pf[m];
-    }
-  };
-  // in-box neighbour sum in the reference's order (x-, x+, y-, y+, z-, z+)
-  auto update = [&](int i, int j, int k, double r) {
-    const int xx = i - x0 + kHalo, yy = j - y0 + kHalo;
-    double(*Pc)[kW] = P[slot(k)];
-    double s = 0.0;
-    int n = 0;
-    if (i > 0) { s = n ? s + Pc[yy][xx - 1] : Pc[yy][xx - 1]; n++; }
-    if (i < X - 1) { s = n ? s + Pc[yy][xx + 1] : Pc[yy][xx + 1]; n++; }
-    if (j > 0) { s = n ? s + Pc[yy - 1][xx] : Pc[yy - 1][xx]; n++; }
-    if (j < Y - 1) { s = n ? s + Pc[yy + 1][xx] : Pc[yy + 1][xx]; n++; }
-    if (k > 0) { const double q = P[slot(k - 1)][yy][xx]; s = n ? s + q : q; n++; }
-    if (k < Z - 1) { const double q = P[slot(k + 1)][yy][xx]; s = n ? s + q : q; n++; }
-    s += r;
-    s = s / n;
-    const double old = Pc[yy][xx];
-    Pc[yy][xx] = old + omega * (s - old);
-  };
-  // stage s on plane m: the voxels of its colour in the column plus halo h;
-  // thread tid takes voxels tid + q kThreads, q < kPer
-  constexpr int kPer = ((kTX / 2 + kStages - 1) * (kTY + 2 * (kStages - 1)) + kThreads - 1) /
-                       kThreads;
-  auto voxel = [&](int s, int m, int q, int* i, int* j) {
+  for (int s = 0; s < kStages; s++) {
     const int h = kStages - 1 - s;
-    const int half = kTX / 2 + h, rows = kTY + 2 * h;
-    const int l = tid + q * kThreads;
-    *j = y0 - h + l / half;
-    *i = x0 - h + ((x0 - h + *j + m + (s & 1)) & 1) + 2 * (l % half);
-    return l < half * rows && m >= 0 && m < Z && m >= z0 - h && m < z1 + h && *i >= 0 &&
-           *i < X && *j >= 0 && *j < Y;
+    const bool rows = tid < kCells && jl >= kHalo - h && jl < kHalo + kTY + h;
+    const int lo = kHalo - h, hi = kHalo + kTX + h;
+    act |= (rows && in0 && 2 * xh >= lo && 2 * xh < hi ? 1u : 0u) << (2 * s);
+    act |= (rows && in1 && 2 * xh + 1 >= lo && 2 * xh + 1 < hi ? 1u : 0u) << (2 * s + 1);
+  }
+  const int ny = (j > 0) + (j < Y - 1);
+  const double n0 = (double)(2 + ny + (i > 0) + (i < X - 1));
+  const double n1 = (double)(2 + ny + (i + 1 > 0) + (i + 1 < X - 1));
+  // the voxel that a step's stages update: e = e0 at even steps
+  const double nE[2] = {e0 ? n1 : n0, e0 ? n0 : n1};
+  const double rE[2] = {1.0 / nE[0], 1.0 / nE[1]};
+  const unsigned int aE[2] = {e0 ? act >> 1 : act, e0 ? act : act >> 1};
+  const int xE[2] = {e0 ? 1 : -1, e0 ? -1 : 1};  // its neighbour outside the pair
+  double pr[kRing], pb[kRing], rr[kRing], rb[kRing];  // red, black; at first the pair as it lies
+#pragma unroll
+  for (int u = 0; u < kRing; u++) pr[u] = pb[u] = rr[u] = rb[u] = -0.0;
+  auto load = [&](const double* __restrict__ a, int k, double* v0, double* v1) {
+    const Two t = *reinterpret_cast<const Two*>(a + (k < 0 ? 0 : (k >= Z ? Z - 1 : k)) * sz + at);
+    *v0 = odd_end ? t.y : t.x;
+    *v1 = t.y;
   };
-  // the right-hand sides of a step's stages load into registers one step
-  // ahead
-  double rr[kStages][kPer];
-  auto issue_rhs = [&](int k) {
-#pragma unroll
-    for (int s = 0; s < kStages; s++) {
-#pragma unroll
-      for (int q = 0; q < kPer; q++) {
-        int i, j;
-        if (voxel(s, k - s, q, &i, &j)) rr[s][q] = rhs[i + j * sy + (int64_t)(k - s) * sz];
-      }
-    }
+  // the pair of plane m by colour (par: whether its second voxel is red),
+  // -0.0 outside the box
+  auto colours = [&](int m, int par, double* r, double* b) {
+    const bool in = m >= 0 && m < Z;
+    const double v0 = in && in0 ? *r : -0.0, v1 = in && in1 ? *b : -0.0;
+    *r = par ? v1 : v0;
+    *b = par ? v0 : v1;
   };
-  auto stage = [&](int s, int m, const double (&r)[kPer]) {
+  // the slot of plane k + d at step k = kb + (a multiple of kRing) + u
+#define RB_SLOT(u, d) (((u) + (d) + 2 * kRing) % kRing)
+  load(pin, kb - 1, &pr[RB_SLOT(0, -1)], &pb[RB_SLOT(0, -1)]);
+  load(pin, kb, &pr[RB_SLOT(0, 0)], &pb[RB_SLOT(0, 0)]);
+  load(pin, kb + 1, &pr[RB_SLOT(0, 1)], &pb[RB_SLOT(0, 1)]);
+  load(pin, kb + 2, &pr[RB_SLOT(0, 2)], &pb[RB_SLOT(0, 2)]);
+  load(rhs, kb, &rr[RB_SLOT(0, 0)], &rb[RB_SLOT(0, 0)]);
+  load(rhs, kb + 1, &rr[RB_SLOT(0, 1)], &rb[RB_SLOT(0, 1)]);
+  colours(kb - 1, e0 ^ 1, &pr[RB_SLOT(0, -1)], &pb[RB_SLOT(0, -1)]);
+  colours(kb, e0, &pr[RB_SLOT(0, 0)], &pb[RB_SLOT(0, 0)]);
+  // what a step reads of the one before: stage 0 the black of its plane
+  if (tid < kCells) {
+    s_p[1][0][tid] = pb[RB_SLOT(0, 0)];
 #pragma unroll
-    for (int q = 0; q < kPer; q++) {
-      int i, j;
-      if (voxel(s, m, q, &i, &j)) update(i, j, m, r[q]);
-    }
-  };
-  const int kb = z0 - kStages + 1;  // the first step: stage 0 on its lowest plane
-  issue(kb - 1);
-  commit(kb - 1);
-  issue(kb);
-  commit(kb);
-  issue(kb + 1);
-  issue_rhs(kb);
-  for (int k = kb; k <= z1 + kStages - 1; k++) {
-    commit(k + 1);
-    issue(k + 2);
-    double r0[kStages][kPer];
+    for (int s = 1; s < kStages; s++) s_p[1][s][tid] = -0.0;
+  }
+  for (int kk = kb; kk <= ke; kk += kRing) {
 #pragma unroll
-    for (int s = 0; s < kStages; s++)
-#pragma unroll
-      for (int q = 0; q < kPer; q++) r0[s][q] = rr[s][q];
-    issue_rhs(k + 1);
-    __syncthreads();
-    stage(0, k, r0[0]);
-    // the plane the last stage finished at the previous step
-    const int ms = k - kStages;
-    if (ms >= z0 && ms < z1) {
-      const double(*Pb)[kW] = P[slot(ms)];
-      for (int l = tid; l < kTX * kTY; l += kThreads) {
-        const int i = x0 + (l % kTX), j = y0 + l / kTX;
-        if (i < X && j < Y) pout[i + j * sy + ms * sz] = Pb[j - y0 + kHalo][i - x0 + kHalo];
-      }
-    }
-#pragma unroll
-    for (int s = 1; s < kStages; s++) {
+    for (int u = 0; u < kRing; u++) {
+      const int k = kk + u;
+      if (k > ke) break;
       __syncthreads();
-      stage(s, k - s, r0[s]);
+      const double(*from)[kCells] = s_p[(u + 1) & 1];
+      double(*to)[kCells] = s_p[u & 1];
+      colours(k + 1, e0 ^ ((u + 1) & 1), &pr[RB_SLOT(u, 1)], &pb[RB_SLOT(u, 1)]);
+      {
+        // (the right-hand sides: outside the box they are not used)
+        const double v0 = rr[RB_SLOT(u, 0)], v1 = rb[RB_SLOT(u, 0)];
+        const bool par = e0 ^ (u & 1);
+        rr[RB_SLOT(u, 0)] = par ? v1 : v0;
+        rb[RB_SLOT(u, 0)] = par ? v0 : v1;
+      }
+      load(pin, k + 3, &pr[RB_SLOT(u, 3)], &pb[RB_SLOT(u, 3)]);
+      load(rhs, k + 2, &rr[RB_SLOT(u, 2)], &rb[RB_SLOT(u, 2)]);
+      if (tid < kCells) to[0][cell] = pb[RB_SLOT(u, 1)];
+#pragma unroll
+      for (int s = 0; s < kStages; s++) {
+        const int m = k - s, h = kStages - 1 - s;
+        double* own = s & 1 ? pb : pr;
+        const double* oth = s & 1 ? pr : pb;
+        const double r = (s & 1 ? rb : rr)[RB_SLOT(u, -s)];
+        if (m >= 0 && m < Z && m >= z0 - h && m < z1 + h && ((aE[u & 1] >> (2 * s)) & 1u)) {
+          double n = nE[u & 1], rn = rE[u & 1];
+          if (m == 0 || m == Z - 1) {
+            n -= (double)((m == 0) + (m == Z - 1));
+            rn = 1.0 / n;
+          }
+          // the neighbours in the reference's order (x-, x+, y-, y+, z-, z+;
+          // a sum of two is the same either way round)
+          double t = oth[RB_SLOT(u, -s)] + from[s][cell + xE[u & 1]];
+          t += from[s][cell - kPairs];
+          t += from[s][cell + kPairs];
+          t += oth[RB_SLOT(u, -s - 1)];
+          t += oth[RB_SLOT(u, -s + 1)];
+          t += r;
+          t = div_small(t, n, rn);
+          const double old = own[RB_SLOT(u, -s)];
+          own[RB_SLOT(u, -s)] = old + omega * (t - old);
+        }
+        if (s + 1 < kStages && tid < kCells) to[s + 1][cell] = own[RB_SLOT(u, -s)];
+      }
+      const int ms = k - (kStages - 1);
+      if (ms >= z0 && ms < z1) {
+        const bool par = e0 ^ ((u + kStages - 1) & 1);
+        const double r = pr[RB_SLOT(u, -(kStages - 1))], b = pb[RB_SLOT(u, -(kStages - 1))];
+        double* __restrict__ o = pout + put + ms * sz;
+        const Two v = {par ? b : r, par ? r : b};
+        if (put1) *reinterpret_cast<Two*>(o) = v;  // (i even and in the box if i + 1 is)
+        else if (put0) *o = v.x;
+      }
     }
   }
+#undef RB_SLOT
 }
 
 // Interior residual sum |sum_nb - 6 p + rhs| (sor3D.cpp:741-781) reduced
@@ -701,13 +751,18 @@ int omni3d_sor_solve_device(int X, int Y, int Z, double omega, int max_iter, dou
   // with no stop test between iterations (eps <= 0) pairs of iterations run
   // as one temporally blocked pass (k_redblack_multi, two iterations, same
   // columns); OMNI3D_SOR=single keeps one pass per iteration
-  // column 64 x 16 over 64 planes, 1024 threads, one workgroup per CU (97 KB
-  // of LDS): the fastest of 32-128 x 8-16 columns, 16-64 planes, 256-1024
-  // threads and two or three iterations per pass at 256^3
-  constexpr int mtx = 64, mty = 16, mtz = 64, mthreads = 1024;
+  // column 64 x 16, 14 wavefronts, one workgroup per CU; as many parts of the
+  // planes as give every CU a workgroup, of 16 planes at least (a part marches
+  // 6 planes more than it holds).  256^3, 200 iterations: 64 x 16 11.3 ms,
+  // 64 x 20 11.7, 56 x 24 11.5, 64 x 8 15.3, 32 x 16 15.7, 96 x 8 17.2; three
+  // iterations a pass 15.6 (64 x 10) and more
+  constexpr int mtx = 64, mty = 16, mthreads = rb_multi_threads<mtx, mty, 2>();
+  const int64_t mcols = (int64_t)((X + mtx - 1) / mtx) * ((Y + mty - 1) / mty);
+  const int mparts = (int)std::max<int64_t>(1, cu_count() / mcols);
+  const int mzc = std::max(16, (Z + mparts - 1) / mparts);
   const dim3 mgrid((unsigned int)((X + mtx - 1) / mtx), (unsigned int)((Y + mty - 1) / mty),
-                   (unsigned int)((Z + mtz - 1) / mtz));
-  const bool pairs = fused && eps <= 0.0 && !(env && std::strcmp(env, "single") == 0) &&
+                   (unsigned int)((Z + mzc - 1) / mzc));
+  const bool pairs = fused && X >= 2 && eps <= 0.0 && !(env && std::strcmp(env, "single") == 0) &&
                      mgrid.y <= 65535 && mgrid.z <= 65535;
   double* src = p_d;  // the buffer holding the latest iterate (fused passes)
   for (int it = 1; it <= max_iter; it++) {
@@ -715,8 +770,8 @@ int omni3d_sor_solve_device(int X, int Y, int Z, double omega, int max_iter, dou
     if (fused) {
       double* dst = src == buf[0] ? buf[1] : buf[0];
       if (pairs && it + 1 <= max_iter) {
-        hipLaunchKernelGGL((k_redblack_multi<mtx, mty, mtz, 2, mthreads>), mgrid, dim3(mthreads), 0,
-                           s, X, Y, Z, omega, src, rhs_d, dst, st);
+        hipLaunchKernelGGL((k_redblack_multi<mtx, mty, 2>), mgrid, dim3(mthreads), 0,
+                           s, X, Y, Z, mzc, omega, src, rhs_d, dst, st);
         it++;
       } else {
         hipLaunchKernelGGL((k_redblack_fused<tx, ty, tz, 256>), fgrid, dim3(256), 0, s, X, Y, Z,
