@@ -113,6 +113,18 @@ __device__ __forceinline__ void iterate_words_body(const unsigned int g, const W
   const int stopped = sload(&sc->converged);
   const double inv = sload(&sc->inv_scale);
   const unsigned long long mx0 = sload(&sc->itmax_bits[0]);
+  const double* __restrict__ pp = q.part + (size_t)((k - 1) & 1) * 3 * m.G;
+  const int i0 = tid < m.G ? tid : 0, i1 = tid + kThreads < m.G ? tid + kThreads : 0;
+  unsigned long long mx = bits64(pp[2 * m.G + i0]), mx1 = bits64(pp[2 * m.G + i1]);
+  double d2 = 0.0, n2 = 0.0, d21 = 0.0, n21 = 0.0;
+  if (tol > 0.0) {
+    d2 = pp[i0];
+    n2 = pp[m.G + i0];
+    d21 = pp[i1];
+    n21 = pp[m.G + i1];
+  }
+  // (before the loads whose places come with the flag: a stopped iteration)
+  if (stopped) return;
   const double* __restrict__ pold = q.pb[(k - 1) & 1];
   double* __restrict__ pnew = q.pb[k & 1];
   const float* __restrict__ din = kInc == 2 ? q.db[(k - 1) & 1] : nullptr;
@@ -128,18 +140,7 @@ __device__ __forceinline__ void iterate_words_body(const unsigned int g, const W
   const Quad dc = reinterpret_cast<const Quad*>(m.dc)[own];
   double sr = 0.0;
   if constexpr (kInc == 2) sr = q.srow[own];
-  const double* __restrict__ pp = q.part + (size_t)((k - 1) & 1) * 3 * m.G;
-  const int i0 = tid < m.G ? tid : 0, i1 = tid + kThreads < m.G ? tid + kThreads : 0;
-  unsigned long long mx = bits64(pp[2 * m.G + i0]), mx1 = bits64(pp[2 * m.G + i1]);
-  double d2 = 0.0, n2 = 0.0, d21 = 0.0, n21 = 0.0;
-  if (tol > 0.0) {
-    d2 = pp[i0];
-    n2 = pp[m.G + i0];
-    d21 = pp[i1];
-    n21 = pp[m.G + i1];
-  }
   s_acc[tid] = 0ull;
-  if (stopped) return;
   if (k > 1) {
     // (the clamped loads repeat group 0: harmless in a max, left out of sums)
     mx = max64(mx, mx1);
