@@ -254,18 +254,18 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
   // entering-run sums per segment, the reverse scan per ray, then the tiles'
   // gather (what 3) or scatter (what 2)
   auto mask_tiles = [&](const double* uu, int what, double* out) -> hipError_t {
-    hipError_t e = launch_adjm_tiles(0, pl.ntiles, pl.tile_ptr1.as<unsigned long long>(),
-                                     pl.segs_slot.as<SegRec>(), nullptr, nullptr, 0, nullptr,
+    hipError_t e = launch_adjm_tiles(0, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
+                                     pl.segs.as<SegRec>(), 0, nullptr,
                                      nullptr, pl.g, pl.tg, wp, uu, mask,
                                      ctx->adj_seg.as<double>(), ctx->adj_span.as<uint8_t>(),
                                      nullptr, st);
     if (e == hipSuccess)
-      e = launch_adjm_tiles(1, pl.ntiles, nullptr, nullptr, nullptr, nullptr, pl.nrays,
+      e = launch_adjm_tiles(1, pl.ntiles, nullptr, nullptr, pl.nrays,
                             pl.nseg.as<unsigned int>(), pl.val_off.as<unsigned long long>(), pl.g,
                             pl.tg, wp, nullptr, nullptr, ctx->adj_seg.as<double>(),
                             ctx->adj_span.as<uint8_t>(), nullptr, st);
     if (e == hipSuccess)
-      e = launch_adjm_tiles(what, pl.ntiles, nullptr, nullptr, pl.tile_ptr.as<unsigned long long>(),
+      e = launch_adjm_tiles(what, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                             pl.segs.as<SegRec>(), 0, nullptr, nullptr, pl.g, pl.tg, wp, uu, mask,
                             ctx->adj_seg.as<double>(), nullptr, out, st);
     return e;
@@ -276,12 +276,12 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
       return launch_adj_gather(mask_rule, pl.rays.as<RayRec>(), pl.nrays, pl.dirs.as<DirConst>(),
                                pl.g, mask, uu, tt, st);
     if (mask_rule) return mask_tiles(uu, 3, tt);
-    hipError_t e = launch_adj_tiles(0, pl.ntiles, pl.tile_ptr1.as<unsigned long long>(),
-                                    pl.segs_slot.as<SegRec>(), nullptr, nullptr, nullptr, 0,
+    hipError_t e = launch_adj_tiles(0, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
+                                    pl.segs.as<SegRec>(), nullptr, 0,
                                     nullptr, nullptr, pl.g, pl.tg, wp, uu,
                                     ctx->adj_seg.as<double>(), nullptr, nullptr, st);
     if (e == hipSuccess)
-      e = launch_adj_tiles(1, pl.ntiles, nullptr, nullptr, nullptr, nullptr, pl.rays.as<RayRec>(),
+      e = launch_adj_tiles(1, pl.ntiles, nullptr, nullptr, pl.rays.as<RayRec>(),
                            pl.nrays, pl.nseg.as<unsigned int>(),
                            pl.val_off.as<unsigned long long>(), pl.g, pl.tg, wp, nullptr,
                            ctx->adj_seg.as<double>(), tt, nullptr, st);
@@ -379,15 +379,15 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
   } else if (tiles) {
     // per-segment sums, per-ray suffix sums, then the tiles' scatter (every
     // voxel of dg stored)
-    OMNI_TRY_HIP(ctx, launch_adj_tiles(0, pl.ntiles, pl.tile_ptr1.as<unsigned long long>(),
-                                       pl.segs_slot.as<SegRec>(), nullptr, nullptr, nullptr, 0,
+    OMNI_TRY_HIP(ctx, launch_adj_tiles(0, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
+                                       pl.segs.as<SegRec>(), nullptr, 0,
                                        nullptr, nullptr, pl.g, pl.tg, wp, u,
                                        ctx->adj_seg.as<double>(), nullptr, nullptr, st));
-    OMNI_TRY_HIP(ctx, launch_adj_tiles(1, pl.ntiles, nullptr, nullptr, nullptr, nullptr,
+    OMNI_TRY_HIP(ctx, launch_adj_tiles(1, pl.ntiles, nullptr, nullptr,
                                        pl.rays.as<RayRec>(), pl.nrays, pl.nseg.as<unsigned int>(),
                                        pl.val_off.as<unsigned long long>(), pl.g, pl.tg, wp,
                                        nullptr, ctx->adj_seg.as<double>(), nullptr, nullptr, st));
-    OMNI_TRY_HIP(ctx, launch_adj_tiles(2, pl.ntiles, nullptr, nullptr,
+    OMNI_TRY_HIP(ctx, launch_adj_tiles(2, pl.ntiles,
                                        pl.tile_ptr.as<unsigned long long>(), pl.segs.as<SegRec>(),
                                        nullptr, 0, nullptr, nullptr, pl.g, pl.tg, wp, u,
                                        ctx->adj_seg.as<double>(), nullptr, dg, st));

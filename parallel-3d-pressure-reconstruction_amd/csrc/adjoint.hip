@@ -495,14 +495,14 @@ hipError_t launch_adj_fixed(int nS, const double* t, DevScalars* sc, long long* 
 
 template <int kBits>
 __global__ void __launch_bounds__(1024)
-k_adj_seg_u(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __restrict__ segs,
+k_adj_seg_u(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
             GridDesc g, TileGrid tg, const double* __restrict__ u, double* __restrict__ useg,
             int parts) {
   constexpr int kTile = 1 << kBits, kTileMask = kTile - 1, kVox = kTile * kTile * kTile;
   __shared__ double U[kVox];
   const TilePart tp = tile_part(xcd_block(), parts);
   const int tile = tp.tile;
-  const unsigned long long b = tile_ptr1[tile], e = tile_ptr1[tile + 1];
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
   if (b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
@@ -650,8 +650,7 @@ k_adj_tile_scatter(const unsigned long long* __restrict__ tile_ptr, const SegRec
   }
 }
 
-hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile_ptr1,
-                            const SegRec* segs_slot, const unsigned long long* tile_ptr,
+hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile_ptr,
                             const SegRec* segs, const RayRec* rays, int64_t nrays,
                             const unsigned int* nseg, const unsigned long long* val_off,
                             GridDesc g, TileGrid tg, const WalkParams& wp, const double* u,
@@ -666,10 +665,10 @@ hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile
   const int parts = tile_parts(ntiles, false);
   if (what == 0) {
     if (tg.bits == 3)
-      hipLaunchKernelGGL(k_adj_seg_u<3>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
+      hipLaunchKernelGGL(k_adj_seg_u<3>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr, segs, g,
                          tg, u, useg, parts);
     else
-      hipLaunchKernelGGL(k_adj_seg_u<4>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
+      hipLaunchKernelGGL(k_adj_seg_u<4>, dim3(ntiles * parts), dim3(1024), 0, st, tile_ptr, segs, g,
                          tg, u, useg, parts);
     return hipGetLastError();
   }
@@ -725,7 +724,7 @@ __device__ __forceinline__ bool adjm_prev_valid(const SegRec& sr, int ox, int oy
 
 template <int kBits>
 __global__ void __launch_bounds__(1024)
-k_adjm_seg_u(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __restrict__ segs,
+k_adjm_seg_u(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
              GridDesc g, TileGrid tg, const double* __restrict__ u,
              const double* __restrict__ mask, double* __restrict__ useg,
              uint8_t* __restrict__ span) {
@@ -744,7 +743,7 @@ k_adjm_seg_u(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __r
     M[lds_slot<kBits>(l)] = in && mask[v] != 0.0 ? 1 : 0;
   }
   __syncthreads();
-  const unsigned long long b = tile_ptr1[tile], e = tile_ptr1[tile + 1];
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
   for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
     const SegRec sr = segs[jj];
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
@@ -888,8 +887,7 @@ k_adjm_tile(const unsigned long long* __restrict__ tile_ptr, const SegRec* __res
   }
 }
 
-hipError_t launch_adjm_tiles(int what, int ntiles, const unsigned long long* tile_ptr1,
-                             const SegRec* segs_slot, const unsigned long long* tile_ptr,
+hipError_t launch_adjm_tiles(int what, int ntiles, const unsigned long long* tile_ptr,
                              const SegRec* segs, int64_t nrays, const unsigned int* nseg,
                              const unsigned long long* val_off, GridDesc g, TileGrid tg,
                              const WalkParams& wp, const double* u, const double* mask,
@@ -903,10 +901,10 @@ hipError_t launch_adjm_tiles(int what, int ntiles, const unsigned long long* til
   }
   if (what == 0) {
     if (tg.bits == 3)
-      hipLaunchKernelGGL(k_adjm_seg_u<3>, dim3(ntiles), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
+      hipLaunchKernelGGL(k_adjm_seg_u<3>, dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g,
                          tg, u, mask, useg, span);
     else
-      hipLaunchKernelGGL(k_adjm_seg_u<4>, dim3(ntiles), dim3(1024), 0, st, tile_ptr1, segs_slot, g,
+      hipLaunchKernelGGL(k_adjm_seg_u<4>, dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g,
                          tg, u, mask, useg, span);
     return hipGetLastError();
   }

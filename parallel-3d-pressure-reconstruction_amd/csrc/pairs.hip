@@ -203,8 +203,8 @@ int boundary_pairs(omni3d_ctx* ctx, int iterations, double* p, int64_t* npairs_o
     // ray the sum of its segments
     OMNI_TRY_HIP(ctx, ctx->segval.alloc(sizeof(T) * pl.nval));
     OMNI_TRY_HIP(ctx, launch_tile_pass<T>(kLocalSum, ctx->tile_threads, pl.ntiles, nullptr,
-                                          pl.tile_ptr1.as<unsigned long long>(),
-                                          pl.segs_slot.as<SegRec>(), pl.g, pl.tg, walk_params(P),
+                                          pl.tile_ptr.as<unsigned long long>(),
+                                          pl.segs.as<SegRec>(), pl.g, pl.tg, walk_params(P),
                                           ctx->field.as<void>(), pl.sid.as<int>(),
                                           pl.cnt.as<unsigned int>(), nullptr, nullptr,
                                           ctx->scal.as<DevScalars>(), ctx->segval.as<T>(),

@@ -195,9 +195,8 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
   const TilePart tp = tile_part(xcd_block(), parts);
   const int tile = tile_list ? tile_list[tp.tile] : tp.tile;
   // kSourceSums walks the compact list of the tile's segments that reach a
-  // source voxel and kLocalSum the tile's segments in value-slot order (one
-  // range per tile: coalesced slot stores); kFull the length groups
-  constexpr int kStride = kMode == kFull ? kLenBuckets : 1;
+  // source voxel (one range per tile), the others the length groups
+  constexpr int kStride = kMode == kSourceSums ? 1 : kLenBuckets;
   const unsigned long long b = tile_ptr[tile * kStride], e = tile_ptr[(tile + 1) * kStride];
   // (parts > 1: the output is cleared before the launch)
   if (parts > 1 && b + (unsigned long long)tp.part * blockDim.x >= e) return;
@@ -400,7 +399,7 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
 // ray is its first segment's first visit).
 template <int kBits>
 __global__ void __launch_bounds__(1024)
-k_tile_counts(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __restrict__ segs,
+k_tile_counts(const unsigned long long* __restrict__ tile_ptr, const SegRec* __restrict__ segs,
               GridDesc g, TileGrid tg, unsigned int* __restrict__ cnt) {
   constexpr int kTile = 1 << kBits, kTileMask = kTile - 1, kVox = kTile * kTile * kTile;
   __shared__ unsigned int C[kVox];
@@ -409,7 +408,7 @@ k_tile_counts(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __
   const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   for (int l = threadIdx.x; l < kVox; l += blockDim.x) C[l] = 0u;
   __syncthreads();
-  const unsigned long long b = tile_ptr1[tile], e = tile_ptr1[tile + 1];
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
   for (unsigned long long jj = b + threadIdx.x; jj < e; jj += blockDim.x) {
     const SegRec sr = segs[jj];
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
@@ -434,13 +433,13 @@ k_tile_counts(const unsigned long long* __restrict__ tile_ptr1, const SegRec* __
   }
 }
 
-hipError_t launch_tile_counts(int ntiles, const unsigned long long* tile_ptr1, const SegRec* segs,
+hipError_t launch_tile_counts(int ntiles, const unsigned long long* tile_ptr, const SegRec* segs,
                               GridDesc g, TileGrid tg, unsigned int* cnt, hipStream_t st) {
   if (tg.bits == 3)
-    hipLaunchKernelGGL(k_tile_counts<3>, dim3(ntiles), dim3(1024), 0, st, tile_ptr1, segs, g, tg,
+    hipLaunchKernelGGL(k_tile_counts<3>, dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g, tg,
                        cnt);
   else
-    hipLaunchKernelGGL(k_tile_counts<4>, dim3(ntiles), dim3(1024), 0, st, tile_ptr1, segs, g, tg,
+    hipLaunchKernelGGL(k_tile_counts<4>, dim3(ntiles), dim3(1024), 0, st, tile_ptr, segs, g, tg,
                        cnt);
   return hipGetLastError();
 }

@@ -126,8 +126,8 @@ hipError_t launch_src_segs(int pass, int nsurf, const int* tile_list,
                            const unsigned long long* tile_ptr, const SegRec* segs, GridDesc g,
                            TileGrid tg, const int* sid, unsigned int* cnt,
                            const unsigned long long* sptr, SegRec* out, hipStream_t st);
-// kSourceSums: tile_ptr / segs are the compact lists, kLocalSum the slot-
-// ordered copy (one range per tile); kFull the length-grouped lists.
+// kSourceSums: tile_ptr / segs are the compact lists; else the length-grouped
+// lists.
 // segval[nval]: per value slot the segment sums (kLocalSum writes them),
 // then the carries (kSourceSums, kFull read them), in the compute precision
 template <typename T>
@@ -228,8 +228,7 @@ hipError_t launch_tile_masked(int method, int ntiles, const unsigned long long* 
 // (what 0: per-segment sums of u over the slot-ordered lists; 1: per-ray
 // suffix sums in place, and each ray's total into tvol at its entry voxel
 // when tvol is given; 2: the scatter of h * S into dg, every voxel stored)
-hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile_ptr1,
-                            const SegRec* segs_slot, const unsigned long long* tile_ptr,
+hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile_ptr,
                             const SegRec* segs, const RayRec* rays, int64_t nrays,
                             const unsigned int* nseg, const unsigned long long* val_off,
                             GridDesc g, TileGrid tg, const WalkParams& wp, const double* u,
@@ -237,8 +236,7 @@ hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile
 // the plain-mask rule's transposed traversals on the tile engine (what 0:
 // entering-run sums and span flags per segment; 1: per-ray reverse scan;
 // 2: scatter into out = dg (3 V); 3: gather of run totals into out (V))
-hipError_t launch_adjm_tiles(int what, int ntiles, const unsigned long long* tile_ptr1,
-                             const SegRec* segs_slot, const unsigned long long* tile_ptr,
+hipError_t launch_adjm_tiles(int what, int ntiles, const unsigned long long* tile_ptr,
                              const SegRec* segs, int64_t nrays, const unsigned int* nseg,
                              const unsigned long long* val_off, GridDesc g, TileGrid tg,
                              const WalkParams& wp, const double* u, const double* mask,
@@ -246,7 +244,7 @@ hipError_t launch_adjm_tiles(int what, int ntiles, const unsigned long long* til
 
 
 // visit counts of every voxel from the tile segments (plan build)
-hipError_t launch_tile_counts(int ntiles, const unsigned long long* tile_ptr1, const SegRec* segs,
+hipError_t launch_tile_counts(int ntiles, const unsigned long long* tile_ptr, const SegRec* segs,
                               GridDesc g, TileGrid tg, unsigned int* cnt, hipStream_t st);
 
 // masked.hip: the masked methods' affine schedule ---------------------------
