@@ -279,12 +279,12 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
     hipError_t e = launch_adj_tiles(0, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                                     pl.segs.as<SegRec>(), nullptr, 0,
                                     nullptr, nullptr, pl.g, pl.tg, wp, uu,
-                                    ctx->adj_seg.as<double>(), nullptr, nullptr, st);
+                                    ctx->adj_seg.as<double>(), nullptr, nullptr, nullptr, st);
     if (e == hipSuccess)
       e = launch_adj_tiles(1, pl.ntiles, nullptr, nullptr, pl.rays.as<RayRec>(),
                            pl.nrays, pl.nseg.as<unsigned int>(),
                            pl.val_off.as<unsigned long long>(), pl.g, pl.tg, wp, nullptr,
-                           ctx->adj_seg.as<double>(), tt, nullptr, st);
+                           ctx->adj_seg.as<double>(), nullptr, tt, nullptr, st);
     return e;
   };
   // z = sum_{j<K} (A^T)^j y
@@ -379,18 +379,21 @@ int omni3d_backward(omni3d_ctx* ctx, const void* dldp_d, void* dldgrad_d) {
   } else if (tiles) {
     // per-segment sums, per-ray suffix sums, then the tiles' scatter (every
     // voxel of dg stored)
+    OMNI_TRY_HIP(ctx, ctx->adj_after.alloc(sizeof(double) * std::max<int64_t>(pl.nval, 1)));
     OMNI_TRY_HIP(ctx, launch_adj_tiles(0, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                                        pl.segs.as<SegRec>(), nullptr, 0,
                                        nullptr, nullptr, pl.g, pl.tg, wp, u,
-                                       ctx->adj_seg.as<double>(), nullptr, nullptr, st));
+                                       ctx->adj_seg.as<double>(), nullptr, nullptr, nullptr, st));
     OMNI_TRY_HIP(ctx, launch_adj_tiles(1, pl.ntiles, nullptr, nullptr,
                                        pl.rays.as<RayRec>(), pl.nrays, pl.nseg.as<unsigned int>(),
                                        pl.val_off.as<unsigned long long>(), pl.g, pl.tg, wp,
-                                       nullptr, ctx->adj_seg.as<double>(), nullptr, nullptr, st));
+                                       nullptr, ctx->adj_seg.as<double>(),
+                                       ctx->adj_after.as<double>(), nullptr, nullptr, st));
     OMNI_TRY_HIP(ctx, launch_adj_tiles(2, pl.ntiles,
                                        pl.tile_ptr.as<unsigned long long>(), pl.segs.as<SegRec>(),
                                        nullptr, 0, nullptr, nullptr, pl.g, pl.tg, wp, u,
-                                       ctx->adj_seg.as<double>(), nullptr, dg, st));
+                                       ctx->adj_seg.as<double>(), ctx->adj_after.as<double>(),
+                                       nullptr, dg, st));
   } else {
     OMNI_TRY_HIP(ctx, launch_fill_f64(dg, 3 * V, 0.0, st));
     OMNI_TRY_HIP(ctx, launch_adj_scatter(mask_rule, pl.rays.as<RayRec>(), pl.nrays,

@@ -9,9 +9,9 @@
 // "carry") comes from a first pass of per-segment sums and a per-ray scan.
 //
 //   plan:   k_tile_count -> scans -> k_tile_fill            (once per grid)
-//   solve:  k_tile_pass<kLocalSum> -> k_carry_scan ->
-//           k_tile_pass<kSourceSums> (surface tiles) -> source iteration ->
-//           k_tile_pass<kFull> -> averaging
+//   solve:  k_tile_walk<kLocalSum> -> k_carry_scan ->
+//           k_tile_sources (surface tiles) -> source iteration ->
+//           k_tile_walk<kFull> -> averaging
 #include <hip/hip_runtime.h>
 
 #include <hipcub/hipcub.hpp>
@@ -149,125 +149,67 @@ k_tile_fill(const RayRec* __restrict__ rays, int64_t nrays, const DirConst* __re
 // ---------------------------------------------------------------------------
 // Tile passes.
 
-// LDS of a tile pass: the tile's gradient; the fixed-point counters (full
-// and source-sum passes); the source ids of the tile's voxels (source-sum
-// pass).  Exact sizes matter: two FP32 16^3 full-pass workgroups fill the
-// 160 KB of a CU.
-// The segment-sum pass keeps a one-voxel halo ((edge + 2)^3 voxels, x
-// fastest) instead: the step into the tile then reads the voxel outside it
-// from LDS.
-template <typename T, int kVox, int kHaloVox, int kMode>
-struct TileLds {
-  T g[3][kVox];
-  long long acc[kVox];
-};
-template <typename T, int kVox, int kHaloVox>
-struct TileLds<T, kVox, kHaloVox, kLocalSum> {
-  T g[3][kHaloVox];
-};
-template <typename T, int kVox, int kHaloVox>
-struct TileLds<T, kVox, kHaloVox, kSourceSums> {
-  T g[3][kVox];
-  long long acc[kVox];
-  int sidl[kVox];
-};
-
-template <typename T, int kMode, int kBits, int kThreads>
+// The source-sum pass (kSourceSums): the visits that land on source voxels,
+// walked from the compact lists of the surface tiles' segments that reach one.
+// LDS: the tile's gradient, the fixed-point sums, the voxels' source ids.
+template <typename T, int kBits, int kThreads>
 __global__ void __launch_bounds__(kThreads)
-k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restrict__ tile_ptr,
-            const SegRec* __restrict__ segs, GridDesc g, TileGrid tg, WalkParams wp,
-            const typename Vec4<T>::type* __restrict__ field, const int* __restrict__ sid,
-            const unsigned int* __restrict__ vcnt,
-            const double* __restrict__ pbuf0, const double* __restrict__ pbuf1,
-            const DevScalars* __restrict__ sc, T* __restrict__ segval,
-            long long* __restrict__ out, int parts) {
+k_tile_sources(const int* __restrict__ tile_list, const unsigned long long* __restrict__ tile_ptr,
+               const SegRec* __restrict__ segs, GridDesc g, TileGrid tg, WalkParams wp,
+               const typename Vec4<T>::type* __restrict__ field, const int* __restrict__ sid,
+               const DevScalars* __restrict__ sc, const T* __restrict__ segval,
+               long long* __restrict__ out, int parts) {
   using V4 = typename Vec4<T>::type;
-  constexpr int kTileBits = kBits;
   constexpr int kTile = 1 << kBits;
   constexpr int kTileMask = kTile - 1;
   constexpr int kTileVox = kTile * kTile * kTile;
-  constexpr bool kHalo = kMode == kLocalSum;
-  constexpr int kW = kTile + 2;  // halo edge
-  constexpr int kHaloVox = kW * kW * kW;
-  constexpr int kPlane = kHalo ? kHaloVox : kTileVox;
-  __shared__ TileLds<T, kTileVox, kHaloVox, kMode> L;
+  __shared__ T s_g[3][kTileVox];
+  __shared__ unsigned long long s_acc[kTileVox];
+  __shared__ int s_sid[kTileVox];
   // contiguous tile ranges per XCD: neighbouring tiles share an L2
   const TilePart tp = tile_part(xcd_block(), parts);
   const int tile = tile_list ? tile_list[tp.tile] : tp.tile;
-  // kSourceSums walks the compact list of the tile's segments that reach a
-  // source voxel (one range per tile), the others the length groups
-  constexpr int kStride = kMode == kSourceSums ? 1 : kLenBuckets;
-  const unsigned long long b = tile_ptr[tile * kStride], e = tile_ptr[(tile + 1) * kStride];
+  const unsigned long long b = tile_ptr[tile], e = tile_ptr[tile + 1];
   // (parts > 1: the output is cleared before the launch)
   if (parts > 1 && b + (unsigned long long)tp.part * blockDim.x >= e) return;
   const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
-  const int ox = tx << kTileBits, oy = ty << kTileBits, oz = tz << kTileBits;
+  const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
   const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
-  // stage the tile's gradient (zero outside the grid) and clear the counters
-  if constexpr (kHalo) {
-    for (int l = threadIdx.x; l < kHaloVox; l += blockDim.x) {
-      const int i = ox + l % kW - 1, j = oy + (l / kW) % kW - 1, k = oz + l / (kW * kW) - 1;
-      V4 v;
-      const bool in = i >= 0 && j >= 0 && k >= 0 && i < g.X && j < g.Y && k < g.Z;
-      if (in) v = field[i + j * sy + k * sz];
-      else v.x = v.y = v.z = v.w = 0;
-      L.g[0][l] = v.x;
-      L.g[1][l] = v.y;
-      L.g[2][l] = v.z;
-    }
-  }
-  for (int l = threadIdx.x; l < (kHalo ? 0 : kTileVox); l += blockDim.x) {
-    const int i = ox + (l & kTileMask), j = oy + ((l >> kTileBits) & kTileMask),
-              k = oz + (l >> (2 * kTileBits));
+  for (int l = threadIdx.x; l < kTileVox; l += blockDim.x) {
+    const int i = ox + (l & kTileMask), j = oy + ((l >> kBits) & kTileMask),
+              k = oz + (l >> (2 * kBits));
     V4 v;
     const bool in = i < g.X && j < g.Y && k < g.Z;
     if (in) v = field[i + j * sy + k * sz];
     else v.x = v.y = v.z = v.w = 0;
-    if constexpr (!kHalo) {
-      const int sl = lds_slot<kBits>(l);
-      L.g[0][sl] = v.x;
-      L.g[1][sl] = v.y;
-      L.g[2][sl] = v.z;
-      L.acc[sl] = 0;
-      // source voxels (all on the box surface) by their compact id
-      if constexpr (kMode == kSourceSums) L.sidl[sl] = in ? sid[i + j * sy + k * sz] : -1;
-    }
+    const int sl = lds_slot<kBits>(l);
+    s_g[0][sl] = v.x;
+    s_g[1][sl] = v.y;
+    s_g[2][sl] = v.z;
+    s_acc[sl] = 0ull;
+    // source voxels (all on the box surface) by their compact id
+    s_sid[sl] = in ? sid[i + j * sy + k * sz] : -1;
   }
   __syncthreads();
   const double scale = sc->scale;
-  const double* __restrict__ ps = ((sc->kstar - 1) & 1) ? pbuf1 : pbuf0;
-  // software pipeline over a thread's segments: the record two segments
-  // ahead and the values the next segment starts from (its carry, entry
-  // term and source pressure) are in flight while this segment is walked
-  struct Pre {
-    double pin = 0.0, cv = 0.0;
-  };
+  // the record two segments ahead and the carry of the next are in flight
+  // while this segment is walked
   const unsigned int bd = blockDim.x * (unsigned int)parts;
-  auto fetch = [&](const SegRec& r, unsigned long long jj) {
-    Pre q;
-    const bool fs = (r.info >> 21) & 1u;
-    if constexpr (kMode == kFull) q.pin = ps[r.src];
-    if constexpr (kMode != kLocalSum) {
-      if (!fs) q.cv = (double)segval[r.g];
-    }
-    (void)jj;
-    return q;
+  auto fetch = [&](const SegRec& r) {
+    return (r.info >> 21) & 1u ? 0.0 : (double)segval[r.g];
   };
   unsigned long long j = part_begin(b, tp);
   SegRec r1, r2;
-  Pre p1;
+  double p1 = 0.0;
   if (j < e) r1 = segs[j];
   if (j + bd < e) r2 = segs[j + bd];
-  if (j < e) p1 = fetch(r1, j);
+  if (j < e) p1 = fetch(r1);
   for (; j < e; j += bd) {
     const SegRec sr = r1;
-    const Pre pr = p1;
+    const double cv = p1;
     r1 = r2;
     if (j + 2ull * bd < e) r2 = segs[j + 2ull * bd];
-    if (j + bd < e) p1 = fetch(r1, j + bd);
-    // carry: the ray's sum before this segment plus the step into the tile
-    // (kLocalSum computes that step, the only read outside the tile, and
-    // stores it per segment in tile order)
+    if (j + bd < e) p1 = fetch(r1);
     int lv = (int)(sr.info & ((1u << kSegLvBits) - 1u));
     const unsigned int n = (sr.info >> kSegLvBits) & 63u;
     const unsigned int sg = (sr.info >> 18) & 7u;
@@ -275,121 +217,231 @@ k_tile_pass(const int* __restrict__ tile_list, const unsigned long long* __restr
     // the segment's step signs are fixed: per axis, the LDS step and the
     // trapezoid factor of a step along it
     const bool up0 = sg & 1u, up1 = (sg >> 1) & 1u, up2 = (sg >> 2) & 1u;
-    constexpr int kSy = kHalo ? kW : kTile;  // LDS strides of the walked index
     const int d0 = up0 ? 1 : -1;
-    const int d1 = up1 ? kSy : -kSy;
-    const int d2 = up2 ? kSy * kSy : -kSy * kSy;
-    // the walked index: the halo index (kLocalSum) or the in-tile index,
-    // whose LDS slot is swizzled
-    if constexpr (kHalo)
-      lv = (lv & kTileMask) + 1 + (((lv >> kTileBits) & kTileMask) + 1) * kW +
-           ((lv >> (2 * kTileBits)) + 1) * kW * kW;
-    auto slot = [&](int l) {
-      if constexpr (kHalo) return l;
-      else return lds_slot<kBits>(l);
-    };
+    const int d1 = up1 ? kTile : -kTile;
+    const int d2 = up2 ? kTile * kTile : -kTile * kTile;
     const T h0 = step_factor<T>(wp, 0, up0);
     const T h1 = step_factor<T>(wp, 1, up1);
     const T h2 = step_factor<T>(wp, 2, up2);
-    // in-tile sums accumulate in FP64: kLocalSum the segment's sum; the
-    // other passes (base + sum so far) * scale + 1.5 * 2^52, whose low
-    // mantissa bits are the 64-bit fixed-point value (|value| < 2^51, the
-    // scale is a power of two: each step adds its term rounded to a unit)
-    double loc = 0.0, accs = 6755399441055744.0;
-    auto add_fixed = [&](int l) {
-      if constexpr (kMode == kFull) {
-        // the biased bits; the flush removes visits x the bias
-        atomicAdd(reinterpret_cast<unsigned long long*>(&L.acc[l]),
-                  (unsigned long long)__double_as_longlong(accs));
-      } else if constexpr (kMode == kSourceSums) {
-        const long long f = __double_as_longlong(accs) - 0x4338000000000000LL;
-        atomicAdd(reinterpret_cast<unsigned long long*>(&L.acc[l]), (unsigned long long)f);
-      }
-    };
-    auto on_source = [&](int l) {
-      if constexpr (kMode == kSourceSums) return L.sidl[l] >= 0;
-      else return false;
+    // sum so far * scale + 1.5 * 2^52, whose low mantissa bits are the 64-bit
+    // fixed-point value (|value| < 2^51, the scale is a power of two: each
+    // step adds its term rounded to a unit)
+    double accs = 6755399441055744.0;
+    auto visit = [&](int sl) {
+      if (s_sid[sl] >= 0)
+        atomicAdd(&s_acc[sl], (unsigned long long)(__double_as_longlong(accs) - 0x4338000000000000LL));
     };
     uint32_t cw = sr.code[0];
-    int inw = 16;  // codes left in the current word
-    if (first) {
-      // the entry visit: self-add p_src (pint = 0)
-      if constexpr (kMode == kFull) {
-        accs = pr.pin * scale + 6755399441055744.0;
-        add_fixed(slot(lv));
-      }
-    } else if constexpr (kMode != kLocalSum) {
+    int slv = lds_slot<kBits>(lv);
+    if (!first) {
       // the carry already holds the step into the tile (it ends the previous
       // segment's sum)
-      accs = (kMode == kFull ? pr.pin + pr.cv : pr.cv) * scale + 6755399441055744.0;
-      const int slv = slot(lv);
-      if (kMode == kFull || on_source(slv)) add_fixed(slv);
+      accs = cv * scale + 6755399441055744.0;
+      visit(slv);
     }
-    // every later visit adds base + (in-tile sum so far)
     int rem = (int)n - 1;
-    int slv = slot(lv);
 #pragma unroll 1
     for (int wi = 0; wi < 3 && rem > 0; wi++) {
-      const int m = rem < inw ? rem : inw;
+      const int m = rem < 16 ? rem : 16;
       for (int q = 0; q < m; q++) {
         const int a = (int)(cw & 3u);
         cw >>= 2;
         const bool a0 = a == 0, a1 = a == 1;
         const int ln = lv + (a0 ? d0 : (a1 ? d1 : d2));
         const T h = a0 ? h0 : (a1 ? h1 : h2);
-        const T* __restrict__ gp = &L.g[0][0] + a * kPlane;
-        const int sln = slot(ln);
+        const T* __restrict__ gp = &s_g[0][0] + a * kTileVox;
+        const int sln = lds_slot<kBits>(ln);
         const T t = h * (gp[sln] + gp[slv]);
         lv = ln;
         slv = sln;
-        if constexpr (kMode == kLocalSum) {
-          loc += (double)t;
-        } else {
-          accs = fma((double)t, scale, accs);
-          if (kMode == kFull || on_source(slv)) add_fixed(slv);
-        }
+        accs = fma((double)t, scale, accs);
+        visit(slv);
       }
       rem -= m;
       cw = wi == 0 ? sr.code[1] : sr.code[2];
-      inw = 16;
-    }
-    if constexpr (kMode == kLocalSum) {
-      if (!((sr.info >> 22) & 1u)) {
-        // the step out of the tile (the next voxel lies in the halo) ends
-        // the segment: its code follows the n - 1 in-tile codes
-        const unsigned int q = n - 1;
-        const uint32_t wq = q < 16 ? sr.code[0] : (q < 32 ? sr.code[1] : sr.code[2]);
-        const int a = (int)((wq >> (2 * (q & 15))) & 3u);
-        const int sgn = ((sg >> a) & 1u) ? 1 : -1;
-        const int dn = a == 0 ? d0 : (a == 1 ? d1 : d2);
-        loc += (double)trapezoid<T>(wp, a, sgn, L.g[a][lv + dn], L.g[a][lv]);
-      }
-      segval[sr.g] = (T)loc;
     }
   }
-  if (kMode == kLocalSum) return;
   __syncthreads();
   for (int l = threadIdx.x; l < kTileVox; l += blockDim.x) {
-    const int i = ox + (l & kTileMask), j = oy + ((l >> kTileBits) & kTileMask),
-              k = oz + (l >> (2 * kTileBits));
-    if (i >= g.X || j >= g.Y || k >= g.Z) continue;
-    const int64_t v = i + j * sy + k * sz;
     const int sl = lds_slot<kBits>(l);
-    // (every visit of v is walked by this tile: cnt[v] biased adds)
-    // several parts: their biased sums add up in memory (modulo 2^64, in any
-    // order), the first one takes the bias of all of the voxel's visits off
-    if constexpr (kMode == kFull) {
-      unsigned long long x = (unsigned long long)L.acc[sl];
-      if (tp.part == 0) x -= (unsigned long long)vcnt[v] * 0x4338000000000000ull;
-      if (parts == 1) out[v] = (long long)x;
-      else if (x) atomicAdd(reinterpret_cast<unsigned long long*>(&out[v]), x);
+    const int s = s_sid[sl];
+    if (s >= 0) {
+      if (parts == 1) out[s] = (long long)s_acc[sl];
+      else fx_add(&out[s], (long long)s_acc[sl]);
     }
-    if constexpr (kMode == kSourceSums) {
-      const int s = L.sidl[sl];
-      if (s >= 0) {
-        if (parts == 1) out[s] = L.acc[sl];
-        else fx_add(&out[s], L.acc[sl]);
+  }
+}
+
+// The walks of the segment sums (kLocalSum) and of the full pass (kFull).
+//
+// What bounded them were the vector instructions of a step (82 and 93 % of the
+// time at 256^3 FP32, a step being 23 and 26 of them): the axis code's
+// selects of step, factor and plane, two gradient reads with a swizzled
+// address each, the term.  Here a step is 10:
+//   - the term of an edge, factor x (sum of the gradients at its two ends), is
+//     in LDS per axis, computed once per tile instead of once per visit; a step
+//     down the axis is the same term negated, to the bit, so the sign goes
+//     into the term's multiplier;
+//   - positions are 16-bit offsets; the step and the edge's place relative to
+//     the position come from two registers per quantity, the half-word of the
+//     axis picked by one byte permute;
+//   - rows and slabs are padded instead of swizzled.
+// What is left is LDS for the full pass (an 8-byte add and a 4-byte read a
+// step, 17 cycles with their conflicts) and the slots' stores for the segment
+// sums.  us per launch before / now, FP32: 128^3 sums 336 / 284, full 471 / 413;
+// 256^3 3415 / 3450, 3406 / 3385 (two workgroups shared a CU, one does now).
+// kLocalSum has the edges into and out of the tile too: cell 0 of an axis is
+// the voxel before the tile.
+template <typename T, int kMode, int kBits, int kThreads>
+__global__ void __launch_bounds__(kThreads)
+k_tile_walk(const int* __restrict__ tile_list, const unsigned long long* __restrict__ tile_ptr,
+            const SegRec* __restrict__ segs, GridDesc g, TileGrid tg, WalkParams wp,
+            const typename Vec4<T>::type* __restrict__ field,
+            const unsigned int* __restrict__ vcnt,
+            const double* __restrict__ pbuf0, const double* __restrict__ pbuf1,
+            const DevScalars* __restrict__ sc, T* __restrict__ segval,
+            long long* __restrict__ out, int parts) {
+  static_assert(kMode == kLocalSum || kMode == kFull, "the walks over all visits");
+  using U16 = unsigned short;
+  constexpr int kTile = 1 << kBits, kMask = kTile - 1, kTileVox = kTile * kTile * kTile;
+  constexpr int kOff = kMode == kLocalSum ? 1 : 0;
+  // (rows and slabs so that positions spread over the banks: the full pass at
+  // 128^3 FP32 took 413 us with slabs of 281 or 292 cells of rows of 17, 430 with
+  // 289, 477 with rows of 16 in 260, 696 with 16 in 256)
+  constexpr int kRow = kTile + 1, kSlab = kRow * kTile + (kOff ? kRow : 9);
+  constexpr int kCells = kSlab * (kTile + kOff);
+  // offsets in bytes of an FP32 plane, or in entries (FP64 planes exceed 16 bits)
+  constexpr int kU = sizeof(T) == 4 ? 4 : 1;
+  static_assert(3 * kCells * kU < 65536, "16-bit offsets");
+  __shared__ T s_e[3 * kCells];
+  __shared__ unsigned long long s_acc[kMode == kFull ? kCells : 1];
+  __shared__ uint4 s_dir[8];  // per sign octant: the steps, the edges' places
+  const TilePart tp = tile_part(xcd_block(), parts);
+  const int tile = tile_list ? tile_list[tp.tile] : tp.tile;
+  const unsigned long long b = tile_ptr[tile * kLenBuckets], e = tile_ptr[(tile + 1) * kLenBuckets];
+  // (parts > 1: the output is cleared before the launch)
+  if (parts > 1 && b + (unsigned long long)tp.part * blockDim.x >= e) return;
+  const int tx = tile % tg.ntx, ty = (tile / tg.ntx) % tg.nty, tz = tile / (tg.ntx * tg.nty);
+  const int ox = tx << kBits, oy = ty << kBits, oz = tz << kBits;
+  const int64_t sy = g.X, sz = (int64_t)g.X * g.Y;
+  const T* __restrict__ comp = reinterpret_cast<const T*>(field);
+  const T up[3] = {step_factor<T>(wp, 0, true), step_factor<T>(wp, 1, true),
+                   step_factor<T>(wp, 2, true)};
+  for (int l = threadIdx.x; l < kCells; l += kThreads) {
+    const int i = ox + (l % kSlab) % kRow - kOff, j = oy + (l % kSlab) / kRow - kOff,
+              k = oz + l / kSlab - kOff;
+    const bool in = i >= 0 && j >= 0 && k >= 0 && i < g.X && j < g.Y && k < g.Z;
+    const bool nx = in && i + 1 < g.X, ny = in && j + 1 < g.Y, nz = in && k + 1 < g.Z;
+    // (loads at clamped places, not under branches; edges out of the grid are
+    // no step's)
+    const int64_t v = in ? i + j * sy + k * sz : 0;
+    const T a0 = comp[4 * v], b0 = comp[4 * (nx ? v + 1 : v)];
+    const T a1 = comp[4 * v + 1], b1 = comp[4 * (ny ? v + sy : v) + 1];
+    const T a2 = comp[4 * v + 2], b2 = comp[4 * (nz ? v + sz : v) + 2];
+    s_e[l] = up[0] * (b0 + a0);
+    s_e[kCells + l] = up[1] * (b1 + a1);
+    s_e[2 * kCells + l] = up[2] * (b2 + a2);
+    if constexpr (kMode == kFull) s_acc[l] = 0ull;
+  }
+  if (threadIdx.x < 8) s_dir[threadIdx.x] = walk_tables<kRow, kSlab, kU>(threadIdx.x, kCells);
+  __syncthreads();
+  const double scale = sc->scale;
+  const double* __restrict__ ps = ((sc->kstar - 1) & 1) ? pbuf1 : pbuf0;
+  // a term's multiplier: the fixed-point scale (a power of two: the product
+  // is exact, each step adds its term rounded to a unit), or one
+  const unsigned long long mul =
+      (unsigned long long)__double_as_longlong(kMode == kFull ? scale : 1.0);
+  const unsigned int mul_lo = (unsigned int)mul, mul_hi = (unsigned int)(mul >> 32);
+  // the record two segments ahead and the values the next one starts from
+  // are in flight while this one is walked
+  struct Pre {
+    double pin = 0.0, cv = 0.0;
+  };
+  auto fetch = [&](const SegRec& r) {
+    Pre q;
+    if constexpr (kMode == kFull) {
+      q.pin = ps[r.src];
+      if (!((r.info >> 21) & 1u)) q.cv = (double)segval[r.g];
+    }
+    return q;
+  };
+  const unsigned int bd = blockDim.x * (unsigned int)parts;
+  unsigned long long jj = part_begin(b, tp);
+  SegRec r1, r2;
+  Pre p1;
+  if (jj < e) r1 = segs[jj];
+  if (jj + bd < e) r2 = segs[jj + bd];
+  if (jj < e) p1 = fetch(r1);
+  for (; jj < e; jj += bd) {
+    const SegRec sr = r1;
+    const Pre pr = p1;
+    r1 = r2;
+    if (jj + 2ull * bd < e) r2 = segs[jj + 2ull * bd];
+    if (jj + bd < e) p1 = fetch(r1);
+    const unsigned int lv = sr.info & ((1u << kSegLvBits) - 1u);
+    const unsigned int n = (sr.info >> kSegLvBits) & 63u;
+    const unsigned int sg = (sr.info >> 18) & 7u;
+    const uint4 dir = s_dir[sg];
+    const unsigned int down = __brev(~sg & 7u);  // the sign of axis a at bit 31 - a
+    U16 at = (U16)(((lv & kMask) + kOff + (((lv >> kBits) & kMask) + kOff) * kRow +
+                    ((lv >> (2 * kBits)) + kOff) * kSlab) * kU);
+    // kFull: base + sum so far in units of the scale + 1.5 * 2^52, whose low
+    // mantissa bits are the fixed-point value (the flush takes visits x the
+    // bias off); else the segment's sum
+    double acc = 0.0;
+    auto visit = [&]() {
+      if constexpr (kMode == kFull)
+        atomicAdd(reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(s_acc) +
+                                                        (unsigned int)at * (8 / kU)),
+                  (unsigned long long)__double_as_longlong(acc));
+    };
+    if constexpr (kMode == kFull) {
+      // the entry visit adds p_src; a later segment's carry already holds the
+      // step into the tile
+      const bool first = (sr.info >> 21) & 1u;
+      acc = (first ? pr.pin : pr.pin + pr.cv) * scale + 6755399441055744.0;
+      visit();
+    }
+    auto step = [&](unsigned int a) {
+      const U16 edge = (U16)(at + walk_pick(dir.z, dir.w, a));
+      at = (U16)(at + walk_pick(dir.x, dir.y, a));
+      const T t = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(s_e) +
+                                              (unsigned int)edge * (sizeof(T) / kU));
+      const unsigned int hi = (mul_hi & 0x7fffffffu) | ((down << a) & 0x80000000u);
+      acc = __builtin_fma((double)t, __hiloint2double((int)hi, (int)mul_lo), acc);
+      visit();
+    };
+    // kLocalSum: the step out of the tile ends the segment
+    int rem = (int)n - 1;
+    if (kMode == kLocalSum && !((sr.info >> 22) & 1u)) rem++;
+    uint32_t cw = sr.code[0];
+#pragma unroll 1
+    for (int wi = 0; wi < 3 && rem > 0; wi++) {
+      int m = rem < 16 ? rem : 16;
+      rem -= m;
+      for (; m >= 4; m -= 4, cw >>= 8) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) step((cw >> (2 * u)) & 3u);
       }
+      for (; m > 0; m--, cw >>= 2) step(cw & 3u);
+      cw = wi == 0 ? sr.code[1] : sr.code[2];
+    }
+    if constexpr (kMode == kLocalSum) segval[sr.g] = (T)acc;
+  }
+  if constexpr (kMode == kFull) {
+    __syncthreads();
+    for (int l = threadIdx.x; l < kTileVox; l += kThreads) {
+      const int x = l & kMask, y = (l >> kBits) & kMask, z = l >> (2 * kBits);
+      const int i = ox + x, j = oy + y, k = oz + z;
+      if (i >= g.X || j >= g.Y || k >= g.Z) continue;
+      const int64_t v = i + j * sy + k * sz;
+      // (every visit of v is walked by this tile: cnt[v] biased adds; several
+      // parts: their biased sums add up in memory (modulo 2^64, in any
+      // order), the first one takes the bias of all of the voxel's visits off)
+      unsigned long long t = s_acc[x + y * kRow + z * kSlab];
+      if (tp.part == 0) t -= (unsigned long long)vcnt[v] * 0x4338000000000000ull;
+      if (parts == 1) out[v] = (long long)t;
+      else if (t) atomicAdd(reinterpret_cast<unsigned long long*>(&out[v]), t);
     }
   }
 }
@@ -887,9 +939,15 @@ static void tile_pass_threads(int threads, int ntiles, const int* tile_list,
                               long long* out, hipStream_t st) {
   const int parts = tile_parts(ntiles, false);
 #define OMNI_TILE(NT)                                                                        \
-  hipLaunchKernelGGL((k_tile_pass<T, kMode, kBits, NT>), dim3(ntiles * parts), dim3(NT), 0, st, \
-                     tile_list, tile_ptr, segs, g, tg, wp, f, sid, vcnt, p0, p1, sc, segval,    \
-                     out, parts)
+  do {                                                                                       \
+    if constexpr (kMode == kSourceSums)                                                      \
+      hipLaunchKernelGGL((k_tile_sources<T, kBits, NT>), dim3(ntiles * parts), dim3(NT), 0, st, \
+                         tile_list, tile_ptr, segs, g, tg, wp, f, sid, sc, segval, out, parts); \
+    else                                                                                     \
+      hipLaunchKernelGGL((k_tile_walk<T, kMode, kBits, NT>), dim3(ntiles * parts), dim3(NT), 0, \
+                         st, tile_list, tile_ptr, segs, g, tg, wp, f, vcnt, p0, p1, sc, segval, \
+                         out, parts);                                                        \
+  } while (0)
   if (threads <= 256) OMNI_TILE(256);
   else if (threads <= 512) OMNI_TILE(512);
   else OMNI_TILE(1024);

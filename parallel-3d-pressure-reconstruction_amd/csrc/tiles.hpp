@@ -75,6 +75,29 @@ __device__ __forceinline__ double step_factor<double>(const WalkParams& wp, int 
   return up ? wp.hs[a][1] : wp.hs[a][0];
 }
 
+// A walk's tables over a tile whose rows are kRow cells and whose slabs are
+// kSlab (positions and places in units of kU, 16 bits): for a segment of
+// step signs sg (bit a: up axis a) the step along each axis (x, y: half-words
+// of x and y components) and where the edge it takes lies from the position it
+// starts at, an edge being kept at its lower end, axis a's in plane a of
+// `plane` cells.
+template <int kRow, int kSlab, int kU>
+__device__ __forceinline__ uint4 walk_tables(unsigned int sg, int plane) {
+  const int d[3] = {kU, kRow * kU, kSlab * kU};
+  unsigned int m[3], p[3];
+  for (int a = 0; a < 3; a++) {
+    const bool u = (sg >> a) & 1u;
+    m[a] = (unsigned int)(u ? d[a] : -d[a]) & 0xffffu;
+    p[a] = (unsigned int)(a * plane * kU - (u ? 0 : d[a])) & 0xffffu;
+  }
+  return uint4{m[0] | (m[1] << 16), m[2], p[0] | (p[1] << 16), p[2]};
+}
+// the half-word of axis a of (lo, hi)
+__device__ __forceinline__ unsigned short walk_pick(unsigned int lo, unsigned int hi,
+                                                    unsigned int a) {
+  return (unsigned short)__builtin_amdgcn_perm(hi, lo, a * 0x0202u + 0x0100u);
+}
+
 // One segment: the visits of one ray inside one tile, self-contained so that
 // a tile pass starts it with one coalesced load.  A monotone staircase visits
 // at most 16+15+15 = 46 voxels of a 16^3 tile, so its step codes fit in 96 bits.
@@ -225,14 +248,13 @@ hipError_t launch_tile_masked(int method, int ntiles, const unsigned long long* 
 
 
 // adjoint.hip: the plain method's transposed traversals on the tile engine
-// (what 0: per-segment sums of u over the slot-ordered lists; 1: per-ray
-// suffix sums in place, and each ray's total into tvol at its entry voxel
-// when tvol is given; 2: the scatter of h * S into dg, every voxel stored)
+// (what 0: per-segment sums of u; 1: per-ray sums of the later segments into
+// tafter, and each ray's total into tvol at its entry voxel, where given; 2: the scatter of h * S into dg, every voxel stored)
 hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile_ptr,
                             const SegRec* segs, const RayRec* rays, int64_t nrays,
                             const unsigned int* nseg, const unsigned long long* val_off,
                             GridDesc g, TileGrid tg, const WalkParams& wp, const double* u,
-                            double* useg, double* tvol, double* dg, hipStream_t st);
+                            double* useg, double* tafter, double* tvol, double* dg, hipStream_t st);
 // the plain-mask rule's transposed traversals on the tile engine (what 0:
 // entering-run sums and span flags per segment; 1: per-ray reverse scan;
 // 2: scatter into out = dg (3 V); 3: gather of run totals into out (V))
