@@ -388,7 +388,7 @@ def sor_measure(args):
         "data": "synthetic",
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": traffic, "kernel": "k_redblack_multi<64, 16, 64, 2, 1024> (two red-black iterations per pass)",
+                     "traffic": traffic, "kernel": "k_redblack_multi<64, 16, 2> (two red-black iterations per pass)",
                      "algorithmic_bytes": bytes_it},
         "cpu_baseline": cpu, "gpu_sor3D_dropin": jacobi_gpu,
         "config": {"workload": f"Neumann right-hand side of the burgers-vortex {n}^3 field, "
@@ -688,8 +688,8 @@ def main():
             f"{tri['rel_l2_vs_analytic_demeaned']:.3e} (staircase {err_analytic:.3e})")
 
     # roofline of the dominant traversal kernel: the slower of the segment-sum
-    # traversal of pass A (k_tile_pass, local-sum mode) and the final full
-    # traversal (k_tile_pass, full mode), each one ray pass.  A ray pass must
+    # traversal of pass A (k_tile_walk, local-sum mode) and the final full
+    # traversal (k_tile_walk, full mode), each one ray pass.  A ray pass must
     # stream the gradient once per direction, D*V*3*4 B in FP32, and read and
     # write the FP64 pressure and FP32 weight once, V*20 B.  The kernels'
     # durations are the library's HIP events around them on its stream.
@@ -701,21 +701,20 @@ def main():
         t = json.load(open(TRAFFIC_FILE))
         if t.get("workload_n") == n and t.get("directions") == D:
             traffic = t.get("traffic_bytes", {})
-    kern = {"local_sum": ("k_tile_pass<float, local-sum, 16^3 tiles + halo, 1024 threads> "
+    kern = {"local_sum": ("k_tile_walk<float, local-sum, 16^3 tiles + halo, 1024 threads> "
                           "(segment sums of pass A)", ms_s),
-            "full": ("k_tile_pass<float, full, 16^3 tiles, 1024 threads> (final traversal)", ms_b)}
+            "full": ("k_tile_walk<float, full, 16^3 tiles, 1024 threads> (final traversal)", ms_b)}
     # the source iteration is the dominant kernel by time (200 launches, half
     # of a reconstruction): one launch must read the iteration matrix once,
     # 4 B per word (equal entries of a row merged), and per source row its
-    # vectors: row sum, p_S, constant, diagonal, source index and visit count
-    # read, row sum, p_S and FP32 increment written, the increment gathered
-    # (60 B).  Its duration is the iteration phase's HIP events / launches.
+    # vectors: row sum, p_S, constant and 16 bytes of diagonal and counts read,
+    # row sum, p_S and FP32 increment written, the increment gathered (64 B).  Its duration is the iteration phase's HIP events / launches.
     it_ms = float(np.mean([x.ms_iterate for x in reps])) / max(1, reps[-1].iterations)
-    it_bytes = reps[-1].matrix_words * 4 + reps[-1].sources * 60
+    it_bytes = reps[-1].matrix_words * 4 + reps[-1].sources * 64
     it_ach = it_bytes / (it_ms * 1e-3) / 1e9
     roof = {"bound": "hbm", "achieved": round(it_ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(it_ach / HBM_PEAK_GBS, 4), "traffic": traffic.get("iteration"),
-            "kernel": "k_iterate_grp<8, increments> (one source iteration)",
+            "kernel": "k_iterate_words<8, increments> (one source iteration)",
             "algorithmic_bytes": it_bytes, "ms": round(it_ms, 5),
             "matrix_words": reps[-1].matrix_words, "source_visits": reps[-1].source_visits,
             # the two ray traversals: the bytes they move (counter traffic per

@@ -571,70 +571,70 @@ int build_plan(omni3d_ctx* ctx) {
     pl.nwords = pl.words.nwords;
   }
   if (!pl.words.valid) {
-  // each row's keys sorted
-  OMNI_TRY_HIP(ctx, launch_sort_rows(nS, pl.rowptr.as<unsigned long long>(),
-                                     key.as<unsigned long long>(), st));
-  // dense words unless sizes exceed their format: 24-bit source ids, rows
-  // shorter than 4096 entries (int64 row sums of terms below 2^51); otherwise
-  // (e.g. thousands of directions) the masked sliced-ELL layout
-  const bool use_dense = !want_slots && nS < (1 << (32 - kDenseRowBits)) && mxh[0] < 4096u &&
-                         nnz > 0 && nnz < (1ull << 31);
-  if (!use_dense) {
-    // masked sliced-ELL copy of the sorted rows for the iteration
-    if (D > 4096) return fail(ctx, OMNI3D_ERR_ARG, "at most 4096 directions");
-    const int nch = (nS + 63) / 64;
-    DevBuf nslot, tmp;
-    OMNI_TRY_HIP(ctx, nslot.alloc(sizeof(unsigned int) * (nch + 1)));
-    OMNI_TRY_HIP(ctx, tmp.alloc(scan_u32_tmp_bytes(nch)));
-    OMNI_TRY_HIP(ctx, pl.moff.alloc(sizeof(unsigned long long) * (nch + 1)));
-    OMNI_TRY_HIP(ctx, launch_sell_layout(nS, D, pl.rowptr.as<unsigned long long>(),
-                                         key.as<unsigned long long>(), nslot.as<unsigned int>(), st));
-    OMNI_TRY_HIP(ctx, launch_scan_u32(nslot.as<unsigned int>(), nch, pl.moff.as<unsigned long long>(),
-                                      0, tmp.as<void>(), tmp.size(), st));
-    unsigned long long nm = 0;
-    OMNI_TRY_HIP(ctx, hipMemcpyAsync(&nm, pl.moff.as<unsigned long long>() + nch, 8,
-                                     hipMemcpyDeviceToHost, st));
-    OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
-    if (nnz >= (1ull << 32)) return fail(ctx, OMNI3D_ERR_ARG, "too many source visits");
-    OMNI_TRY_HIP(ctx, pl.masks.alloc(sizeof(unsigned long long) * (nm + 1)));
-    OMNI_TRY_HIP(ctx, pl.cell_eb.alloc(sizeof(unsigned int) * (nm + 1)));
-    OMNI_TRY_HIP(ctx, pl.sdir.alloc(sizeof(unsigned short) * (nm + 1)));
-    // slack after the entries: the iteration stages them with 16-byte loads
-    OMNI_TRY_HIP(ctx, pl.ent.alloc(sizeof(int) * (nnz + 8)));
-    OMNI_TRY_HIP(ctx, launch_sell_fill(nS, D, pl.rowptr.as<unsigned long long>(),
-                                       key.as<unsigned long long>(), pl.moff.as<unsigned long long>(),
-                                       pl.masks.as<unsigned long long>(),
-                                       pl.cell_eb.as<unsigned int>(),
-                                       pl.sdir.as<unsigned short>(), pl.ent.as<int>(), st));
-    pl.ncell = (int64_t)nm;
-  }
-  {
-    if (use_dense) {
-      DevBuf ka, kb, tmp;
-      OMNI_TRY_HIP(ctx, ka.alloc(sizeof(unsigned long long) * nnz));
-      OMNI_TRY_HIP(ctx, kb.alloc(sizeof(unsigned long long) * nnz));
-      OMNI_TRY_HIP(ctx, tmp.alloc(dense_tmp_bytes((int64_t)nnz)));
-      // slack after the words: the iteration stages them with 16-byte loads
-      OMNI_TRY_HIP(ctx, pl.dent.alloc(sizeof(unsigned int) * (nnz + 8)));
-      OMNI_TRY_HIP(ctx, hipMemsetAsync(pl.dent.as<void>(), 0, sizeof(unsigned int) * (nnz + 8), st));
-      OMNI_TRY_HIP(ctx, sort_entry_keys(nS, (int64_t)nnz, kDenseRowBits,
-                                        pl.rowptr.as<unsigned long long>(),
-                                        key.as<unsigned long long>(), nullptr, nullptr, 0,
-                                        ka.as<unsigned long long>(), kb.as<unsigned long long>(),
-                                        tmp.as<void>(), tmp.size(), st));
-      OMNI_TRY_HIP(ctx, launch_dense_words((int64_t)nnz, kb.as<unsigned long long>(),
-                                           pl.dent.as<unsigned int>(), st));
-      pl.nwords = (int64_t)nnz;
+    // each row's keys sorted
+    OMNI_TRY_HIP(ctx, launch_sort_rows(nS, pl.rowptr.as<unsigned long long>(),
+                                       key.as<unsigned long long>(), st));
+    // dense words unless sizes exceed their format: 24-bit source ids, rows
+    // shorter than 4096 entries (int64 row sums of terms below 2^51); otherwise
+    // (e.g. thousands of directions) the masked sliced-ELL layout
+    const bool use_dense = !want_slots && nS < (1 << (32 - kDenseRowBits)) && mxh[0] < 4096u &&
+                           nnz > 0 && nnz < (1ull << 31);
+    if (!use_dense) {
+      // masked sliced-ELL copy of the sorted rows for the iteration
+      if (D > 4096) return fail(ctx, OMNI3D_ERR_ARG, "at most 4096 directions");
+      const int nch = (nS + 63) / 64;
+      DevBuf nslot, tmp;
+      OMNI_TRY_HIP(ctx, nslot.alloc(sizeof(unsigned int) * (nch + 1)));
+      OMNI_TRY_HIP(ctx, tmp.alloc(scan_u32_tmp_bytes(nch)));
+      OMNI_TRY_HIP(ctx, pl.moff.alloc(sizeof(unsigned long long) * (nch + 1)));
+      OMNI_TRY_HIP(ctx, launch_sell_layout(nS, D, pl.rowptr.as<unsigned long long>(),
+                                           key.as<unsigned long long>(), nslot.as<unsigned int>(), st));
+      OMNI_TRY_HIP(ctx, launch_scan_u32(nslot.as<unsigned int>(), nch, pl.moff.as<unsigned long long>(),
+                                        0, tmp.as<void>(), tmp.size(), st));
+      unsigned long long nm = 0;
+      OMNI_TRY_HIP(ctx, hipMemcpyAsync(&nm, pl.moff.as<unsigned long long>() + nch, 8,
+                                       hipMemcpyDeviceToHost, st));
       OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
-      pl.dense = true;
+      if (nnz >= (1ull << 32)) return fail(ctx, OMNI3D_ERR_ARG, "too many source visits");
+      OMNI_TRY_HIP(ctx, pl.masks.alloc(sizeof(unsigned long long) * (nm + 1)));
+      OMNI_TRY_HIP(ctx, pl.cell_eb.alloc(sizeof(unsigned int) * (nm + 1)));
+      OMNI_TRY_HIP(ctx, pl.sdir.alloc(sizeof(unsigned short) * (nm + 1)));
+      // slack after the entries: the iteration stages them with 16-byte loads
+      OMNI_TRY_HIP(ctx, pl.ent.alloc(sizeof(int) * (nnz + 8)));
+      OMNI_TRY_HIP(ctx, launch_sell_fill(nS, D, pl.rowptr.as<unsigned long long>(),
+                                         key.as<unsigned long long>(), pl.moff.as<unsigned long long>(),
+                                         pl.masks.as<unsigned long long>(),
+                                         pl.cell_eb.as<unsigned int>(),
+                                         pl.sdir.as<unsigned short>(), pl.ent.as<int>(), st));
+      pl.ncell = (int64_t)nm;
     }
+    {
+      if (use_dense) {
+        DevBuf ka, kb, tmp;
+        OMNI_TRY_HIP(ctx, ka.alloc(sizeof(unsigned long long) * nnz));
+        OMNI_TRY_HIP(ctx, kb.alloc(sizeof(unsigned long long) * nnz));
+        OMNI_TRY_HIP(ctx, tmp.alloc(dense_tmp_bytes((int64_t)nnz)));
+        // slack after the words: the iteration stages them with 16-byte loads
+        OMNI_TRY_HIP(ctx, pl.dent.alloc(sizeof(unsigned int) * (nnz + 8)));
+        OMNI_TRY_HIP(ctx, hipMemsetAsync(pl.dent.as<void>(), 0, sizeof(unsigned int) * (nnz + 8), st));
+        OMNI_TRY_HIP(ctx, sort_entry_keys(nS, (int64_t)nnz, kDenseRowBits,
+                                          pl.rowptr.as<unsigned long long>(),
+                                          key.as<unsigned long long>(), nullptr, nullptr, 0,
+                                          ka.as<unsigned long long>(), kb.as<unsigned long long>(),
+                                          tmp.as<void>(), tmp.size(), st));
+        OMNI_TRY_HIP(ctx, launch_dense_words((int64_t)nnz, kb.as<unsigned long long>(),
+                                             pl.dent.as<unsigned int>(), st));
+        pl.nwords = (int64_t)nnz;
+        OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
+        pl.dense = true;
+      }
 #ifdef OMNI3D_LAYOUT_STUDY
-    if (iter_env && std::strcmp(iter_env, "staged") == 0) {
-      const int rc = build_staged(ctx, nS, D, (int64_t)nnz);
-      if (rc) return rc;
-    }
+      if (iter_env && std::strcmp(iter_env, "staged") == 0) {
+        const int rc = build_staged(ctx, nS, D, (int64_t)nnz);
+        if (rc) return rc;
+      }
 #endif
-  }
+    }
   }
   OMNI_TRY_HIP(ctx, hipStreamSynchronize(st));
   pl.X = X;

@@ -40,8 +40,7 @@ struct DevScalars {
   unsigned int ticket;           // last-block counter of the reductions
   unsigned int pad;
   unsigned long long steps;      // staircase steps of the last full pass
-  unsigned long long itmax_bits[3];  // max |p_S| (or increment) after iteration k, slot k & 1
-                                     // (k % 3 with the finish folded into the next launch)
+  unsigned long long itmax_bits[2];  // max |p_S| after iteration k, slot k & 1
 };
 
 // Fingerprint of a kernel-level drop-in's inputs (directions; field and

@@ -458,7 +458,7 @@ k_mask_carry(int64_t nrays, const unsigned int* __restrict__ nseg,
 // What bounds it: per visit two LDS reads of the gradient, one LDS atomic and
 // the term's arithmetic; around it the loads a segment starts with, which
 // depend on one another (record, then flags and carry), so the next segment's
-// are in flight while one is walked, as in k_tile_pass.  The rule itself
+// are in flight while one is walked, as in k_tile_walk.  The rule itself
 // (compares of FP64 curl values, a dozen state operations per step) runs once
 // per field; curl / 10000, the division every curl weight needs, once per
 // voxel.
