@@ -343,15 +343,20 @@ int cu_count() {
   return std::max(n, 1);
 }
 
+// where 4 wavefronts per group reach every CU, 8 only cost their launch: us an
+// iteration with 4 / 8, FP64: 32^3 4.9 / 6.2, 48^3 6.0 / 6.2, 80^3 8.0 / 8.1,
+// 96^3 9.6 / 9.2, 160x128x96 (past the line) 13.5 each
+int word_chunks(int64_t nS, int fill) {
+  return nS >= word_max_sources(8) || nS <= (int64_t)word_rows(4) * fill ? 4 : 8;
+}
+
 int build_words(omni3d_ctx* ctx, int nS, int chunks, int fill, const unsigned long long* rowptr,
                 const unsigned long long* key, const unsigned int* diag, const unsigned int* cnt,
                 const int* slist, WordPlan* out) {
   hipStream_t st = ctx->stream;
   out->valid = false;
   if (nS < 1 || nS >= word_max_sources(4)) return OMNI3D_OK;
-  // where 4 wavefronts per group reach every CU, 8 only cost their launch: 32^3
-  // 5.3 us an iteration with 4, 5.6 with 8; 160x128x96 (past the line) 13.5 each
-  if (chunks == 0) chunks = nS <= word_rows(4) * fill ? 4 : 8;
+  if (chunks == 0) chunks = word_chunks(nS, fill);
   if (nS >= word_max_sources(8)) chunks = 4;
   std::vector<unsigned long long> hrp((size_t)nS + 1);
   OMNI_TRY_HIP(ctx, hipMemcpyAsync(hrp.data(), rowptr, sizeof(unsigned long long) * hrp.size(),

@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cstdio>
 #include <cstdlib>
 #include <map>
 #include <memory>
@@ -153,6 +154,33 @@ int prepare(omni3d_batch* b) {
   return OMNI3D_OK;
 }
 
+// Wavefronts per group of the snapshots' merged words, one choice for the
+// batch where their iterations shall share a launch; 0: each snapshot's own.
+// Grids that choose alike share it.  A mix of small and large ones takes 4 for
+// all, unless it is a few large ones: those gain more from their branches.  ms
+// per run, 200 iterations FP64, one launch with 4 / with 8 / a launch each (the
+// last also what a mix took when every snapshot chose for itself): 8 x 32^3 +
+// 8 x 20x24x22 3.4 / 3.6 / 14.6, 3 x (32^3 + 64^3) 3.6 / 4.9 / 6.6, 32^3 + 96^3
+// 3.1 / 3.5 / 4.1, 64^3 + 160x128x96 (118 k sources) 4.7 / 5.0 / 4.8, 15 x
+// 160x128x96 + 24^3 37.0 / 36.8 / 39.9; the other way 64^3 + 192^3 (243 k) 9.4 /
+// 9.2 / 8.7, 3 x 160x128x96 + 48^3 9.8 / 10.3 / 8.3, 7 x 160x128x96 + 32^3 18.8 /
+// 19.4 / 18.2.  So from more than two snapshots a branch on, or up to 160 k
+// sources in all.
+int batch_chunks(int count, const int* nx, const int* ny, const int* nz, int fill) {
+  int64_t total = 0;
+  bool four = false, eight = false;
+  for (int i = 0; i < count; i++) {
+    // (the sources are the surface voxels, or fewer where lines are sparse)
+    auto inner = [](int n) { return (int64_t)std::max(n - 2, 0); };
+    const int64_t surf =
+        (int64_t)nx[i] * ny[i] * nz[i] - inner(nx[i]) * inner(ny[i]) * inner(nz[i]);
+    total += surf;
+    (word_chunks(surf, fill) == 4 ? four : eight) = true;
+  }
+  if (!four || !eight) return four ? 4 : 8;
+  return count > 2 * kBranches || total <= 160000 ? 4 : 0;
+}
+
 // Uploads the iteration descriptors when every snapshot's source iteration
 // can share one launch per iteration (same precision for all); else 0.
 int fused_descriptors(omni3d_batch* b, bool* fused) {
@@ -215,6 +243,9 @@ int capture(omni3d_batch* b) {
   bool fused = false;
   int rc = fused_descriptors(b, &fused);
   if (rc) return rc;
+  if (std::getenv("OMNI3D_VERBOSE"))
+    std::fprintf(stderr, "omni3d batch: %d snapshots, %s\n", (int)b->snap.size(),
+                 fused ? "one launch per iteration" : "a launch per snapshot and iteration");
   BATCH_TRY_HIP(b, hipStreamBeginCapture(b->main, hipStreamCaptureModeThreadLocal));
   rc = enqueue_branches(b, fused ? 1 : 0, b->fork);
   if (rc == OMNI3D_OK && fused) {
@@ -252,6 +283,8 @@ int omni3d_batch_create(const omni3d_params* base, int count, const int* nx, con
     return fail(nullptr, OMNI3D_ERR_ARG, "batch: null argument or empty batch");
   omni3d_batch* b = new omni3d_batch();
   b->base = *base;
+  const int fill = std::max(1, cu_count() / count);
+  const int chunks = batch_chunks(count, nx, ny, nz, fill);
   for (int i = 0; i < count; i++) {
     omni3d_params p = *base;
     p.nx = nx[i];
@@ -268,6 +301,7 @@ int omni3d_batch_create(const omni3d_params* base, int count, const int* nx, con
     // reference schedule instead
     c->affine_masked = false;
     c->cu_share = count;  // the snapshots' iterations share one launch
+    if (c->dense_group == 0) c->dense_group = chunks;
     b->snap.push_back(c);
   }
   for (int i = 0; i < count; i++) b->out.emplace_back(new DevBuf());

@@ -37,6 +37,9 @@ double path_bound(const omni3d_params& P, const Plan& pl);
 // first row of every group (nS last), rgroup[nS] the group of every row.
 void balance_groups(const std::vector<unsigned long long>& rowptr, int maxrows, int ncu,
                     std::vector<int>* grow, std::vector<int>* rgroup);
+// Wavefronts per group (times 64 rows) of the merged words of nS rows, the
+// groups' number being a multiple of fill.
+int word_chunks(int64_t nS, int fill);
 // CSR rows (nS + 1 offsets rowptr on the device, the entries' sources in the
 // low halves of key) as merged words in groups of `chunks` (8 or 4; 4 where
 // the sources need it) times 64 rows at most, sized to about equal entries,

@@ -7,7 +7,9 @@
     snapshot, bit for bit the result of the snapshot-by-snapshot schedule and
     the iteration count of a single-context reconstruction; replays after
     new fields (with eager work in between) give the new results;
-  * the autotuner's choices are valid shapes and keep the results.
+  * the autotuner's choices are valid shapes and keep the results;
+  * grids of unlike sizes share the iteration's launches where that is the
+    faster schedule.
 """
 import numpy as np
 import pytest
@@ -141,3 +143,44 @@ def test_batch_graph_masked_methods(gpu_available, ref_dirs2, method):
                 ctx.set_field(fs[i]["acc"], mask=masks[i])
                 ps = ctx.reconstruct()[0]
             assert F.rel_l2(seq[i], ps) < 1e-12
+
+
+# ([shapes], whether their iterations share a launch): small and large grids
+# whose rows alone would be grouped unlike; a few large ones and a small one
+# keep a launch each
+MIXES = [([(32, 32, 32), (96, 96, 96)], True),
+         ([(64, 64, 64), (96, 128, 160)], True),
+         ([(20, 24, 22)] * 8 + [(40, 40, 40)], True),
+         ([(128, 128, 128)] * 3 + [(24, 24, 24)], False)]
+
+
+@pytest.mark.parametrize("shapes,shared", MIXES)
+@pytest.mark.parametrize("precision", [omni3d.FP64, omni3d.FP32_KAHAN])
+def test_mixed_grids_share_the_iteration(gpu_available, ref_dirs2, monkeypatch, capfd, shapes,
+                                         shared, precision):
+    """The captured batch runs one launch per iteration for grids of unlike
+    sizes; which rows a group holds changes no sum (they are exact, of the same
+    rounded terms): the results are those of lone contexts bit for bit."""
+    print(f"case batch mix {shapes} {precision}", flush=True)
+    monkeypatch.setenv("OMNI3D_VERBOSE", "1")
+    dtype = np.float64 if precision == omni3d.FP64 else np.float32
+    h = 0.1
+    kw = dict(max_iterations=7, tolerance=0.0, precision=precision)
+    fs = [[a.astype(dtype) for a in
+           F.taylor_green(max(s), noise=0.05, seed=20 + i, shape=s)["acc"]]
+          for i, s in enumerate(shapes)]
+    with omni3d.Batch(shapes, (h, h, h), **kw) as b:
+        b.set_directions(ref_dirs2)
+        for i, f in enumerate(fs):
+            b.set_field(i, f, dtype=dtype)
+        b.run(use_graph=True)
+        b.run(use_graph=True)
+        got = [b.result(i)[0] for i in range(len(shapes))]
+    err = capfd.readouterr().err
+    assert ("one launch per iteration" in err) == shared
+    monkeypatch.delenv("OMNI3D_VERBOSE")
+    for i in sorted({0, len(shapes) - 1}):
+        with omni3d.Context(shapes[i], (h, h, h), **kw) as ctx:
+            ctx.set_directions(ref_dirs2)
+            ctx.set_field(fs[i], dtype=dtype)
+            np.testing.assert_array_equal(got[i], ctx.reconstruct()[0])
