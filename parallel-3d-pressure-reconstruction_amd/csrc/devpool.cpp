@@ -25,6 +25,7 @@ namespace {
 constexpr size_t kBound = (size_t)2 << 30;  // under a hundredth of the card's memory
 
 struct Pool {
+  std::mutex wait;  // held (before mu) while blocks are out of the lists to be waited for
   std::mutex mu;
   std::multimap<size_t, void*> ready, pending;  // by size
 };
@@ -67,7 +68,9 @@ void count(size_t cap, bool add) {
 size_t give_back(int dev) {
   std::multimap<size_t, void*> all;
   {
+    // (blocks another thread waits for come back to the lists first)
     Pool& q = pool(dev);
+    std::lock_guard<std::mutex> held(q.wait);
     std::lock_guard<std::mutex> lock(q.mu);
     all.swap(q.ready);
     all.merge(q.pending);
@@ -81,6 +84,28 @@ size_t give_back(int dev) {
   return bytes;
 }
 
+// A pending block, after one of the others went back to the driver.
+void* take_after_wait(Pool& q, size_t need, size_t* cap) {
+  std::lock_guard<std::mutex> held(q.wait);
+  std::multimap<size_t, void*> waited;
+  {
+    std::lock_guard<std::mutex> lock(q.mu);
+    if (void* p = take(&q.ready, need, cap)) return p;
+    if (!fits(q.pending, need)) return nullptr;
+    waited.swap(q.pending);
+  }
+  auto fence = waited.begin();
+  if (fence->first >= need) ++fence;
+  const bool idle = fence != waited.end() && hipFree(fence->second) == hipSuccess;
+  if (idle) {
+    count(fence->first, false);
+    waited.erase(fence);
+  }
+  std::lock_guard<std::mutex> lock(q.mu);
+  (idle ? q.ready : q.pending).merge(waited);
+  return idle ? take(&q.ready, need, cap) : nullptr;
+}
+
 }  // namespace
 
 hipError_t device_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
@@ -90,24 +115,13 @@ hipError_t device_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
   const size_t need = rounded(bytes ? bytes : 1);
   if (*dev < kDevices) {
     Pool& q = pool(*dev);
-    std::multimap<size_t, void*> waited;
+    bool fence = false;
     {
       std::lock_guard<std::mutex> lock(q.mu);
       *p = take(&q.ready, need, cap);
-      if (!*p && fits(q.pending, need)) waited.swap(q.pending);
+      fence = !*p && fits(q.pending, need);
     }
-    if (!waited.empty()) {
-      auto fence = waited.begin();
-      if (fence->first >= need) ++fence;
-      const bool idle = fence != waited.end() && hipFree(fence->second) == hipSuccess;
-      if (idle) {
-        count(fence->first, false);
-        waited.erase(fence);
-      }
-      std::lock_guard<std::mutex> lock(q.mu);
-      (idle ? q.ready : q.pending).merge(waited);
-      if (idle) *p = take(&q.ready, need, cap);
-    }
+    if (fence) *p = take_after_wait(q, need, cap);
     if (*p) {
       count(*cap, false);
       return hipSuccess;

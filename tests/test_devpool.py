@@ -1,0 +1,27 @@
+"""The device-memory pool's rules over a counting allocator in place of the
+driver's (devpool_host.cpp): what serves again and when, the bound, and that
+what waits goes back before a request is refused, whoever holds it.
+"""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "parallel-3d-pressure-reconstruction_amd", "csrc")
+CHECKS = ["reuse", "bound", "out_of_memory", "out_of_memory_beside_a_wait"]
+
+
+@pytest.fixture(scope="module")
+def checker(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("devpool") / "devpool_host")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-I" + CSRC, os.path.join(HERE, "devpool_host.cpp"),
+                    os.path.join(CSRC, "devpool.cpp"), "-o", exe, "-lpthread"], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("check", CHECKS)
+def test_pool_rules(checker, check):
+    r = subprocess.run([checker, check], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
