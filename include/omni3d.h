@@ -268,10 +268,16 @@ int omni3d_es_inner_weighted_minicurl(long X, long Y, long Z, int NoAngles, floa
  * p = pn / pcountinner and pn = 0. */
 int omni3d_devide_count_inner(long X, long Y, long Z, float* p, float* pn,
                               const float* pcountinner, void* hip_stream);
-/* Frees the calling thread's hidden drop-in context (plan, staged field), and
- * returns the device memory that released objects of the library left for the
- * next ones (2 GiB at most; also returned when the driver has no more). */
+/* Frees the calling thread's hidden drop-in context (plan, staged field), then
+ * does what omni3d_release_unused does. */
 void omni3d_dropin_release(void);
+/* Returns to the driver the device memory that released buffers of the library
+ * left for the next ones, 2 GiB at most over all devices; the bytes returned.
+ * It waits for the devices.  Nothing in use is touched (contexts and the hidden
+ * drop-in context keep their plans).  The library itself does so before it
+ * reports that the driver is out of memory; call it where another allocator of
+ * the process needs that memory, and before a hipDeviceReset. */
+int64_t omni3d_release_unused(void);
 
 /* The same six under the reference kernels' own names and argument lists
  * (kernel.cu:6151, 6281, 6414, 6481, 6347, 6746): a reference call site

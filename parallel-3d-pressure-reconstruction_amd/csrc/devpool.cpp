@@ -1,9 +1,9 @@
 // Device memory of the library's buffers.
 //
 // Building a plan and its first reconstruction take some 60 buffers, and
-// hipMalloc / hipFree of them cost as much as the kernels: 8.7 of 24 ms at
-// 128^3 (20 ms with the blocks passed on).  So a released block waits here for the next
-// request of about its size.
+// hipMalloc / hipFree of them cost as much as the kernels: 8.7 of 24.4 ms at
+// 128^3 (18.2 ms with the blocks passed on; 21.0 to 21.7 when all go back with the last
+// context).  So a released block waits here for the next request of about its size.
 //
 // hipFree waits for the device; a block given up here may still be in use on
 // some stream, so it is `pending` until one of the pending blocks -- the

@@ -364,6 +364,8 @@ void omni3d_dropin_release(void) {
   (void)device_release_unused();
 }
 
+int64_t omni3d_release_unused(void) { return (int64_t)device_release_unused(); }
+
 // The reference kernels' own names (a call site minus its <<<grid, block>>>).
 void omni3dparallellinesESInner(long Xsize, long Ysize, long Zsize, int NoAngles,
                                 float linespacing, float* k1_d, float* k2_d, float* k3_d,

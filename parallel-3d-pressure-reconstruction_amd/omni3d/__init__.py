@@ -39,7 +39,8 @@ EXPORTS = [
     "omni3d_read_parameter_file", "omni3d_run_parameter_file_ex",
     "thredholdHistMaterialAccCPU", "omni3d_threshold_hist", "omni3d_boundary_pairs",
     "omni3d_es_inner_select_fixedbc", "omni3d_es_inner_weighted_minicurl",
-    "omni3d_set_velocity", "omni3d_dropin_release", "initialIntegration",
+    "omni3d_set_velocity", "omni3d_dropin_release", "omni3d_release_unused",
+    "initialIntegration",
     "omni3d_initial_integration", "omni3dparallellinesESInner",
     "omni3dparallellinesESInnerWeighted", "omni3dparallellinesESInnerSelect",
     "omni3dparallellinesESInnerSelectFixedBC", "omni3dparallellinesESInnerWeightedMiniCurl",
@@ -131,6 +132,8 @@ def _declare(L):
     L.omni3d_devide_count_inner.argtypes = [lg, lg, lg, vp, vp, vp, vp]
     L.omni3d_dropin_release.argtypes = []
     L.omni3d_dropin_release.restype = None
+    L.omni3d_release_unused.argtypes = []
+    L.omni3d_release_unused.restype = C.c_int64
     for name, extra in (("omni3dparallellinesESInner", [vp, vp, vp]),
                         ("omni3dparallellinesESInnerWeighted", [vp, vp, vp, vp]),
                         ("omni3dparallellinesESInnerSelect", [vp, vp, vp, vp, f]),
@@ -184,6 +187,12 @@ def check(rc, ctx=None):
         L = lib()
         msg = (L.omni3d_last_error(ctx) if ctx else L.omni3d_last_global_error()) or b""
         raise Omni3DError(rc, msg.decode(errors="replace"))
+
+
+def release_unused():
+    """Returns to the driver the device memory that closed contexts and finished
+    calls left for the next ones (2 GiB at most); the bytes returned."""
+    return lib().omni3d_release_unused()
 
 
 def generate_directions(divide):
