@@ -1,6 +1,6 @@
 """The merged words of the source iteration at the edges of their layout:
-fewer sources than groups (empty groups, whose first loads are the filling
-block's), rows of many equal entries (words of 1, 2 and 4), one block per
+few sources (groups of one row, groups whose rows have no entries and which
+load the filling block alone), rows of many equal entries (words of 1, 2 and 4), one block per
 group and several rounds per wavefront, groups of 4 and of 8 wavefronts.
 Against the dense words (one entry per word, 64 rows per chunk): both round
 every FP64 term to the same unit and add exactly, so p is bit-equal there.
