@@ -285,12 +285,6 @@ def methods_mode(args):
                "kind": "port",
                "sample": f"oracle FP64 serial Select pass over {len(sub)} of {D} directions at "
                          f"{n}^3 took {ts:.2f}s, scaled x{D / len(sub):.1f} to one pass"}
-    traffic = None
-    tf = os.path.join(ROOT, "profiles", "traffic_masked_fourier128.json")
-    if os.path.exists(tf):
-        t = json.load(open(tf))
-        if t.get("workload_n") == n and t.get("directions") == D:
-            traffic = t.get("traffic_bytes", {}).get("select")
     print(json.dumps({
         "metric": "ms per reference-schedule pass, 128^3 masked Fourier sphere",
         "value": first["ms_per_pass"], "unit": "ms", "n_gpus": 1, "steps": args.steps,
@@ -298,7 +292,7 @@ def methods_mode(args):
         "data": "synthetic",
         "roofline": {"bound": "hbm", "achieved": round(bytes_pass / (first["ms_per_pass"] * 1e-3)
                                                        / 1e9, 1),
-                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": first["frac"], "traffic": traffic,
+                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": first["frac"],
                      "kernel": "k_mask_carry + k_tile_masked<float, select, 16^3, 1024> "
                                "(one iteration)", "algorithmic_bytes": bytes_pass},
         "cpu_baseline": cpu,
