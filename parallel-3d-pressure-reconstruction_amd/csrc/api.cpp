@@ -414,7 +414,8 @@ int build_words(omni3d_ctx* ctx, int nS, int chunks, int fill, const unsigned lo
   out->nwords = (int64_t)nb * kWordBlock;
   out->valid = true;
   if (std::getenv("OMNI3D_VERBOSE"))
-    std::fprintf(stderr, "omni3d words: %d rows, %llu entries in %u words, %u blocks, %d groups of %d chunks\n",
+    std::fprintf(stderr,
+                 "omni3d words: %d rows, %llu entries in %u words, %u blocks, %d groups of %d chunks\n",
                  nS, n, nw, nb, ng, chunks);
   return OMNI3D_OK;
 }
@@ -1080,7 +1081,8 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype) {
                                           m == OMNI3D_METHOD_PLAIN_MASK
                                               ? ctx->wcnt.as<unsigned int>() : nullptr,
                                           fixed ? nullptr : ctx->wsum.as<double>(),
-                                          ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(), st));
+                                          ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(),
+                                          st));
   record_event(ctx, 8);
   record_event(ctx, 3);
   for (int k = 1; k <= P.max_iterations; k++) {
@@ -1096,7 +1098,8 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype) {
                                               ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), pa,
                                               pb, k, sc,
                                               fixed ? ctx->sum.as<long long>() : nullptr,
-                                              fixed ? nullptr : ctx->sumd.as<double>(), ctx->mk_bits.as<void>(), st));
+                                              fixed ? nullptr : ctx->sumd.as<double>(),
+                                              ctx->mk_bits.as<void>(), st));
       OMNI_TRY_HIP(ctx, launch_naive_update(k, V, fixed ? 1 : 0,
                                             fixed ? ctx->sum.as<long long>() : nullptr, cntw,
                                             fixed ? nullptr : ctx->sumd.as<double>(),
@@ -1142,13 +1145,6 @@ int run_naive(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype) {
   return OMNI3D_OK;
 }
 
-// The masked methods (plain-mask, Select, Weighted) on their affine
-// schedule (masked.hip): the rule replay of the field, the run starts S and
-// the rows of the visits landing on them, the pass from p = 0 (the constant
-// b), the iteration on S, and one full pass from p_S^{k*-1}.  Sets
-// *fallback (nothing of the result queued) when the rows do not fit the
-// iteration's fixed-point sums (a voxel visited 4096 times or more) or there
-// is no run start, for the caller to run the reference schedule.
 // Entries of a workgroup of the tile-layout iteration at most (Weighted 128^3:
 // an iteration's share of the call is 11.9 ms with a 4096th, 12.1 with a
 // 1024th, 13.0 with a 512th of the entries).
@@ -1156,6 +1152,13 @@ unsigned long long mask_chunk_entries(unsigned long long nnz) {
   return std::max<unsigned long long>(2048ull, std::min<unsigned long long>(65536ull, nnz / 4096ull));
 }
 
+// The masked methods (plain-mask, Select, Weighted) on their affine
+// schedule (masked.hip): the rule replay of the field, the run starts S and
+// the rows of the visits landing on them, the pass from p = 0 (the constant
+// b), the iteration on S, and one full pass from p_S^{k*-1}.  Sets
+// *fallback (nothing of the result queued) when the rows do not fit the
+// iteration's fixed-point sums (a voxel visited 4096 times or more) or there
+// is no run start, for the caller to run the reference schedule.
 template <typename T>
 int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dtype,
                       bool* fallback) {
@@ -1266,7 +1269,8 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                           ctx->mk_s.as<double>(), ctx->mk_r.as<uint32_t>(),
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
                                           ctx->mk_wn.as<double>(), wcnt, wsum,
-                                          ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(), st));
+                                          ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(),
+                                          st));
   }
   record_event(ctx, 8);
   // S: compact ids of the run starts (the voxels a pass reads p at), in tile
@@ -1318,7 +1322,8 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
     OMNI_TRY_HIP(ctx, launch_tile_rows(false, m, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                                        pl.segs.as<SegRec>(), pl.g, pl.tg, wp, aux,
                                        ctx->mk_f.as<uint32_t>(), ctx->am_run.as<uint32_t>(), sid,
-                                       rcnt.as<unsigned int>(), nullptr, nullptr, ctx->mk_bits.as<void>(), st));
+                                       rcnt.as<unsigned int>(), nullptr, nullptr,
+                                       ctx->mk_bits.as<void>(), st));
     OMNI_TRY_HIP(ctx, stmp.alloc(scan_u32_tmp_bytes(nS)));
     OMNI_TRY_HIP(ctx, launch_scan_u32(rcnt.as<unsigned int>(), nS,
                                       ctx->am_ptr.as<unsigned long long>(), 0, stmp.as<void>(),
@@ -1393,7 +1398,8 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
                                           ctx->am_tbase.as<unsigned long long>(),
                                           ctx->am_src.as<unsigned int>(),
                                           ctx->am_erow.as<unsigned short>(),
-                                          fixed ? nullptr : ctx->am_w.as<double>(), ctx->mk_bits.as<void>(), st));
+                                          fixed ? nullptr : ctx->am_w.as<double>(),
+                                          ctx->mk_bits.as<void>(), st));
     // chunks of at most csz entries of one tile, a workgroup each
     const unsigned long long csz = mask_chunk_entries(nnz);
     std::vector<MaskChunk> chunks;
@@ -1427,8 +1433,8 @@ int run_affine_masked(omni3d_ctx* ctx, int seed, void* pdst, void* wdst, int dty
   OMNI_TRY_HIP(ctx, launch_tile_masked<T>(m, pl.ntiles, pl.tile_ptr.as<unsigned long long>(),
                                           pl.segs.as<SegRec>(), pl.g, pl.tg, wp, field, aux,
                                           ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
-                                          ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), nullptr, nullptr,
-                                          1, sc, sumfx, sumd, ctx->mk_bits.as<void>(), st));
+                                          ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(), nullptr,
+                                          nullptr, 1, sc, sumfx, sumd, ctx->mk_bits.as<void>(), st));
   const size_t ns = (size_t)nS;
   const size_t ns16 = (ns + 15) & ~(size_t)15;
   double* q0 = nullptr;

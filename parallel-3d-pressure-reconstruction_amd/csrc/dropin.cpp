@@ -240,7 +240,8 @@ int es_pass(int method, long X, long Y, long Z, int D, float ls, const float* k1
                                                  ctx->mk_f.as<uint32_t>(), ctx->mk_wc.as<double>(),
                                                  ctx->mk_wn.as<double>(), nullptr,
                                                  fixed ? nullptr : ctx->wsum.as<double>(),
-                                                 ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(), st));
+                                                 ctx->srcf.as<uint8_t>(), rule, ctx->mk_bits.as<void>(),
+                                                 st));
     }
     const double* pa = ctx->pa.as<double>();
     OMNI_TRY_HIP(ctx, ctx->mk_c.alloc(sizeof(double) * nv));
@@ -257,7 +258,8 @@ int es_pass(int method, long X, long Y, long Z, int D, float ls, const float* k1
                                                  ctx->mk_wn.as<double>(), ctx->mk_c.as<double>(),
                                                  pa, pa, 1, sc,
                                                  fixed ? ctx->sum.as<long long>() : nullptr,
-                                                 fixed ? nullptr : ctx->sumd.as<double>(), ctx->mk_bits.as<void>(), st));
+                                                 fixed ? nullptr : ctx->sumd.as<double>(),
+                                                 ctx->mk_bits.as<void>(), st));
   } else {
     if (!fixed) OMNI_TRY_HIP(ctx, launch_fill_u32(ctx->wsum.as<void>(), 2 * V, 0u, st));
     OMNI_TRY_HIP(ctx, launch_walk_naive<double>(method, pl.rays.as<RayRec>(), pl.nrays,

@@ -305,7 +305,7 @@ __device__ __forceinline__ double div_small(double s, double n, double r) {
 // in an LDS ring and four barriers, every stage read its right-hand side from
 // memory again -- 1.2 GB a pass for 0.5 at 256^3 -- and spent most of its
 // instructions on places and bounds: 232 us a pass; a ring with one barrier
-// 200; this 108, of which one read of p and of the right-hand side and one
+// 200; this 111, of which one read of p and of the right-hand side and one
 // write take 82.)
 //
 // Voxels outside the box are -0.0, which adds to any value without changing

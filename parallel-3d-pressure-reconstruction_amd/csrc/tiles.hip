@@ -289,7 +289,9 @@ k_tile_sources(const int* __restrict__ tile_list, const unsigned long long* __re
 // What is left is LDS for the full pass (an 8-byte add and a 4-byte read a
 // step, 17 cycles with their conflicts) and the slots' stores for the segment
 // sums.  us per launch before / now, FP32: 128^3 sums 336 / 284, full 471 / 413;
-// 256^3 3415 / 3450, 3406 / 3385 (two workgroups shared a CU, one does now).
+// 256^3 sums 3060 / 2730 (before: on a copy of the segments in slot order), full
+// 3300 / 3260 (two workgroups shared a CU, one does now).  A context's first
+// launch of the sums takes 5400 to 7600 there, the first use of its slots.
 // kLocalSum has the edges into and out of the tile too: cell 0 of an axis is
 // the voxel before the tile.
 template <typename T, int kMode, int kBits, int kThreads>
@@ -500,10 +502,8 @@ hipError_t launch_tile_counts(int ntiles, const unsigned long long* tile_ptr, co
 // workgroup per surface tile replays the step codes of the tile's segments
 // and keeps those whose visits reach a source voxel after the ray's entry
 // (for a later segment the first visit counts too), with the visit count
-// cut after the last such visit and the position in the full list (where
-// the pass reads the segment's step term) in the source field.  pass 0
-// counts per tile, pass 1 writes at sptr[tile] (order inside a tile
-// immaterial: the pass sums exactly).
+// cut after the last such visit.  pass 0 counts per tile, pass 1 writes at
+// sptr[tile] (order inside a tile immaterial: the pass sums exactly).
 template <int kBits>
 __global__ void __launch_bounds__(256)
 k_src_segs(int pass, const int* __restrict__ tile_list, const unsigned long long* __restrict__ tile_ptr,
@@ -554,7 +554,6 @@ k_src_segs(int pass, const int* __restrict__ tile_list, const unsigned long long
     if (pass == 1) {
       SegRec r = sr;
       r.info = (sr.info & ~(63u << kSegLvBits)) | ((unsigned int)(last + 1) << kSegLvBits);
-      r.src = (uint32_t)j;
       out[sptr[tile] + pos] = r;
     }
   }

@@ -249,7 +249,8 @@ hipError_t launch_tile_masked(int method, int ntiles, const unsigned long long* 
 
 // adjoint.hip: the plain method's transposed traversals on the tile engine
 // (what 0: per-segment sums of u; 1: per-ray sums of the later segments into
-// tafter, and each ray's total into tvol at its entry voxel, where given; 2: the scatter of h * S into dg, every voxel stored)
+// tafter, and each ray's total into tvol at its entry voxel, where given; 2: the
+// scatter of h * S into dg, every voxel stored)
 hipError_t launch_adj_tiles(int what, int ntiles, const unsigned long long* tile_ptr,
                             const SegRec* segs, const RayRec* rays, int64_t nrays,
                             const unsigned int* nseg, const unsigned long long* val_off,
