@@ -13,7 +13,7 @@ CHECKS = ["reuse", "bound", "out_of_memory", "out_of_memory_beside_a_wait"]
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def devpool_host(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("devpool") / "devpool_host")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__",
                     "-I/opt/rocm/include", "-I" + CSRC, os.path.join(HERE, "devpool_host.cpp"),
@@ -22,6 +22,6 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", CHECKS)
-def test_pool_rules(checker, check):
-    r = subprocess.run([checker, check], capture_output=True, text=True, timeout=60)
+def test_pool_rules(devpool_host, check):
+    r = subprocess.run([devpool_host, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
